@@ -24,7 +24,7 @@ ROOT = Path(__file__).resolve().parent
 CSRC = ROOT / "csrc"
 OUT_DIR = ROOT / "musa_aiter" / "_lib"
 LIB_NAME = "libmusa_aiter_kv_hip.so"
-SOURCES = ("kv_paged_tiles.hip", "kv_paged_waves.hip", "kv_rows.hip", "kv_batch_copy.hip", "kv_cachegen.hip",
+SOURCES = ("kv_paged_tiles.hip", "kv_paged_waves.hip", "kv_paged_wide.hip", "kv_rows.hip", "kv_batch_copy.hip", "kv_cachegen.hip",
            "kv_pattern.hip", "kv_abi.hip")
 ARCH = os.environ.get("MUSA_AITER_HIP_ARCH", "gfx950")
 

@@ -99,6 +99,10 @@ __device__ __forceinline__ u32x4 buf_ld16(buf_t r, uint32_t off, uint32_t soff) 
 __device__ __forceinline__ u32x4 buf_ld16_cached(buf_t r, uint32_t off) {
   return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
 }
+// 16-byte stores never take a scalar offset: with one, the compiler issues no
+// wait between the store and a VALU write to its data registers, and gfx950
+// then stored the overwritten first dword for the last lanes of each 16 (seen
+// as one wrong column per tile, now and then).  With offset 0 it waits.
 __device__ __forceinline__ void buf_st16(buf_t r, uint32_t off, u32x4 v) {
   __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, kBufNT);
 }

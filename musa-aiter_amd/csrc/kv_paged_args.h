@@ -26,7 +26,7 @@ struct TileArgs {
   int32_t fill_zeros;
   uint32_t epoch;
   int32_t owner_exclusive;     // every tag of `epoch` in owner was claimed by this call
-  int32_t block_size;          // used by the generic kernel only
+  int32_t block_size;          // used by the wide and generic kernels
   float inv_head_dim;          // 1 / head_dim, for small-integer division by head_dim
   BlockTableSlots bt;          // block_tables set: slots derived per dense token
   int32_t row_groups;          // tile kernel: row groups per block (grid x of a gather = tile * row_groups + group)
@@ -161,5 +161,14 @@ hipError_t launch_wave_scatter(const TileArgs& a, int64_t planes, hipStream_t st
 // (kv_paged_waves.hip): needs this call's claim tags as the inverse map.
 template <int BS>
 hipError_t launch_wave_copy_scatter(const TileArgs& a, int64_t planes, hipStream_t stream);
+
+// Paged-A copies whose cache rows are whole 128-byte lines (kv_paged_wide.hip).
+// `lines`: every linear row covers whole 128-byte lines.
+template <int ELT, bool SCATTER>
+hipError_t launch_wide(const TileArgs& a, int64_t planes, bool lines, hipStream_t stream);
+
+// Largest block size launch_wide takes: its 32-bit offsets span a workgroup's
+// rows (at most 64) at a row pitch of block_size elements.
+constexpr int64_t kWideMaxBlockSize = 65536;
 
 }  // namespace kvhip

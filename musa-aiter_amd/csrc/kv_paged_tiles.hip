@@ -733,6 +733,8 @@ hipError_t dispatch_bs(const TileArgs& a, int64_t bs, bool fast, int64_t planes,
       if (bs == 8) return launch_tile<ELT_C, 8, SCATTER>(a, planes, stream);
       if (bs == 16) return launch_tile<ELT_C, 16, SCATTER>(a, planes, stream);
       if (bs == 32) return launch_tile<ELT_C, 32, SCATTER>(a, planes, stream);
+      if (bs % (128 / ELT_C) == 0 && bs <= kWideMaxBlockSize)
+        return launch_wide<ELT_C, SCATTER>(a, planes, linear_rows_whole_lines(a, ELT_C), stream);
     } else if constexpr (!SCATTER) {
       // FP8 dequant-gather: per-wave kernel (kv_paged_waves.hip), unless a chunk
       // of its rows spans more heads than its decode tables hold.

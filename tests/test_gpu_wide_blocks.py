@@ -1,0 +1,88 @@
+"""GPU parity of caches whose block size is a multiple of 64, against the oracle.
+
+Such blocks are copied in units of 64 columns by kernels of their own, with 64-token tiles and a
+two-register slot window.  The mappings put runs across tile and unit edges, full units, partial
+units, single tokens, skipped and repeated slots into one call; token counts sit on both sides of
+the forms' limits (256 tokens: per-token gathers and in-kernel duplicate resolution).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import musa_aiter
+from oracle import kv_oracle as ko
+from tests.kvgen import bits, make_slots, random_payload
+from tests.test_gpu_destination_order import tricky_slots
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _round_trip(dtype, layers, nh, hd, bs, slots, nb):
+    gen = torch.Generator().manual_seed(len(slots) + bs)
+    kc, vc = (random_payload((layers, nb, nh, hd, bs), dtype, gen) for _ in range(2))
+    kl, vl = (random_payload((layers, len(slots), nh, hd), dtype, gen) for _ in range(2))
+    s_d = torch.from_numpy(slots).to(DEV)
+    ok, ov = musa_aiter.kv_paged_to_linear_multi_layer(kc.to(DEV), vc.to(DEV), s_d)
+    assert np.array_equal(bits(ok), ko.paged_to_linear_multi_layer(bits(kc), slots))
+    assert np.array_equal(bits(ov), ko.paged_to_linear_multi_layer(bits(vc), slots))
+    kc_d, vc_d = kc.to(DEV), vc.to(DEV)
+    musa_aiter.kv_linear_to_paged_multi_layer(kl.to(DEV), vl.to(DEV), kc_d, vc_d, s_d)
+    want_k, want_v = bits(kc).copy(), bits(vc).copy()
+    ko.linear_to_paged_multi_layer(bits(kl), want_k, slots)
+    ko.linear_to_paged_multi_layer(bits(vl), want_v, slots)
+    assert np.array_equal(bits(kc_d), want_k)
+    assert np.array_equal(bits(vc_d), want_v)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bs", [32, 64, 128, 192])
+@pytest.mark.parametrize("nh, hd", [(4, 64), (3, 40)])
+@pytest.mark.parametrize("layers,tokens,kind", [
+    (1, 1, "sequences"),
+    (1, 63, "decode"),
+    (2, 256, "decode"),
+    (1, 200, "duplicates"),
+    (1, 257, "random"),
+    (2, 700, "sequences"),
+    (2, 900, "skips"),
+    (1, 1500, "duplicates"),
+])
+def test_wide_blocks_match_oracle(dtype, bs, nh, hd, layers, tokens, kind):
+    slots, nb = make_slots(kind, np.random.default_rng(tokens + bs), block_size=bs, tokens=tokens)
+    _round_trip(dtype, layers, nh, hd, bs, slots, nb)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bs", [32, 64, 128])
+@pytest.mark.parametrize("layers", [3, 17])  # 17: past 32 planes, the XCD-contiguous order
+def test_wide_blocks_in_destination_order(dtype, bs, layers):
+    slots = tricky_slots(np.random.default_rng(bs), 12, bs)
+    assert len(slots) * 4 >= 12 * bs
+    _round_trip(dtype, layers, 2, 72, bs, slots, 12)
+
+
+@pytest.mark.parametrize("bs", [32, 64, 128])
+def test_wide_blocks_through_block_tables(bs):
+    rng = np.random.default_rng(bs)
+    nh, hd, nb, batch = 2, 64, 9, 3
+    lengths = np.array([2 * bs, bs // 2 + 1, bs + 6])
+    tables = rng.permutation(nb)[:batch * 2].reshape(batch, 2)
+    gen = torch.Generator().manual_seed(3)
+    kc, vc = (random_payload((nb, nh, hd, bs), torch.bfloat16, gen) for _ in range(2))
+    dk, dv = (random_payload((batch, 2 * bs, nh, hd), torch.bfloat16, gen) for _ in range(2))
+    t_d, l_d = torch.from_numpy(tables).to(DEV), torch.from_numpy(lengths).to(DEV)
+    got = musa_aiter.kv_load_and_reshape_flash(kc.to(DEV), vc.to(DEV), t_d, l_d)
+    pos = np.arange(2 * bs)
+    slots = np.where(pos < lengths[:, None], tables[:, pos // bs] * bs + pos % bs, -1).reshape(-1)
+    for out, cache in zip(got, (kc, vc)):
+        assert np.array_equal(bits(out).reshape(-1, nh, hd), ko.paged_to_linear(bits(cache), slots))
+    kc_d, vc_d = kc.to(DEV), vc.to(DEV)
+    musa_aiter.kv_reshape_and_cache_back_flash(dk.to(DEV), dv.to(DEV), kc_d, vc_d, t_d, l_d)
+    for cache, cache_d, dense in ((kc, kc_d, dk), (vc, vc_d, dv)):
+        want = bits(cache).copy()
+        ko.linear_to_paged(bits(dense).reshape(-1, nh, hd), want, slots)
+        assert np.array_equal(bits(cache_d), want)
