@@ -42,6 +42,36 @@ __device__ __forceinline__ int64_t slot_at(const TileArgs& a, int64_t t) {
 
 constexpr int kTileTokens = 16;
 
+// Cache columns of a per-wave kernel's BS-column unit: a block of 16 or 32
+// columns, or with BS = 64 the 64 columns of a block whose size is any
+// multiple of 64 (consecutive rows then lie block_size elements apart).  Slot
+// s lies in unit s / BS either way.
+template <int ELT, int BS>
+__device__ __forceinline__ uint32_t unit_pitch(const TileArgs& a) {
+  if constexpr (BS < 64) return BS * ELT;
+  else return static_cast<uint32_t>(a.block_size) * ELT;
+}
+
+// Byte offset of row `row` of unit `unit` inside its plane.
+template <int ELT, int BS>
+__device__ __forceinline__ int64_t unit_row_offset(const TileArgs& a, int64_t unit, int64_t row) {
+  if constexpr (BS < 64) {
+    return (unit * a.nrows + row) * (BS * ELT);
+  } else {
+    const int64_t units = a.block_size / BS;
+    const int64_t blk = unit / units;
+    return ((blk * a.nrows + row) * a.block_size + (unit - blk * units) * BS) * ELT;
+  }
+}
+
+// Length of the run starting at lane i, given the continuation bits of its
+// 64-token window and of the 64 tokens after it (`hi`, 0 where a run cannot
+// reach them).
+__device__ __forceinline__ int run_length(uint64_t lo, uint64_t hi, int i) {
+  const int n = i < 63 ? __builtin_ctzll(~(lo >> (i + 1))) : 0;  // the shift fills with zeros
+  return i + 1 + n < 64 ? 1 + n : 1 + n + __builtin_ctzll(~hi);  // a unit ends before `hi` runs out
+}
+
 // Small scatters resolve repeated destinations without the claim pass (one
 // launch and one dependent load fewer): every workgroup maps each slot of the
 // call to the last token that writes it, in LDS -- open addressing over
@@ -170,5 +200,28 @@ hipError_t launch_wide(const TileArgs& a, int64_t planes, bool lines, hipStream_
 // Largest block size launch_wide takes: its 32-bit offsets span a workgroup's
 // rows (at most 64) at a row pitch of block_size elements.
 constexpr int64_t kWideMaxBlockSize = 65536;
+
+// Scatters into wide blocks (64-column units) of at most 2,048 tokens x planes,
+// or 128 tokens of any number of planes, take kWideFewScatterTile-token tiles:
+// more, shorter waves.  One layer, 64-token pages: 1,000 tokens of whole
+// sequences 12.1 us (FP8) and 11.3 us (bf16) with 8-token tiles, 12.6 and 11.5
+// with 16; 4,000 tokens 19.0 us with 16, 16.0 with 64.
+constexpr int kWideFewScatterTile = 8;
+constexpr bool wide_scatter_few(int64_t tokens, int64_t planes) { return tokens * planes <= 2048 || tokens <= 128; }
+
+// Small calls on wide blocks that stay with the element kernel, whose one
+// element per thread spreads single tokens over more waves (tokens x planes;
+// one layer, 64-token pages, element against wide kernels).  Scatters: 256
+// single tokens 11.6 us against 13.2 (bf16) and 11.9 against 15.3 (FP8), 500
+// level for bf16 and 19.7 against 20.8 for FP8; at 128 the wide kernels win
+// (11.4 -> 8.6 and 12.0 -> 9.8 us), past 600 both wait for the memory's
+// partial-line writes, and whole sequences are level at 600 and faster from
+// 1,000 (16.4 -> 11.3 us).  Gathers: 128 single tokens 7.2 us against 8.3
+// (bf16) and 7.3 against 9.8 (FP8), 300 tokens of whole sequences level at 7
+// us, 2,000 20.3 -> 7.0 us.
+constexpr bool wide_scatter_wins(int64_t tokens, int64_t planes) {
+  return tokens * planes <= 256 || tokens * planes > 1200;
+}
+constexpr bool wide_gather_wins(int64_t tokens, int64_t planes) { return tokens * planes > 600; }
 
 }  // namespace kvhip

@@ -733,7 +733,8 @@ hipError_t dispatch_bs(const TileArgs& a, int64_t bs, bool fast, int64_t planes,
       if (bs == 8) return launch_tile<ELT_C, 8, SCATTER>(a, planes, stream);
       if (bs == 16) return launch_tile<ELT_C, 16, SCATTER>(a, planes, stream);
       if (bs == 32) return launch_tile<ELT_C, 32, SCATTER>(a, planes, stream);
-      if (bs % (128 / ELT_C) == 0 && bs <= kWideMaxBlockSize)
+      if (bs % (128 / ELT_C) == 0 && bs <= kWideMaxBlockSize && 
+          (SCATTER ? wide_scatter_wins(a.num_tokens, planes) : wide_gather_wins(a.num_tokens, planes)))
         return launch_wide<ELT_C, SCATTER>(a, planes, linear_rows_whole_lines(a, ELT_C), stream);
     } else if constexpr (!SCATTER) {
       // FP8 dequant-gather: per-wave kernel (kv_paged_waves.hip), unless a chunk
@@ -741,11 +742,15 @@ hipError_t dispatch_bs(const TileArgs& a, int64_t bs, bool fast, int64_t planes,
       hipError_t err = hipErrorNotSupported;
       if (bs == 16) err = launch_wave_gather<ELT_C, ELT_L, CODEC, LDT, 16>(a, planes, stream);
       if (bs == 32) err = launch_wave_gather<ELT_C, ELT_L, CODEC, LDT, 32>(a, planes, stream);
+      if (bs % 64 == 0 && bs <= kWideMaxBlockSize && wide_gather_wins(a.num_tokens, planes))
+        err = launch_wave_gather<ELT_C, ELT_L, CODEC, LDT, 64>(a, planes, stream);
       if (err != hipErrorNotSupported) return err;
     } else {
       // FP8 quant-store: per-wave kernel (kv_paged_waves.hip).
       if (bs == 16) return launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 16>(a, planes, stream);
       if (bs == 32) return launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 32>(a, planes, stream);
+      if (bs % 64 == 0 && bs <= kWideMaxBlockSize && wide_scatter_wins(a.num_tokens, planes))
+        return launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 64>(a, planes, stream);
     }
   }
   // The element kernel checks claim tags only: a call without them takes the

@@ -115,34 +115,35 @@ struct WaveShape {
 // buffer descriptor of its block column (no records for a token that does
 // not move), its value from the head's decode table, and the element to the
 // token's linear row.  `lut_off[m]` is the offset of row m's table.  Lane
-// i + 1 of `s` holds the slot of token t0 + i; bit i + 1 of `vw` says that the
-// token moves.
-template <int ELT_L, int BS, int M, typename LutT>
+// i + LEAD of `s` holds the slot of token t0 + i (i < TT); bit i + LEAD of `vw`
+// says that the token moves.
+template <int ELT_L, int BS, int TT, int LEAD, int M, typename LutT>
 __device__ __forceinline__ void dequant_token_rows(const TileArgs& a, const uint8_t* cache, uint8_t* lin,
                                                    const LutT* lut_all, const int (&lut_off)[M], int64_t s,
                                                    uint64_t vw, int64_t t0, int64_t r0, int64_t r_end) {
   constexpr int TB = 32 / M < kTileTokens ? 32 / M : kTileTokens;  // tokens per batch: 32 codes in flight per lane
-  static_assert(kTileTokens % TB == 0, "whole batches");
+  static_assert(TT % TB == 0, "whole batches");
   int lane = lane_id();
   asm volatile("" : "+v"(lane));
-  const int64_t blk = s / BS;
-  const int64_t cbase = (blk * a.nrows + r0) * BS + (s - blk * BS);
+  const int64_t unit = s / BS;
+  const int64_t cbase = unit_row_offset<1, BS>(a, unit, r0) + (s - unit * BS);
+  const int pitch = static_cast<int>(unit_pitch<1, BS>(a));
   uint8_t* const lin0 = lin + t0 * a.lin_token_stride + r0 * ELT_L;
   const int rows = static_cast<int>(r_end - r0);
   auto off = [&](int m, int bytes) -> uint32_t {
     return m * kWave + lane < rows ? static_cast<uint32_t>((m * kWave + lane) * bytes) : kOffOob;
   };
-  auto records = [&](int i) -> int { return ((vw >> (i + 1)) & 1ull) ? 0x7FFFFFFF : 0; };
+  auto records = [&](int i) -> int { return ((vw >> (i + LEAD)) & 1ull) ? 0x7FFFFFFF : 0; };
 #pragma unroll 1
-  for (int i0 = 0; i0 < kTileTokens; i0 += TB) {
-    if (((vw >> (i0 + 1)) & ((1ull << TB) - 1ull)) == 0) continue;
+  for (int i0 = 0; i0 < TT; i0 += TB) {
+    if (((vw >> (i0 + LEAD)) & ((1ull << TB) - 1ull)) == 0) continue;
     uint32_t code[TB][M];
 #pragma unroll
     for (int k = 0; k < TB; ++k) {
-      const buf_t src = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(cache) + readlane64(cbase, i0 + k + 1), 0,
-                                                          records(i0 + k), 0x00020000);
+      const buf_t src = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<uint8_t*>(cache) + readlane64(cbase, i0 + k + LEAD), 0, records(i0 + k), 0x00020000);
 #pragma unroll
-      for (int m = 0; m < M; ++m) code[k][m] = __builtin_amdgcn_raw_buffer_load_b8(src, off(m, BS), 0, 0);
+      for (int m = 0; m < M; ++m) code[k][m] = __builtin_amdgcn_raw_buffer_load_b8(src, off(m, pitch), 0, 0);
     }
 #pragma unroll
     for (int k = 0; k < TB; ++k) {
@@ -164,11 +165,68 @@ __device__ __forceinline__ void dequant_token_rows(const TileArgs& a, const uint
 constexpr int64_t kTokenDequantTokens = 256;
 constexpr int kShortDequantRunTokens = 3;
 
-template <int ELT_C, int ELT_L, int CODEC, int LDT, int BS, int STP, bool TOKG = false>
+// Slot window of a tile of TT tokens.  Units of at most 32 columns: lane i holds
+// token t0 - 1 + i (LEAD = 1), and every run that starts in the tile ends inside
+// the wave.  64-column units: lane i holds token t0 + i, and a second register
+// the 64 tokens after them; the tile is one unit long (TT = 64: with 16 tokens
+// three of four waves would find no run to start), shorter in small calls
+// (more, shorter waves for a decode step).
+template <int BS>
+constexpr int kWindowLead = BS < 64 ? 1 : 0;
+
+// The window's continuation bits (see run_length): token t continues token
+// t - 1 when both are valid and lie in consecutive slots of one unit.
+struct Window {
+  uint64_t valid, lo, hi;
+};
+
+// `s`: this lane's slot; `usable(slot, t)`: token t moves.
+template <int BS, typename Usable>
+__device__ __forceinline__ Window slot_window(const TileArgs& a, int64_t t0, int64_t s, Usable usable) {
+  const int lane = lane_id();
+  auto continues = [](int64_t slot, int64_t before) { return slot == before + 1 && (slot % BS) != 0; };
+  Window w;
+  const bool valid = usable(s, t0 - kWindowLead<BS> + lane);
+  w.valid = ballot(valid);
+  // The lane shuffles run in every lane: a lane switched off by a condition
+  // would hand its neighbour nothing.
+  const int64_t s_prev = from_prev_lane(s);
+  if constexpr (BS < 64) {
+    const bool prev_valid = lane > 0 && ((w.valid >> (lane - 1)) & 1ull);
+    w.lo = ballot(valid && prev_valid && continues(s, s_prev));
+    w.hi = 0;
+  } else {
+    auto slot_of = [&](int64_t t) -> int64_t { return t >= 0 && t < a.num_tokens ? slot_at(a, t) : -1; };
+    const int64_t before = slot_of(t0 - 1);
+    const int64_t s_hi = slot_of(t0 + kWave + lane);
+    const bool valid_hi = usable(s_hi, t0 + kWave + lane);
+    const uint64_t pv = (w.valid << 1) | (usable(before, t0 - 1) ? 1ull : 0ull);
+    const uint64_t pv_hi = (ballot(valid_hi) << 1) | (w.valid >> 63);
+    const int64_t s_hi_prev = from_prev_lane(s_hi);
+    const int64_t last = readlane64(s, 63);
+    const int64_t prev = lane == 0 ? before : s_prev;
+    const int64_t prev_hi = lane == 0 ? last : s_hi_prev;
+    w.lo = ballot(valid && ((pv >> lane) & 1ull) && continues(s, prev));
+    w.hi = ballot(valid_hi && ((pv_hi >> lane) & 1ull) && continues(s_hi, prev_hi));
+  }
+  return w;
+}
+
+// Bits of the tile's own tokens (at most TT of the call's remaining ones).
+template <int BS, int TT>
+__device__ __forceinline__ uint64_t tile_bits(int64_t remaining) {
+  if (remaining <= 0) return 0;
+  const uint64_t n = remaining < TT ? (1ull << remaining) - 1ull : ~0ull >> (64 - TT);
+  return n << kWindowLead<BS>;
+}
+
+template <int ELT_C, int ELT_L, int CODEC, int LDT, int BS, int STP, bool TOKG = false,
+          int TT = (BS < 64 ? kTileTokens : BS)>
 __global__ __launch_bounds__(kBlockThreads) void paged_wave_gather_kernel(const TileArgs a) {
   using W = WaveShape<ELT_C, ELT_L, BS>;
   constexpr int RPL = W::RPL, CG = W::CG, NCG = W::NCG, kChunkRows = W::kChunkRows;
-  static_assert(kTileTokens + BS + 1 <= kWave, "run window must fit one wave");
+  constexpr int LEAD = kWindowLead<BS>;
+  static_assert(BS == 64 || TT + BS + LEAD <= kWave, "run window must fit one wave");
   using LutT = typename LutEntry<ELT_L>::T;
   constexpr bool kLut = CODEC != kCopy;
   // Full runs stage the chunk through LDS (copies) or load lane tiles
@@ -180,26 +238,21 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_gather_kernel(const 
 
   const int lane = lane_id();
   const int64_t tile = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + wave_in_block();
-  const int64_t t0 = tile * kTileTokens;
+  const int64_t t0 = tile * TT;
   const int plane = static_cast<int>(blockIdx.y);
   const int layer = plane >> 1;
   const int kv = plane & 1;
   const int64_t r0 = static_cast<int64_t>(blockIdx.z) * kChunkRows;  // this wave's cache rows
   const int64_t r_end = (r0 + kChunkRows < a.nrows) ? r0 + kChunkRows : a.nrows;
 
-  // Slot window: lane i holds token t0 - 1 + i, and the runs of the tile.
-  const int64_t t = t0 - 1 + lane;
+  // The slot window and the runs of the tile.
+  const int64_t t = t0 - LEAD + lane;
   int64_t s = -1;
   if (t >= 0 && t < a.num_tokens) s = slot_at(a, t);
-  const bool valid = (s >= 0) && (s < a.num_slots);
-  const uint64_t vmask = ballot(valid);
-  const int64_t s_prev = from_prev_lane(s);
-  const bool prev_valid = lane > 0 && ((vmask >> (lane - 1)) & 1ull);
-  const bool cont = valid && prev_valid && (s == s_prev + 1) && ((s % BS) != 0);
-  const uint64_t cmask = ballot(cont);
-  const int64_t remaining = a.num_tokens - t0;
-  const int ntile = remaining <= 0 ? 0 : (remaining < kTileTokens ? static_cast<int>(remaining) : kTileTokens);
-  const uint64_t window = ((1ull << ntile) - 1ull) << 1;
+  const Window win =
+      slot_window<BS>(a, t0, s, [&](int64_t slot, int64_t) { return slot >= 0 && slot < a.num_slots; });
+  const uint64_t vmask = win.valid, cmask = win.lo;
+  const uint64_t window = tile_bits<BS, TT>(a.num_tokens - t0);
   uint64_t heads = vmask & ~cmask & window;
 
   uint8_t* const cache = a.cache[kv] + static_cast<int64_t>(layer) * a.cache_layer_stride;
@@ -208,29 +261,38 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_gather_kernel(const 
   const int ct = lane % NCG;
   const int64_t trow = r0 + rg * RPL;
   const bool tile_in = trow < r_end;
-  const uint32_t toff = static_cast<uint32_t>((rg * RPL * NCG + ct) * 16);
+  const uint32_t pitch = unit_pitch<ELT_C, BS>(a);
+  const uint32_t toff = static_cast<uint32_t>(rg * RPL) * pitch + static_cast<uint32_t>(ct) * 16u;
 
-  // One run starting at lane i of the window: its block, columns and first token.
+  // One run starting at lane i of the window: its unit, columns and first token.
   struct Run {
     int64_t blk, tf;
     int c0, c1;
   };
   auto run_at = [&](int i) {
-    const int len = 1 + __builtin_ctzll(~(cmask >> (i + 1)));  // i <= kTileTokens < 63
+    const int len = run_length(cmask, win.hi, i);
     const int64_t sh = readlane64(s, i);
     const int64_t blk = sh / BS;
     const int c0 = static_cast<int>(sh - blk * BS);
-    return Run{blk, t0 - 1 + i, c0, c0 + len};
+    return Run{blk, t0 - LEAD + i, c0, c0 + len};
   };
-  auto whole_chunk = [&](const Run& r) { return r.c0 < CG && r.c1 > BS - CG; };
+  // Runs that take the whole-chunk form: those that touch every column group,
+  // and in 64-column units all of them (groups outside the run are not loaded).
+  auto whole_chunk = [&](const Run& r) { return BS == 64 || (r.c0 < CG && r.c1 > BS - CG); };
   // FP8: each lane loads its own tile, RPL pieces 16 * NCG bytes apart.  A wave
   // instruction touches 64 lines partially; the loads are cached so that the L2
   // serves the rest of each line to the wave's next instructions.
   auto load_tile = [&](const Run& r, u32x4 (&d)[RPL]) {
-    const buf_t cb = make_buf(cache + (r.blk * a.nrows + r0) * BS * ELT_C);
+    const buf_t cb = make_buf(cache + unit_row_offset<ELT_C, BS>(a, r.blk, r0));
+    if constexpr (BS < 64) {
 #pragma unroll
-    for (int q = 0; q < RPL; ++q)
-      d[q] = buf_ld16_cached(cb, tile_in ? toff + static_cast<uint32_t>(q * NCG * 16) : kOffOob);
+      for (int q = 0; q < RPL; ++q)
+        d[q] = buf_ld16_cached(cb, tile_in ? toff + static_cast<uint32_t>(q * NCG * 16) : kOffOob);
+    } else {
+      const uint32_t off = tile_in && ct * CG < r.c1 && ct * CG + CG > r.c0 ? toff : kOffOob;
+#pragma unroll
+      for (int q = 0; q < RPL; ++q) d[q] = buf_ld16_cached(cb, off + static_cast<uint32_t>(q) * pitch);
+    }
   };
 
   // FP8: the first run's tile is loaded before the workgroup builds its decode
@@ -285,7 +347,8 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_gather_kernel(const 
     // next bit carries through in cmask.
     const uint64_t owned = heads | (((cmask + (heads << 1)) ^ cmask) & cmask);
     const int nr = __builtin_popcountll(heads);
-    if (nr > 0 && (owned & ~window) == 0 && __builtin_popcountll(owned) < nr * kShortDequantRunTokens) {
+    const bool goes_on = TT == 64 ? (win.hi & 1ull) : (owned & ~window) != 0;
+    if (nr > 0 && !goes_on && __builtin_popcountll(owned) < nr * kShortDequantRunTokens) {
       constexpr int M = kChunkRows / kWave;
       static_assert(kChunkRows % kWave == 0, "whole rows per lane");
       int lut_off[M];
@@ -294,7 +357,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_gather_kernel(const 
         const int64_t row = r0 + m * kWave + lane;
         lut_off[m] = (a.scale_mode != 0 && row < r_end) ? (head_of_row(a, static_cast<int>(row)) - h_lo) * 256 : 0;
       }
-      dequant_token_rows<ELT_L, BS, M, LutT>(a, cache, lin, lut_all, lut_off, s, owned, t0, r0, r_end);
+      dequant_token_rows<ELT_L, BS, TT, LEAD, M, LutT>(a, cache, lin, lut_all, lut_off, s, owned, t0, r0, r_end);
       heads = 0;
     }
   }
@@ -353,7 +416,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_gather_kernel(const 
       const int64_t gr = static_cast<int64_t>(g) * RPL;
       const LutT* glut = lut_all;
       if (kLut && a.scale_mode != 0) glut += (head_of_row(a, static_cast<int>(gr)) - h_lo) * 256;
-      uint8_t* const crow = cache + (blk * a.nrows + gr) * BS * ELT_C;
+      uint8_t* const crow = cache + unit_row_offset<ELT_C, BS>(a, blk, gr);
       uint8_t* const grow = lin + tf * a.lin_token_stride + gr * ELT_L;
 #pragma unroll 1
       for (int j = j0; j <= j1; ++j) {
@@ -378,7 +441,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_gather_kernel(const 
     while (skipped) {
       const int i = __builtin_ctzll(skipped);
       skipped &= skipped - 1;
-      uint8_t* const row = lin + (t0 - 1 + i) * a.lin_token_stride;
+      uint8_t* const row = lin + (t0 - LEAD + i) * a.lin_token_stride;
       for (int64_t k = r0 * ELT_L + static_cast<int64_t>(lane) * 16; k < r_end * ELT_L; k += kWave * 16)
         st16(row + k, zero);
     }
@@ -486,13 +549,13 @@ __device__ __forceinline__ float tile_elem(const u32x4& piece, int q) {
 // records for a token that does not move) and a wave instruction covers 64
 // consecutive rows: 64 elements of the linear row, 64 bytes of the block
 // column at a row stride.  Every element is encoded on its own, as the
-// element path of the run form does.  Lane i + 1 of `s` holds the slot of
-// token t0 + i; bit i + 1 of `vw` says that the token moves.
-template <int CODEC, int LDT, int ELT_L, int BS, int M>
+// element path of the run form does.  Lane i + LEAD of `s` holds the slot of
+// token t0 + i (i < TT); bit i + LEAD of `vw` says that the token moves.
+template <int CODEC, int LDT, int ELT_L, int BS, int TT, int LEAD, int M>
 __device__ __forceinline__ void quant_token_rows(const TileArgs& a, uint8_t* cache, const uint8_t* lin, int kv,
                                                  int layer, int64_t s, uint64_t vw, int64_t t0, int r0, int r_end) {
-  constexpr int TB = 16 / M < kTileTokens ? 16 / M : kTileTokens;  // tokens per batch: 16 elements in flight per lane
-  static_assert(kTileTokens % TB == 0, "whole batches");
+  constexpr int TB = 16 / M < TT ? 16 / M : TT;  // tokens per batch: at most 16 elements in flight per lane
+  static_assert(TT % TB == 0, "whole batches");
   // The lane id and slot pass through an opaque copy, so that nothing derived
   // from them is hoisted out of the caller's chunk loop (it would stay live
   // across the run form and cost it a wave per SIMD).
@@ -509,13 +572,14 @@ __device__ __forceinline__ void quant_token_rows(const TileArgs& a, uint8_t* cac
   auto off = [&](int m, int bytes) -> uint32_t {
     return r0 + m * kWave + lane < r_end ? static_cast<uint32_t>((m * kWave + lane) * bytes) : kOffOob;
   };
-  const int64_t blk = s / BS;
-  const int64_t cbase = (blk * a.nrows + r0) * BS + (s - blk * BS);
+  const int64_t unit = s / BS;
+  const int64_t cbase = unit_row_offset<1, BS>(a, unit, r0) + (s - unit * BS);
+  const int pitch = static_cast<int>(unit_pitch<1, BS>(a));
   const uint8_t* const lin0 = lin + t0 * a.lin_token_stride + static_cast<int64_t>(r0) * ELT_L;
-  auto records = [&](int i) -> int { return ((vw >> (i + 1)) & 1ull) ? 0x7FFFFFFF : 0; };
+  auto records = [&](int i) -> int { return ((vw >> (i + LEAD)) & 1ull) ? 0x7FFFFFFF : 0; };
 #pragma unroll 1
-  for (int i0 = 0; i0 < kTileTokens; i0 += TB) {
-    if (((vw >> (i0 + 1)) & ((1ull << TB) - 1ull)) == 0) continue;
+  for (int i0 = 0; i0 < TT; i0 += TB) {
+    if (((vw >> (i0 + LEAD)) & ((1ull << TB) - 1ull)) == 0) continue;
     uint32_t v[TB][M];
 #pragma unroll
     for (int k = 0; k < TB; ++k) {
@@ -530,7 +594,7 @@ __device__ __forceinline__ void quant_token_rows(const TileArgs& a, uint8_t* cac
     }
     auto elem = [&](uint32_t bits) { return ELT_L == 2 ? lin_to_f32<LDT>(bits) : __uint_as_float(bits); };
     auto cdesc = [&](int k) {
-      return __builtin_amdgcn_make_buffer_rsrc(cache + readlane64(cbase, i0 + k + 1), 0, records(i0 + k),
+      return __builtin_amdgcn_make_buffer_rsrc(cache + readlane64(cbase, i0 + k + LEAD), 0, records(i0 + k),
                                                0x00020000);
     };
     // The fast quotient's range (quant_one's test), for the whole batch at once.
@@ -551,7 +615,7 @@ __device__ __forceinline__ void quant_token_rows(const TileArgs& a, uint8_t* cac
 #pragma unroll
         for (int m = 0; m < M; ++m) {
           const uint32_t code = fp8_encode_fast<CODEC>(quot_fast<LDT != kLinF32>(elem(v[k][m]), sc[m], rc[m]));
-          __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(code), dst, off(m, BS), 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(code), dst, off(m, pitch), 0, 0);
         }
       }
     } else {
@@ -574,7 +638,7 @@ __device__ __forceinline__ void quant_token_rows(const TileArgs& a, uint8_t* cac
             rcm = m == j ? rc[j] : rcm;
           }
           const uint32_t code = quant_one<CODEC, LDT>(elem(x), scm, rcm, fast_scale_ok(scm));
-          __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(code), dst, off(m, BS), 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(code), dst, off(m, pitch), 0, 0);
         }
       }
     }
@@ -595,13 +659,15 @@ constexpr int kQuantShortRunTokens = 6;
 // scatter (see paged_block_scatter_kernel): the cache is then written in
 // address order, and a workgroup reads its block's linear rows and writes its
 // cache bytes as one contiguous span each.
-template <int ELT_C, int ELT_L, int CODEC, int LDT, int BS, bool BM>
+// TT: tokens of a tile in token order (see paged_wave_gather_kernel).
+template <int ELT_C, int ELT_L, int CODEC, int LDT, int BS, bool BM, int TT = (BS < 64 ? kTileTokens : BS)>
 __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const TileArgs a) {
   static_assert(ELT_C == 1 && CODEC != kCopy, "the per-wave scatter quantises into one-byte caches");
   using W = ScatterShape<ELT_L, BS>;
   constexpr int RPL = W::RPL, CG = W::CG, NCG = W::NCG, COLS = W::COLS;
   constexpr int kChunkRows = W::kChunkRows, kPieces = W::kPieces;
-  static_assert(kTileTokens + BS + 1 <= kWave, "run window must fit one wave");
+  constexpr int LEAD = kWindowLead<BS>;
+  static_assert(BS == 64 || TT + BS + LEAD <= kWave, "run window must fit one wave");
   __shared__ u32x4 lds_all[kWavesPerBlock * kPieces];
   u32x4* const lds = lds_all + wave_in_block() * kPieces;
 
@@ -637,31 +703,31 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
 
   // Runs: `heads` marks the first lane of each, `cmask` the lanes continuing
   // one.
-  uint64_t heads, cmask;
+  uint64_t heads, cmask, cmask_hi = 0;
   uint64_t tok_lanes = 0;  // token order: lanes whose tokens take quant_token_rows
   int64_t s = -1, tok = -1;
-  const int64_t t0 = unit * kTileTokens;
+  const int64_t t0 = unit * TT;
   if constexpr (!BM) {
-    // Slot window: lane i holds token t0 - 1 + i; a token whose claim lost to a
-    // later duplicate writes nothing.  The duplicate table is built by every
-    // wave of the workgroup, before any of them leaves.
+    // The slot window; a token whose claim lost to a later duplicate writes
+    // nothing.  The duplicate table is built by every wave of the workgroup,
+    // before any of them leaves.
     if (a.scan_dupes) scan_build<kBlockThreads>(scan_table(), a);
     if (t0 >= a.num_tokens) return;
-    const int64_t t = t0 - 1 + lane;
+    const int64_t t = t0 - LEAD + lane;
     if (t >= 0 && t < a.num_tokens) s = slot_at(a, t);
-    bool valid = (s >= 0) && (s < a.num_slots);
-    if (a.scan_dupes) {
-      if (valid) valid = scan_is_last(scan_table(), s, t);
-    } else if (valid && a.owner != nullptr) {
-      valid = (a.owner[s] == claim_tag(a.epoch, t));
-    }
-    const uint64_t vmask = ballot(valid);
-    const int64_t s_prev = from_prev_lane(s);
-    const bool prev_valid = lane > 0 && ((vmask >> (lane - 1)) & 1ull);
-    cmask = ballot(valid && prev_valid && (s == s_prev + 1) && ((s % BS) != 0));
-    const int64_t remaining = a.num_tokens - t0;
-    const int ntile = remaining < kTileTokens ? static_cast<int>(remaining) : kTileTokens;
-    const uint64_t window = ((1ull << ntile) - 1ull) << 1;
+    const Window win = slot_window<BS>(a, t0, s, [&](int64_t slot, int64_t tk) {
+      bool valid = (slot >= 0) && (slot < a.num_slots);
+      if (a.scan_dupes) {
+        if (valid) valid = scan_is_last(scan_table(), slot, tk);
+      } else if (valid && a.owner != nullptr) {
+        valid = (a.owner[slot] == claim_tag(a.epoch, tk));
+      }
+      return valid;
+    });
+    const uint64_t vmask = win.valid;
+    cmask = win.lo;
+    cmask_hi = win.hi;
+    const uint64_t window = tile_bits<BS, TT>(a.num_tokens - t0);
     heads = vmask & ~cmask & window;
     // Lanes of the runs that start in this tile: adding a head's next bit to
     // cmask carries through exactly the continuation bits of its run.  A last
@@ -669,7 +735,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
     // before it move with quant_token_rows.
     uint64_t tok_heads = heads;
     tok_lanes = heads | (((cmask + (heads << 1)) ^ cmask) & cmask);
-    if (tok_lanes & ~window) {
+    if (heads != 0 && (TT == 64 ? (cmask_hi & 1ull) != 0 : (tok_lanes & ~window) != 0)) {
       const uint64_t below_last = (1ull << (63 - __builtin_clzll(heads))) - 1ull;
       tok_heads &= below_last;
       tok_lanes &= below_last;
@@ -696,10 +762,10 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
   for (int r0 = rw0; r0 < rw_end; r0 += kChunkRows) {
     const int r_end = (r0 + kChunkRows < rw_end) ? r0 + kChunkRows : rw_end;
     if constexpr (!BM) {
-      static_assert(kChunkRows % kWave == 0, "whole rows per lane");
+      constexpr int M = (kChunkRows + kWave - 1) / kWave;
+      static_assert(kChunkRows % kWave == 0 || M == 1, "whole rows per lane, or one masked row");
       if (tok_lanes != 0)
-        quant_token_rows<CODEC, LDT, ELT_L, BS, kChunkRows / kWave>(a, cache, lin, kv, layer, s, tok_lanes, t0, r0,
-                                                                    r_end);
+        quant_token_rows<CODEC, LDT, ELT_L, BS, TT, LEAD, M>(a, cache, lin, kv, layer, s, tok_lanes, t0, r0, r_end);
     }
     const float sc = r0 == rw0 ? sc_first : chunk_scale(r0);
     const bool scale_ok = fast_scale_ok(sc);
@@ -720,7 +786,8 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
       const int trow = r0 + rg * RPL;
       const bool tile_in = trow < r_end;
       u32x2* const lds_half = reinterpret_cast<u32x2*>(lds) + half;
-      uint8_t* const chunk = cache + (blk * a.nrows + r0) * BS;
+      uint8_t* const chunk = cache + unit_row_offset<1, BS>(a, blk, r0);
+      const uint32_t pitch = unit_pitch<1, BS>(a);
       const bool whole = c0 == 0 && c1 == BS;
       // Linear pieces: a descriptor at the run's first token and row r0 and a
       // per-lane offset (row group, column); lanes past the chunk, and columns
@@ -772,14 +839,16 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
           const int pc = k * kWave + lane;
           const u32x4 v = lds[lds_slot<RPL, NCG>(pc)];
           const bool row_in = r0 + pc / NCG < r_end;
+          const uint32_t coff = BS < 64 ? static_cast<uint32_t>(pc) * 16u
+                                        : static_cast<uint32_t>(pc / NCG) * pitch + static_cast<uint32_t>(pc % NCG) * 16u;
           if (whole) {
-            buf_st16(cbuf, row_in ? static_cast<uint32_t>(pc) * 16u : kOffOob, v);
+            buf_st16(cbuf, row_in ? coff : kOffOob, v);
           } else if (row_in) {
             // The piece's bytes inside the run: [b0, b1) of its 16 columns.
             const int cg0 = (pc % NCG) * CG;
             const int b0 = c0 > cg0 ? c0 - cg0 : 0;
             const int b1 = c1 < cg0 + CG ? c1 - cg0 : CG;
-            uint8_t* const p = chunk + static_cast<int64_t>(pc) * 16;
+            uint8_t* const p = chunk + coff;
 #pragma unroll 1
             for (int b = b0; b < b1; ++b) {
               const uint32_t d = (b >> 2) == 0 ? v[0] : (b >> 2) == 1 ? v[1] : (b >> 2) == 2 ? v[2] : v[3];
@@ -799,7 +868,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
       if (!tile_in) return;
       const int ja = c0 > lo ? c0 - lo : 0;
       const int jb = c1 < lo + COLS ? c1 - lo : COLS;
-      uint8_t* const crow = chunk + static_cast<int64_t>(rg * RPL) * BS + lo;
+      uint8_t* const crow = chunk + static_cast<int64_t>(rg * RPL) * pitch + lo;
 #pragma unroll 1
       for (int j = ja; j < jb; ++j) {
         u32x4 piece = in[0];
@@ -807,7 +876,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
         for (int k = 1; k < COLS; ++k) piece = (j == k) ? in[k] : piece;
 #pragma unroll 1
         for (int q = 0; q < RPL; ++q)
-          crow[q * BS + j] =
+          crow[static_cast<int64_t>(q) * pitch + j] =
               static_cast<uint8_t>(quant_one<CODEC, LDT>(tile_elem<ELT_L, LDT, RPL>(piece, q), sc, r, scale_ok));
       }
     };
@@ -816,12 +885,12 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
     while (hs) {
       const int i = __builtin_ctzll(hs);
       hs &= hs - 1;
-      const int len = 1 + __builtin_ctzll(~(cmask >> (i + 1)));  // i < 63
+      const int len = run_length(cmask, cmask_hi, i);
       if constexpr (!BM) {
         const int64_t sh = readlane64(s, i);
         const int64_t blk = sh / BS;
         const int c0 = static_cast<int>(sh - blk * BS);
-        run(blk, c0, c0 + len, t0 - 1 + i);
+        run(blk, c0, c0 + len, t0 - LEAD + i);
       } else {
         run(unit, i, i + len, readlane64(tok, i));
       }
@@ -968,7 +1037,10 @@ hipError_t launch_wave_gather(const TileArgs& a, int64_t planes, hipStream_t str
       if (r1 / a.head_dim - r0 / a.head_dim + 1 > kLutHeads) return hipErrorNotSupported;
     }
   }
-  const int64_t tiles = (a.num_tokens + kTileTokens - 1) / kTileTokens;
+  // (The form costs 64-column units nothing; the others compile it apart.)
+  const bool tok = BS == 64 || a.num_tokens <= kTokenDequantTokens;
+  constexpr int tt = BS < 64 ? kTileTokens : BS;
+  const int64_t tiles = (a.num_tokens + tt - 1) / tt;
   const int64_t blocks = (tiles + kWavesPerBlock - 1) / kWavesPerBlock;
   if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
   const dim3 grid(static_cast<uint32_t>(blocks), static_cast<uint32_t>(planes), static_cast<uint32_t>(chunks));
@@ -982,19 +1054,18 @@ hipError_t launch_wave_gather(const TileArgs& a, int64_t planes, hipStream_t str
   // FP8 preload -0.3-0.5 %;
   // 5 per CU was 2-5 % slower, and staging the tiles through LDS with
   // whole-line loads gained 1.6 % on cfg 3 but lost 6 % on the dense preload.
-  const bool tok = a.num_tokens <= kTokenDequantTokens;
   if (whole_line_rows(a, ELT_L) && tok)
     hipLaunchKernelGGL((paged_wave_gather_kernel<ELT_C, ELT_L, CODEC, LDT, BS, kBufWT, true>), grid,
                        dim3(kBlockThreads), kGatherLdsPad, stream, a);
   else if (whole_line_rows(a, ELT_L))
-    hipLaunchKernelGGL((paged_wave_gather_kernel<ELT_C, ELT_L, CODEC, LDT, BS, kBufWT>), grid, dim3(kBlockThreads),
-                       kGatherLdsPad, stream, a);
+    hipLaunchKernelGGL((paged_wave_gather_kernel<ELT_C, ELT_L, CODEC, LDT, BS, kBufWT, BS == 64>), grid,
+                       dim3(kBlockThreads), kGatherLdsPad, stream, a);
   else if (tok)
     hipLaunchKernelGGL((paged_wave_gather_kernel<ELT_C, ELT_L, CODEC, LDT, BS, kBufNT, true>), grid,
                        dim3(kBlockThreads), kGatherLdsPad, stream, a);
   else
-    hipLaunchKernelGGL((paged_wave_gather_kernel<ELT_C, ELT_L, CODEC, LDT, BS, kBufNT>), grid, dim3(kBlockThreads),
-                       kGatherLdsPad, stream, a);
+    hipLaunchKernelGGL((paged_wave_gather_kernel<ELT_C, ELT_L, CODEC, LDT, BS, kBufNT, BS == 64>), grid,
+                       dim3(kBlockThreads), kGatherLdsPad, stream, a);
   return hipGetLastError();
 }
 
@@ -1006,8 +1077,11 @@ hipError_t launch_wave_scatter(const TileArgs& a, int64_t planes, hipStream_t st
   // Block order when the claim tags are this call's inverse map and the tokens
   // cover a good share of the slots (as for the 16- and 32-bit scatter).
   const bool bm = a.owner != nullptr && a.owner_exclusive && a.num_tokens * 4 >= a.num_slots;
-  const int64_t blocks = bm ? a.num_slots / BS : ((a.num_tokens + kTileTokens - 1) / kTileTokens + kWavesPerBlock - 1) /
-                                                     kWavesPerBlock;
+  const bool few = BS == 64 && wide_scatter_few(a.num_tokens, planes);
+  constexpr int kFewTile = BS < 64 ? kTileTokens : kWideFewScatterTile;
+  const int tt = few ? kFewTile : BS < 64 ? kTileTokens : BS;
+  const int64_t blocks =
+      bm ? a.num_slots / BS : ((a.num_tokens + tt - 1) / tt + kWavesPerBlock - 1) / kWavesPerBlock;
   const int64_t zs = bm ? (chunks + kWavesPerBlock - 1) / kWavesPerBlock : chunks;
   if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
   const dim3 grid(static_cast<uint32_t>(blocks), static_cast<uint32_t>(planes), static_cast<uint32_t>(zs));
@@ -1028,6 +1102,9 @@ hipError_t launch_wave_scatter(const TileArgs& a, int64_t planes, hipStream_t st
   if (bm)
     hipLaunchKernelGGL((paged_wave_scatter_kernel<ELT_C, ELT_L, CODEC, LDT, BS, true>), grid, dim3(kBlockThreads), 0,
                        stream, a);
+  else if (few)
+    hipLaunchKernelGGL((paged_wave_scatter_kernel<ELT_C, ELT_L, CODEC, LDT, BS, false, kFewTile>), grid,
+                       dim3(kBlockThreads), 0, stream, a);
   else
     hipLaunchKernelGGL((paged_wave_scatter_kernel<ELT_C, ELT_L, CODEC, LDT, BS, false>), grid, dim3(kBlockThreads), 0,
                        stream, a);
@@ -1053,8 +1130,10 @@ template hipError_t launch_wave_copy_scatter<32>(const TileArgs&, int64_t, hipSt
 #define KVHIP_WAVE_GATHER(CODEC, ELT_L, LDT)                                                             \
   template hipError_t launch_wave_gather<1, ELT_L, CODEC, LDT, 16>(const TileArgs&, int64_t, hipStream_t);  \
   template hipError_t launch_wave_gather<1, ELT_L, CODEC, LDT, 32>(const TileArgs&, int64_t, hipStream_t);  \
+  template hipError_t launch_wave_gather<1, ELT_L, CODEC, LDT, 64>(const TileArgs&, int64_t, hipStream_t);  \
   template hipError_t launch_wave_scatter<1, ELT_L, CODEC, LDT, 16>(const TileArgs&, int64_t, hipStream_t); \
-  template hipError_t launch_wave_scatter<1, ELT_L, CODEC, LDT, 32>(const TileArgs&, int64_t, hipStream_t);
+  template hipError_t launch_wave_scatter<1, ELT_L, CODEC, LDT, 32>(const TileArgs&, int64_t, hipStream_t); \
+  template hipError_t launch_wave_scatter<1, ELT_L, CODEC, LDT, 64>(const TileArgs&, int64_t, hipStream_t);
 KVHIP_WAVE_GATHER(kE4M3, 2, kLinBF16)
 KVHIP_WAVE_GATHER(kE4M3, 2, kLinF16)
 KVHIP_WAVE_GATHER(kE4M3, 4, kLinF32)

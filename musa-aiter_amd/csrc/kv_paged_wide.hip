@@ -164,7 +164,7 @@ __device__ __forceinline__ void wide_token_rows(const TileArgs& a, const WaveChu
     uint8_t* const base = cache_side ? w.cache + readlane64(cbase, i) : w.lin + (t0 + i) * a.lin_token_stride;
     return __builtin_amdgcn_make_buffer_rsrc(base, 0, ((move >> i) & 1ull) ? 0x7FFFFFFF : 0, 0x00020000);
   };
-  constexpr int TB = 16;  // tokens in flight
+  constexpr int TB = TT < 16 ? TT : 16;  // tokens in flight
   static_assert(TT % TB == 0, "whole batches");
 #pragma unroll 1
   for (int i0 = 0; i0 < TT; i0 += TB) {
@@ -189,10 +189,8 @@ __device__ __forceinline__ void wide_token_rows(const TileArgs& a, const WaveChu
 
 // Tiles whose runs average fewer than this many tokens move token by token.
 constexpr int kWideShortRun = 6;
-// Launches of at most kWideFewTokens tokens take 16-token tiles (more, shorter
-// waves); gathers move tiles of short runs token by token only there.
-constexpr int64_t kWideFewTokens = 256;
-constexpr int kWideFewTile = 16;
+// Gather tiles do below this (as the narrow kernels' gathers).
+constexpr int kWideShortGatherRun = 3;
 
 __device__ __forceinline__ int64_t slot_or_none(const TileArgs& a, int64_t t) {
   return t >= 0 && t < a.num_tokens ? slot_at(a, t) : -1;
@@ -200,14 +198,22 @@ __device__ __forceinline__ int64_t slot_or_none(const TileArgs& a, int64_t t) {
 
 __device__ __forceinline__ uint64_t low_bits(int64_t n) { return n >= 64 ? ~0ull : (1ull << n) - 1ull; }
 
+// True when the runs of a tile average fewer than kWideShortGatherRun tokens:
+// `v` marks its valid tokens, `c` those that continue the token before them.
+__device__ __forceinline__ bool short_gather_tile(uint64_t v, uint64_t c) {
+  return __builtin_popcountll(v) < kWideShortGatherRun * __builtin_popcountll(v & ~c);
+}
+
 // Gather.  Grid: x = tile * row_groups + group of 4 chunks, y = plane.  A run
 // is every token of the window whose slot lies in the head's unit at the
 // head's distance from its token, so tokens skipped in between (slot < 0) do
-// not cut it; its first token's tile moves it.  FEW (TT = kWideFewTile): every
-// tile moves its own tokens only.
-template <int ELT, int TT, bool FEW, bool XCD, int STP>
+// not cut it; its first token's tile moves it.  A tile of short runs instead
+// moves its own tokens, no more, and the tile after it knows that from the
+// same slots.
+template <int ELT, bool XCD, int STP>
 __global__ __launch_bounds__(kBlockThreads) void paged_wide_gather_kernel(const TileArgs a) {
   using W = Wide<ELT>;
+  constexpr int TT = W::UC;
   const int lane = lane_id();
   const WgXyz wg = xcd_contiguous_wg<XCD>();
   const uint32_t tile = wg.x / static_cast<uint32_t>(a.row_groups);
@@ -217,22 +223,23 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wide_gather_kernel(const 
   if (w.rows == 0) return;
 
   const int64_t s = slot_or_none(a, t0 + lane);
+  const int64_t s_hi = slot_or_none(a, t0 + kWave + lane);
+  const int64_t s_pre = slot_or_none(a, t0 - kWave + lane);
   const bool valid = s >= 0 && s < a.num_slots;
+  const bool valid_pre = s_pre >= 0 && s_pre < a.num_slots;
   const uint64_t in_tile = low_bits(a.num_tokens - t0) & low_bits(TT);
   const uint64_t v_lo = ballot(valid);
   uint64_t pending = v_lo & in_tile;
-  [[maybe_unused]] int64_t s_hi = -1, s_pre = -1;
-  if constexpr (FEW) {
-    const int64_t prev = from_prev_lane(s);
-    const uint64_t c = ballot(valid && lane > 0 && s == prev + 1 && (s & (W::UC - 1)) != 0);
-    const int runs = __builtin_popcountll(pending & ~(c & ~1ull));
-    if (__builtin_popcountll(pending) < runs * kWideShortRun) {
-      wide_token_rows<ELT, false, TT>(a, w, s, pending, t0);
-      pending = 0;
-    }
-  } else {
-    s_hi = slot_or_none(a, t0 + kWave + lane);
-    s_pre = slot_or_none(a, t0 - kWave + lane);
+  // Short runs, judged on a tile's own tokens alone; the tile before is the
+  // last TT lanes of s_pre.
+  const int64_t s_prev = from_prev_lane(s), s_pre_prev = from_prev_lane(s_pre);
+  auto continues = [&](int64_t slot, int64_t before) { return slot == before + 1 && (slot & (W::UC - 1)) != 0; };
+  const uint64_t c = ballot(valid && lane > 0 && continues(s, s_prev));
+  const uint64_t c_pre = ballot(valid_pre && lane > kWave - TT && continues(s_pre, s_pre_prev));
+  const bool pre_short = short_gather_tile(ballot(valid_pre) >> (kWave - TT), c_pre >> (kWave - TT));
+  if (short_gather_tile(pending, c)) {
+    wide_token_rows<ELT, false, TT>(a, w, s, pending, t0);
+    pending = 0;
   }
   while (pending) {
     const int i = __builtin_ctzll(pending);
@@ -240,15 +247,9 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wide_gather_kernel(const 
     const int64_t unit = head >> W::kUnitShift;
     const int64_t first = head - i;  // slot of lane 0, had the run begun there
     auto member = [&](int64_t slot, int at) { return (slot >> W::kUnitShift) == unit && slot - at == first; };
-    uint64_t lo = ballot(valid && member(s, lane));
-    uint64_t hi = 0;
-    bool earlier = false;
-    if constexpr (FEW) {
-      lo &= in_tile;
-    } else {
-      hi = ballot(member(s_hi, lane + kWave));
-      earlier = ballot(member(s_pre, lane - kWave)) != 0;  // the run began in the tile before
-    }
+    const uint64_t lo = ballot(valid && member(s, lane));
+    const uint64_t hi = ballot(member(s_hi, lane + kWave));
+    const bool earlier = !pre_short && ballot(member(s_pre, lane - kWave)) != 0;  // the tile before moves the run
     pending &= ~lo;
     if (earlier) continue;
     const int c0 = static_cast<int>(head & (W::UC - 1));
@@ -268,13 +269,6 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wide_gather_kernel(const 
       buf_st16(lbuf, mine ? static_cast<uint32_t>(i) * w.stride + static_cast<uint32_t>(w.cg) * 16u : kOffOob, zero);
     }
   }
-}
-
-// Length of the run starting at lane i: the continuation bits after it, going
-// on into the second window register.
-__device__ __forceinline__ int run_length(uint64_t c_lo, uint64_t c_hi, int i) {
-  const int n = i < 63 ? __builtin_ctzll(~(c_lo >> (i + 1))) : 0;  // the shift fills with zeros
-  return i + 1 + n < 64 ? 1 + n : 1 + n + __builtin_ctzll(~c_hi);  // a unit ends before c_hi runs out
 }
 
 // A run of consecutive tokens loaded for a scatter: unit columns [c0, c0 + n).
@@ -321,9 +315,12 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wide_scatter_kernel(const
   // The token before lane 0 of each register: t0 - 1, and lane 63 of the first.
   const uint64_t pv_lo = (v_lo << 1) | (writes(s_before, t0 - 1) ? 1ull : 0ull);
   const uint64_t pv_hi = (v_hi << 1) | (v_lo >> 63);
-  const int64_t prev = lane == 0 ? s_before : from_prev_lane(s);
+  // The lane shuffles run in every lane: a lane switched off by a condition
+  // would hand its neighbour nothing.
+  const int64_t s_prev = from_prev_lane(s), s_hi_prev = from_prev_lane(s_hi);
   const int64_t last = readlane64(s, 63);
-  const int64_t prev_hi = lane == 0 ? last : from_prev_lane(s_hi);
+  const int64_t prev = lane == 0 ? s_before : s_prev;
+  const int64_t prev_hi = lane == 0 ? last : s_hi_prev;
   auto continues = [&](int64_t slot, int64_t before) { return slot == before + 1 && (slot & (W::UC - 1)) != 0; };
   const uint64_t c_lo = ballot(valid && ((pv_lo >> lane) & 1ull) && continues(s, prev));
   const uint64_t c_hi = ballot(valid_hi && ((pv_hi >> lane) & 1ull) && continues(s_hi, prev_hi));
@@ -399,8 +396,8 @@ hipError_t launch_wide(const TileArgs& a0, int64_t planes, bool lines, hipStream
   TileArgs a = a0;
   const int64_t chunks = (a.nrows + W::UC - 1) / W::UC;
   const int64_t groups = (chunks + kWavesPerBlock - 1) / kWavesPerBlock;
-  const bool few = a.num_tokens <= kWideFewTokens;
-  const int tt = few ? kWideFewTile : W::UC;
+  const bool few = SCATTER && wide_scatter_few(a.num_tokens, planes);
+  const int tt = few ? kWideFewScatterTile : W::UC;
   // Destination order under the narrow scatter's rule: the claim tags are this
   // call's inverse map and the tokens cover a quarter of the slots.
   const bool by_unit = SCATTER && a.owner != nullptr && a.owner_exclusive && a.num_tokens * 4 >= a.num_slots &&
@@ -417,20 +414,18 @@ hipError_t launch_wide(const TileArgs& a0, int64_t planes, bool lines, hipStream
     else if (by_unit)
       hipLaunchKernelGGL((paged_wide_unit_scatter_kernel<ELT, false, kBufWT>), grid, block, 0, stream, a);
     else if (few)
-      hipLaunchKernelGGL((paged_wide_scatter_kernel<ELT, kWideFewTile>), grid, block, 0, stream, a);
+      hipLaunchKernelGGL((paged_wide_scatter_kernel<ELT, kWideFewScatterTile>), grid, block, 0, stream, a);
     else
       hipLaunchKernelGGL((paged_wide_scatter_kernel<ELT, W::UC>), grid, block, 0, stream, a);
   } else {
-    if (few)
-      hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, kWideFewTile, true, false, kBufNT>), grid, block, 0, stream, a);
-    else if (xcd && lines)
-      hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, W::UC, false, true, kBufWT>), grid, block, 0, stream, a);
+    if (xcd && lines)
+      hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, true, kBufWT>), grid, block, 0, stream, a);
     else if (xcd)
-      hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, W::UC, false, true, kBufNT>), grid, block, 0, stream, a);
+      hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, true, kBufNT>), grid, block, 0, stream, a);
     else if (lines)
-      hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, W::UC, false, false, kBufWT>), grid, block, 0, stream, a);
+      hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, false, kBufWT>), grid, block, 0, stream, a);
     else
-      hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, W::UC, false, false, kBufNT>), grid, block, 0, stream, a);
+      hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, false, kBufNT>), grid, block, 0, stream, a);
   }
   return hipGetLastError();
 }

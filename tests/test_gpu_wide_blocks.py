@@ -50,6 +50,7 @@ def _round_trip(dtype, layers, nh, hd, bs, slots, nb):
     (2, 700, "sequences"),
     (2, 900, "skips"),
     (1, 1500, "duplicates"),
+    (3, 1500, "decode"),
 ])
 def test_wide_blocks_match_oracle(dtype, bs, nh, hd, layers, tokens, kind):
     slots, nb = make_slots(kind, np.random.default_rng(tokens + bs), block_size=bs, tokens=tokens)
@@ -86,3 +87,46 @@ def test_wide_blocks_through_block_tables(bs):
         want = bits(cache).copy()
         ko.linear_to_paged(bits(dense).reshape(-1, nh, hd), want, slots)
         assert np.array_equal(bits(cache_d), want)
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "e5m2"])
+@pytest.mark.parametrize("lin", ["bfloat16", "float32"])
+@pytest.mark.parametrize("bs", [64, 128])
+@pytest.mark.parametrize("nh, hd", [(8, 128), (5, 72)])
+@pytest.mark.parametrize("tokens,kind", [
+    (1, "sequences"),
+    (61, "decode"),
+    (256, "decode"),
+    (200, "duplicates"),
+    (700, "decode"),
+    (900, "skips"),
+    (0, "tricky"),              # destination order
+])
+def test_wide_fp8_blocks_match_oracle(fmt, lin, bs, nh, hd, tokens, kind):
+    rng = np.random.default_rng(tokens + bs)
+    if kind == "tricky":
+        nb = 12
+        slots = tricky_slots(rng, nb, bs)
+        assert len(slots) * 4 >= nb * bs
+    else:
+        slots, nb = make_slots(kind, rng, block_size=bs, tokens=tokens, spare_blocks=40)
+    gen = torch.Generator().manual_seed(tokens)
+    dtype = getattr(torch, lin)
+    # Every eighth row far outside the fast quotient's range, so that tiles of both encoders appear.
+    x = [(torch.randn((len(slots), nh, hd), generator=gen) * 3).to(dtype) for _ in range(2)]
+    for t in x:
+        t[3::8] *= 2.0 ** 70
+    scales = [torch.rand(nh, generator=gen) * 0.02 + 0.001, torch.tensor(0.0071)]
+    caches = [torch.randint(0, 256, (nb, nh, hd, bs), dtype=torch.uint8, generator=gen) for _ in range(2)]
+    s_d = torch.from_numpy(slots).to(DEV)
+    got = musa_aiter.kv_paged_fp8_to_linear(*(c.to(DEV) for c in caches), s_d, *(s.to(DEV) for s in scales),
+                                            out_dtype=dtype, fp8_format=fmt)
+    for out, cache, scale in zip(got, caches, scales):
+        assert np.array_equal(bits(out), ko.paged_fp8_to_linear(cache.numpy(), slots, scale.numpy(), fmt, lin))
+    caches_d = [c.to(DEV) for c in caches]
+    musa_aiter.kv_linear_to_paged_fp8(*(t.to(DEV) for t in x), *caches_d, s_d, *(s.to(DEV) for s in scales),
+                                      fp8_format=fmt)
+    for t, cache, cache_d, scale in zip(x, caches, caches_d, scales):
+        want = cache.numpy().copy()
+        ko.linear_to_paged_fp8(t.to(torch.float32).numpy(), want, slots, scale.numpy(), fmt)
+        assert np.array_equal(cache_d.cpu().numpy(), want)
