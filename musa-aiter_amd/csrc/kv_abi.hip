@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "kv_hip_common.h"
+#include "kv_host_calls.h"
 #include "kv_launch.h"
 #include "musa_aiter_kv_hip.h"
 
@@ -369,6 +370,111 @@ int paged_tiles(int scatter, int codec, int cache_elt, int lin_elt, int lin_dtyp
   return kvhip::launch_paged_tiles(p, stream);
 }
 
+// Waits until each of `words` verdict words carries `stamp`; *refused tells
+// whether any of them refuses the call.  The words arrive as the checking
+// kernel runs, so polling them returns sooner than a stream synchronisation; a
+// kernel that has not run after 0.2 s (the stream busy with earlier work) is
+// waited for by the synchronisation.
+hipError_t await_verdict(const int64_t* report, int64_t words, int64_t stamp, hipStream_t stream, bool* refused) {
+  const auto deadline = std::chrono::steady_clock::now() + std::chrono::milliseconds(200);
+  *refused = false;
+  bool synced = false;
+  for (int64_t w = 0; w < words;) {
+    const int64_t v = __atomic_load_n(&report[w], __ATOMIC_ACQUIRE);
+    if ((v >> 1) == stamp) {
+      *refused = *refused || (v & 1) != 0;
+      ++w;
+    } else if (synced) {
+      return hipErrorUnknown;  // the kernel has ended without its verdict
+    } else if (std::chrono::steady_clock::now() > deadline) {
+      const hipError_t err = hipStreamSynchronize(stream);
+      if (err != hipSuccess) return err;
+      synced = true;
+    } else {
+      __builtin_ia32_pause();
+    }
+  }
+  return hipSuccess;
+}
+
+// Slots checked by one workgroup of the check kernel (more, once the report
+// words run out): four loads per thread.
+constexpr int64_t kCheckPerGroup = 1024;
+
+int paged_tiles_checked(const musa_aiter_hip_paged_tiles_call& c, hipStream_t stream) {
+  if (c.num_tokens <= 0 || c.num_layers <= 0 || c.slot_mapping == nullptr || c.report == nullptr ||
+      c.guard == nullptr || c.report_words < 1 || c.stamp <= 0)
+    return hipErrorInvalidValue;
+  PagedTileParams p{};
+  p.scatter = c.scatter;
+  p.codec = c.codec;
+  p.cache_elt = c.cache_elt;
+  p.lin_elt = c.lin_elt;
+  p.lin_dtype = c.lin_dtype;
+  p.cache[0] = c.key_cache;
+  p.cache[1] = c.value_cache;
+  p.lin[0] = c.key_linear;
+  p.lin[1] = c.value_linear;
+  p.slots = c.slot_mapping;
+  p.num_layers = c.num_layers;
+  p.num_tokens = c.num_tokens;
+  p.num_blocks = c.num_blocks;
+  p.num_heads = c.num_heads;
+  p.head_dim = c.head_dim;
+  p.block_size = c.block_size;
+  p.lin_token_stride = c.lin_token_stride * c.lin_elt;
+  p.lin_layer_stride = c.lin_layer_stride * c.lin_elt;
+  p.scale[0] = c.k_scale;
+  p.scale[1] = c.v_scale;
+  p.scale_mode = c.scale_mode;
+  p.fill_zeros = c.fill_zeros;
+  p.check.stamp = c.stamp;
+  bool refused = false;
+  hipError_t err;
+  if (c.num_tokens <= kvhip::kScanTokens && (!c.scatter || c.dedupe)) {
+    // Small calls check themselves (one launch); a call whose kernel cannot is
+    // refused by the launcher and takes the check kernel.
+    p.scan_dupes = c.scatter;
+    p.check.report = c.report;
+    err = kvhip::launch_paged_tiles(p, stream);
+    if (err == hipSuccess) {
+      err = await_verdict(c.report, 1, c.stamp, stream, &refused);
+      return err != hipSuccess ? err : refused ? MUSA_AITER_HIP_REFUSED : 0;
+    }
+    if (err != hipErrorNotSupported) return err;
+    p.scan_dupes = 0;
+    p.check.report = nullptr;
+  }
+  kvhip::CheckSource src{};
+  src.idx = c.slot_mapping;
+  src.n = c.num_tokens;
+  src.rows = c.num_blocks * c.block_size;
+  if (c.codec != kvhip::kCopy) {
+    src.scale[0] = c.k_scale;
+    src.scale[1] = c.v_scale != nullptr ? c.v_scale : c.k_scale;
+    src.num_scales = c.k_scale == nullptr ? 0 : c.scale_mode == 0 ? 1
+                     : c.scale_mode == 1 ? c.num_heads : c.num_layers * c.num_heads;
+  }
+  if (c.scatter && c.dedupe && c.num_tokens > 1) {
+    // The claim pass rides along: the caller's tags under an epoch of this call.
+    if (c.claims == nullptr || c.claims->tags == nullptr || c.claims->capacity < src.rows || c.claims->epoch == 0)
+      return hipErrorInvalidValue;
+    p.owner = src.owner = c.claims->tags;
+    p.epoch = src.epoch = c.claims->epoch;
+    p.owner_exclusive = 1;
+  }
+  int64_t groups = (c.num_tokens + kCheckPerGroup - 1) / kCheckPerGroup;
+  if (groups > c.report_words) groups = c.report_words;
+  kvhip::CallCheck check{c.report, c.guard, c.stamp};
+  err = kvhip::launch_check(src, check, groups, stream);
+  if (err != hipSuccess) return err;
+  p.check.guard = c.guard;
+  const hipError_t moved = kvhip::launch_paged_tiles(p, stream);
+  err = await_verdict(c.report, groups, c.stamp, stream, &refused);
+  if (err != hipSuccess || refused) return err != hipSuccess ? err : MUSA_AITER_HIP_REFUSED;
+  return moved;
+}
+
 // Paged-A caches <-> dense [batch, dense_len, NH, HD] tensors whose tokens are
 // addressed through block tables (the Flash-style preload); the dense side is
 // token-major with `tok_stride_elems` elements between tokens.
@@ -681,6 +787,10 @@ int musa_aiter_hip_paged_tiles(int scatter, int codec, int cache_elt, int lin_el
                      slot_mapping, num_layers, num_tokens, num_blocks, num_heads, head_dim, block_size,
                      lin_token_stride, lin_layer_stride, k_scale, v_scale, scale_mode, fill_zeros, dedupe,
                      as_stream(stream), nullptr, nullptr, claims);
+}
+
+int musa_aiter_hip_paged_tiles_checked(const musa_aiter_hip_paged_tiles_call* call, void* stream) {
+  return call == nullptr ? static_cast<int>(hipErrorInvalidValue) : paged_tiles_checked(*call, as_stream(stream));
 }
 
 int musa_aiter_hip_paged_tiles_noalloc(int scatter, int codec, int cache_elt, int lin_elt, int lin_dtype,

@@ -193,6 +193,26 @@ __device__ __forceinline__ uint64_t claim_tag(uint32_t epoch, int64_t token) {
 }
 
 // ---------------------------------------------------------------------------
+// Argument values checked on the device.  A call that must refuse, before it
+// moves anything, a slot past the cache or an FP8 scale that is not positive
+// and finite does not wait for the host to read the values first: either its
+// own kernel checks them (report set: every workgroup reads them all and
+// workgroup 0 reports), or a check kernel ahead of it on the stream does, and
+// the kernel behind it returns at once if the guard holds its stamp.  The host
+// reads the verdict while the kernel runs.
+// ---------------------------------------------------------------------------
+struct CallCheck {
+  int64_t* report;       // pinned host memory: verdict word(s), 2 * stamp + refused
+  const int64_t* guard;  // device word: `stamp` when the call with that stamp is refused
+  int64_t stamp;         // unique among the calls sharing the guard
+};
+
+// True when a check kernel ahead of this one refused the call.
+__device__ __forceinline__ bool refused_ahead(const CallCheck& c) { return c.guard != nullptr && *c.guard == c.stamp; }
+
+__device__ __forceinline__ bool scale_refused(float s) { return !(s > 0.0f && s < __builtin_inff()); }
+
+// ---------------------------------------------------------------------------
 // Block-table addressing of a dense [batch, dense_len] token range (the
 // Flash-style preload, reference csrc/kvcache/kv_transfer_float.mu:985-1037):
 // token t = b * dense_len + pos lives in slot

@@ -49,9 +49,26 @@ struct PagedTileParams {
   // each slot's last token themselves (ScanTable).  launch_paged_tiles returns
   // hipErrorNotSupported, launching nothing, when the call's kernel cannot.
   int scan_dupes;
+  CallCheck check;           // argument values checked on the device
 };
 
 hipError_t launch_paged_tiles(const PagedTileParams& p, hipStream_t stream);
+
+// One launch ahead of a checked call's kernel (kv_rows.hip): `groups`
+// workgroups check that every idx entry lies below `rows` and every scale is
+// positive and finite, claim the tokens' destinations as launch_claim does
+// (owner set), write their verdicts to check.report[0, groups) and, where
+// something is refused, the call's stamp to check.guard.
+struct CheckSource {
+  const int64_t* idx;
+  int64_t n;
+  int64_t rows;
+  const float* scale[2];
+  int64_t num_scales;      // entries of each scale array (0: none)
+  uint64_t* owner;
+  uint32_t epoch;
+};
+hipError_t launch_check(const CheckSource& src, const CallCheck& check, int64_t groups, hipStream_t stream);
 
 // Row copies between two row-addressed planes: token-major caches
 // ([NB, BS, ...] slot rows), linear buffers and opaque byte rows.  Either side

@@ -31,6 +31,7 @@ struct TileArgs {
   BlockTableSlots bt;          // block_tables set: slots derived per dense token
   int32_t row_groups;          // tile kernel: row groups per block (grid x of a gather = tile * row_groups + group)
   int32_t scan_dupes;          // scatter: resolve repeated slots with a ScanTable instead of claim tags
+  CallCheck check;             // report set: this kernel checks the call's slots and scales; guard set: one ahead did
 };
 
 // Slot of token t: the slot vector's entry, or the block-table slot of the
@@ -86,7 +87,47 @@ constexpr unsigned long long kScanEmpty = ~0ull;
 struct ScanTable {
   unsigned long long key[kScanEntries];
   int last[kScanEntries];
+  int refused;  // some slot or scale of a checked call is not acceptable
 };
+
+// Entries of each scale array of the call.
+__device__ __forceinline__ int64_t scale_count(const TileArgs& a) {
+  if (a.scale[0] == nullptr) return 0;
+  const int64_t layers = static_cast<int64_t>(gridDim.y) / 2;  // every paged kernel runs (.., plane, ..) grids
+  return a.scale_mode == 0 ? 1 : a.scale_mode == 1 ? a.num_heads : layers * a.num_heads;
+}
+
+// This thread's share of the scales of a call checked by its own kernel.
+template <int NT>
+__device__ __forceinline__ bool scales_refused(const TileArgs& a) {
+  bool bad = false;
+  const int64_t n = scale_count(a);
+  for (int64_t j = threadIdx.x; j < 2 * n; j += NT) bad |= scale_refused(a.scale[j >= n][j >= n ? j - n : j]);
+  return bad;
+}
+
+// Workgroup 0's verdict on a checked call, for the polling host.
+__device__ __forceinline__ void report_check(const CallCheck& c, bool refused) {
+  if ((blockIdx.x | blockIdx.y | blockIdx.z | threadIdx.x) == 0)
+    __hip_atomic_store(c.report, 2 * c.stamp + (refused ? 1 : 0), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Checks a small call in the kernel that moves it (report set): every
+// workgroup reads all slots and scales, so all of them decide alike.  Every
+// thread of the workgroup calls it (it holds two barriers).  True: move nothing.
+template <int NT>
+__device__ bool check_in_kernel(const TileArgs& a) {
+  __shared__ int refused;
+  if (threadIdx.x == 0) refused = 0;
+  __syncthreads();
+  bool bad = scales_refused<NT>(a);
+  for (int64_t j = threadIdx.x; j < a.num_tokens; j += NT) bad |= a.slots[j] >= a.num_slots;
+  if (bad) refused = 1;
+  __syncthreads();
+  const bool r = refused != 0;
+  report_check(a.check, r);
+  return r;
+}
 
 // The workgroup's table (static LDS of the kernels that call it).
 __device__ __forceinline__ ScanTable& scan_table() {
@@ -99,17 +140,22 @@ __device__ __forceinline__ uint32_t scan_hash(int64_t s) {
 }
 
 // Fills the table from the call's slots; every thread of the workgroup calls
-// it (it holds two workgroup barriers).
+// it (it holds two workgroup barriers).  A call checked by its own kernel is
+// checked on the way; false: it is refused, move nothing.
 template <int NT>
-__device__ void scan_build(ScanTable& tb, const TileArgs& a) {
+__device__ bool scan_build(ScanTable& tb, const TileArgs& a) {
   const int tid = static_cast<int>(threadIdx.x);
+  const bool checked = a.check.report != nullptr;
+  if (tid == 0) tb.refused = 0;
   for (int e = tid; e < kScanEntries; e += NT) {
     tb.key[e] = kScanEmpty;
     tb.last[e] = -1;
   }
   __syncthreads();
+  bool bad = checked && scales_refused<NT>(a);
   for (int64_t j = tid; j < a.num_tokens; j += NT) {
     const int64_t s = slot_at(a, j);
+    bad |= s >= a.num_slots;
     if (s < 0 || s >= a.num_slots) continue;
     uint32_t h = scan_hash(s);
     for (int probe = 0; probe < kScanEntries; ++probe) {
@@ -121,7 +167,12 @@ __device__ void scan_build(ScanTable& tb, const TileArgs& a) {
       h = (h + 1) & (kScanEntries - 1);
     }
   }
+  if (checked && bad) tb.refused = 1;
   __syncthreads();
+  if (!checked) return true;
+  const bool refused = tb.refused != 0;
+  report_check(a.check, refused);
+  return !refused;
 }
 
 // True when token t is the last token of the call writing slot s (s valid).

@@ -288,11 +288,15 @@ void paged_tile_kernel(const TileArgs a) {
   const int64_t t = t0 - 1 + lane;
   int64_t s = -1;
   if (t >= 0 && t < a.num_tokens) s = slot_at(a, t);
+  if (refused_ahead(a.check)) return;
+  if constexpr (!SCATTER && TOKG) {
+    if (a.check.report != nullptr && check_in_kernel<NT>(a)) return;
+  }
   bool valid = (s >= 0) && (s < a.num_slots);
   if constexpr (SCATTER) {
     if (a.scan_dupes) {
       ScanTable& scan = scan_table();
-      scan_build<NT>(scan, a);
+      if (!scan_build<NT>(scan, a)) return;
       if (valid) valid = scan_is_last(scan, s, t);
     } else if (valid && a.owner != nullptr) {
       valid = (a.owner[s] == claim_tag(a.epoch, t));
@@ -502,6 +506,7 @@ __global__ __launch_bounds__(NT) void paged_block_scatter_kernel(const TileArgs 
   // Lane p < BS holds the tag of slot blk * BS + p.
   uint64_t tag = 0;
   if (lane < BS) tag = a.owner[blk * BS + lane];
+  if (refused_ahead(a.check)) return;
   const bool valid = lane < BS && static_cast<uint32_t>(tag >> 32) == a.epoch && static_cast<uint32_t>(tag) != 0u;
   const int64_t tok = static_cast<int64_t>(static_cast<uint32_t>(tag)) - 1;
   const uint64_t vmask = ballot(valid);
@@ -537,6 +542,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_elem_kernel(const TileArg
   uint8_t* const lin = a.lin[kv] + static_cast<int64_t>(layer) * a.lin_layer_stride;
   const int64_t total = a.num_tokens * a.nrows;
   const int64_t bs = a.block_size;
+  if (refused_ahead(a.check)) return;
   for (int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; e < total;
        e += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const int64_t t = e / a.nrows;
@@ -634,6 +640,10 @@ bool linear_rows_whole_lines(const TileArgs& a, int elt) {
 
 template <int ELT, int BS, bool SCATTER>
 hipError_t launch_tile(const TileArgs& a0, int64_t planes, hipStream_t stream) {
+  // Checked by its own kernel: scatters with a duplicate table and the small
+  // gathers' instantiations.
+  if (a0.check.report != nullptr && (SCATTER ? a0.scan_dupes == 0 : a0.num_tokens > kTokenGatherTokens))
+    return hipErrorNotSupported;
   if constexpr (SCATTER) {
     // Destination order when the claim tags form this call's inverse map and
     // the tokens cover a good share of the cache's slots (each block of the
@@ -711,6 +721,7 @@ hipError_t launch_tile(const TileArgs& a0, int64_t planes, hipStream_t stream) {
   const bool few = SCATTER ? workgroups <= kFewGroups
                            : !(planes >= kXcdOrderPlanes && workgroups > kFewGroups &&
                                workgroups <= int64_t{0xFFFFFFFF});
+  if (!SCATTER && a0.check.report != nullptr && !few) return hipErrorNotSupported;
   if (few && !SCATTER && a0.num_tokens <= kTokenGatherTokens)
     hipLaunchKernelGGL((paged_tile_kernel<ELT, BS, SCATTER, true, kCoopThreads, kBufNT, !SCATTER>), grid,
                        dim3(kCoopThreads), 0, stream, a);
@@ -755,7 +766,7 @@ hipError_t dispatch_bs(const TileArgs& a, int64_t bs, bool fast, int64_t planes,
   }
   // The element kernel checks claim tags only: a call without them takes the
   // claim pass first.
-  if (SCATTER && a.scan_dupes) return hipErrorNotSupported;
+  if ((SCATTER && a.scan_dupes) || a.check.report != nullptr) return hipErrorNotSupported;
   return launch_elem<ELT_C, ELT_L, CODEC, LDT, SCATTER>(a, planes, stream);
 }
 
@@ -811,6 +822,7 @@ hipError_t launch_paged_tiles(const PagedTileParams& p, hipStream_t stream) {
   a.owner_exclusive = p.owner_exclusive;
   a.scan_dupes = p.scan_dupes;
   if (a.scan_dupes && (!p.scatter || p.num_tokens > kScanTokens)) return hipErrorInvalidValue;
+  a.check = p.check;
   a.block_size = static_cast<int32_t>(p.block_size);
   a.inv_head_dim = 1.0f / static_cast<float>(p.head_dim);
   a.bt = p.bt;

@@ -249,6 +249,10 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_gather_kernel(const 
   const int64_t t = t0 - LEAD + lane;
   int64_t s = -1;
   if (t >= 0 && t < a.num_tokens) s = slot_at(a, t);
+  if (refused_ahead(a.check)) return;
+  if constexpr (TOKG && BS < 64) {
+    if (a.check.report != nullptr && check_in_kernel<kBlockThreads>(a)) return;
+  }
   const Window win =
       slot_window<BS>(a, t0, s, [&](int64_t slot, int64_t) { return slot >= 0 && slot < a.num_slots; });
   const uint64_t vmask = win.valid, cmask = win.lo;
@@ -711,10 +715,11 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
     // The slot window; a token whose claim lost to a later duplicate writes
     // nothing.  The duplicate table is built by every wave of the workgroup,
     // before any of them leaves.
-    if (a.scan_dupes) scan_build<kBlockThreads>(scan_table(), a);
+    if (a.scan_dupes && !scan_build<kBlockThreads>(scan_table(), a)) return;
     if (t0 >= a.num_tokens) return;
     const int64_t t = t0 - LEAD + lane;
     if (t >= 0 && t < a.num_tokens) s = slot_at(a, t);
+    if (refused_ahead(a.check)) return;
     const Window win = slot_window<BS>(a, t0, s, [&](int64_t slot, int64_t tk) {
       bool valid = (slot >= 0) && (slot < a.num_slots);
       if (a.scan_dupes) {
@@ -748,6 +753,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_scatter_kernel(const
     if (unit * BS >= a.num_slots) return;
     uint64_t tag = 0;
     if (lane < BS) tag = a.owner[unit * BS + lane];
+    if (refused_ahead(a.check)) return;
     const bool valid = lane < BS && static_cast<uint32_t>(tag >> 32) == a.epoch && static_cast<uint32_t>(tag) != 0u;
     tok = static_cast<int64_t>(static_cast<uint32_t>(tag)) - 1;
     const uint64_t vmask = ballot(valid);
@@ -940,6 +946,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_copy_scatter_kernel(
   // Lane p < BS holds the tag of slot blk * BS + p: runs of consecutive tokens.
   uint64_t tag = 0;
   if (lane < BS) tag = a.owner[blk * BS + lane];
+  if (refused_ahead(a.check)) return;
   const bool valid = lane < BS && static_cast<uint32_t>(tag >> 32) == a.epoch && static_cast<uint32_t>(tag) != 0u;
   const int64_t tok = static_cast<int64_t>(static_cast<uint32_t>(tag)) - 1;
   const uint64_t vmask = ballot(valid);
@@ -1027,6 +1034,7 @@ static_assert(4 * (kGatherLdsPad + kLutHeads * 256 * 2) > 160 * 1024 &&
 template <int ELT_C, int ELT_L, int CODEC, int LDT, int BS>
 hipError_t launch_wave_gather(const TileArgs& a, int64_t planes, hipStream_t stream) {
   using W = WaveShape<ELT_C, ELT_L, BS>;
+  if (a.check.report != nullptr && (BS == 64 || a.num_tokens > kTokenDequantTokens)) return hipErrorNotSupported;
   const int64_t chunks = (a.nrows + W::kChunkRows - 1) / W::kChunkRows;
   if (chunks > 65535) return hipErrorInvalidValue;
   if (CODEC != kCopy && a.scale_mode != 0) {
@@ -1072,6 +1080,7 @@ hipError_t launch_wave_gather(const TileArgs& a, int64_t planes, hipStream_t str
 template <int ELT_C, int ELT_L, int CODEC, int LDT, int BS>
 hipError_t launch_wave_scatter(const TileArgs& a, int64_t planes, hipStream_t stream) {
   using W = ScatterShape<ELT_L, BS>;
+  if (a.check.report != nullptr && !a.scan_dupes) return hipErrorNotSupported;
   const int64_t chunks = (a.nrows + W::kChunkRows * W::kWaveChunks - 1) / (W::kChunkRows * W::kWaveChunks);
   if (chunks > 65535) return hipErrorInvalidValue;
   // Block order when the claim tags are this call's inverse map and the tokens

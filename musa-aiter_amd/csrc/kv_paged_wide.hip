@@ -225,6 +225,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wide_gather_kernel(const 
   const int64_t s = slot_or_none(a, t0 + lane);
   const int64_t s_hi = slot_or_none(a, t0 + kWave + lane);
   const int64_t s_pre = slot_or_none(a, t0 - kWave + lane);
+  if (refused_ahead(a.check)) return;
   const bool valid = s >= 0 && s < a.num_slots;
   const bool valid_pre = s_pre >= 0 && s_pre < a.num_slots;
   const uint64_t in_tile = low_bits(a.num_tokens - t0) & low_bits(TT);
@@ -298,7 +299,8 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wide_scatter_kernel(const
   const int64_t s = slot_or_none(a, t0 + lane);
   const int64_t s_hi = slot_or_none(a, t0 + kWave + lane);
   const int64_t s_before = slot_or_none(a, t0 - 1);
-  if (a.scan_dupes) scan_build<kBlockThreads>(scan_table(), a);  // every wave, before any of them leaves
+  if (a.scan_dupes && !scan_build<kBlockThreads>(scan_table(), a)) return;  // every wave, before any of them leaves
+  if (refused_ahead(a.check)) return;
   if (w.rows == 0) return;
   auto writes = [&](int64_t slot, int64_t t) -> bool {
     bool valid = slot >= 0 && slot < a.num_slots;
@@ -370,6 +372,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wide_unit_scatter_kernel(
   if (w.rows == 0) return;
   uint64_t tag = 0;
   if (lane < W::UC) tag = a.owner[static_cast<int64_t>(unit) * W::UC + lane];
+  if (refused_ahead(a.check)) return;
   const bool valid = static_cast<uint32_t>(tag >> 32) == a.epoch && static_cast<uint32_t>(tag) != 0u;
   const uint64_t cols = ballot(valid);
   if (cols == 0) return;
@@ -393,6 +396,7 @@ constexpr int64_t kWideXcdPlanes = 32;
 template <int ELT, bool SCATTER>
 hipError_t launch_wide(const TileArgs& a0, int64_t planes, bool lines, hipStream_t stream) {
   using W = Wide<ELT>;
+  if (a0.check.report != nullptr && !a0.scan_dupes) return hipErrorNotSupported;
   TileArgs a = a0;
   const int64_t chunks = (a.nrows + W::UC - 1) / W::UC;
   const int64_t groups = (chunks + kWavesPerBlock - 1) / kWavesPerBlock;

@@ -356,6 +356,49 @@ __global__ __launch_bounds__(kBlockThreads) void index_max_kernel(const int64_t*
   }
 }
 
+// The check kernel of a checked call (see CallCheck and launch_check).
+// kCheckTokens entries per workgroup and round, four loads in flight per thread.
+constexpr int kCheckTokens = 4 * kBlockThreads;
+
+struct CheckArgs {
+  CheckSource src;
+  CallCheck check;
+  int64_t* guard;
+};
+
+__global__ __launch_bounds__(kBlockThreads) void check_kernel(const CheckArgs a) {
+  const CheckSource& c = a.src;
+  bool bad = false;
+  for (int64_t base = static_cast<int64_t>(blockIdx.x) * kCheckTokens; base < c.n;
+       base += static_cast<int64_t>(gridDim.x) * kCheckTokens) {
+    int64_t s[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t i = base + k * kBlockThreads + threadIdx.x;
+      s[k] = i < c.n ? c.idx[i] : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      bad |= s[k] >= c.rows;
+      if (c.owner != nullptr && s[k] >= 0 && s[k] < c.rows)
+        atomicMax(reinterpret_cast<unsigned long long*>(c.owner + s[k]),
+                  static_cast<unsigned long long>(claim_tag(c.epoch, base + k * kBlockThreads + threadIdx.x)));
+    }
+  }
+  if (blockIdx.x == 0)
+    for (int64_t j = threadIdx.x; j < c.num_scales; j += kBlockThreads)
+      bad |= scale_refused(c.scale[0][j]) || scale_refused(c.scale[1][j]);
+  __shared__ int refused;
+  if (threadIdx.x == 0) refused = 0;
+  __syncthreads();
+  if (bad) refused = 1;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  if (refused) *a.guard = a.check.stamp;
+  __hip_atomic_store(a.check.report + blockIdx.x, 2 * a.check.stamp + refused, __ATOMIC_RELEASE,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ----- strided block transfer ------------------------------------------------------
 // Staging [NL, staging_tokens, row_bytes] <-> per-layer pages addressed by block
 // id.  Mode 0 pages hold plain rows at block*stride + t*row_bytes; mode 1 pages
@@ -639,6 +682,14 @@ hipError_t launch_index_max(const int64_t* idx, int64_t n, int64_t* partial, int
   if (idx == nullptr || partial == nullptr || n <= 0 || parts < 1 || parts > 4096) return hipErrorInvalidValue;
   hipLaunchKernelGGL(index_max_kernel, dim3(static_cast<uint32_t>(parts)), dim3(kBlockThreads), 0, stream, idx, n,
                      partial, stamp);
+  return hipGetLastError();
+}
+
+hipError_t launch_check(const CheckSource& src, const CallCheck& check, int64_t groups, hipStream_t stream) {
+  if (src.idx == nullptr || src.n <= 0 || groups < 1 || check.report == nullptr || check.guard == nullptr)
+    return hipErrorInvalidValue;
+  const CheckArgs a{src, check, const_cast<int64_t*>(check.guard)};
+  hipLaunchKernelGGL(check_kernel, dim3(static_cast<uint32_t>(groups)), dim3(kBlockThreads), 0, stream, a);
   return hipGetLastError();
 }
 

@@ -90,6 +90,7 @@ _SIGNATURES: dict[str, list] = {
     # (src_k, src_v, dst_k, dst_v, block_mapping, pairs, layers, src_blocks, dst_blocks, heads,
     #  head_dim, block_size, stream); the "_fp8_vec8" entry copies one-byte elements.
     "musa_aiter_kv_copy_paged_blocks_fp8_vec8": [_c_void_p] * 5 + [_i64] * 7 + [_c_void_p],
+    "musa_aiter_hip_paged_tiles_checked": [ctypes.c_char_p, _c_void_p],  # musa_aiter_hip_paged_tiles_call, stream
     "musa_aiter_hip_error_string": [_i32],
     "musa_aiter_hip_backend_name": [],
     "musa_aiter_hip_graph_claim_arrays": [],
@@ -304,6 +305,72 @@ def index_max(idx: torch.Tensor) -> int:
         check(fn("musa_aiter_hip_index_max")(ptr(idx), n, ptr(buf), parts, entry[1], stream_ptr(device)),
               "index_max")
         return int(buf.numpy()[:parts].max())
+
+
+# musa_aiter_hip_paged_tiles_call: eight int32 flags, five tensors, eight int64 sizes and strides, two
+# scale pointers, the claims pointer, report and guard addresses, report words and stamp.
+_PAGED_TILES_CALL = struct.Struct("<8i5Q8q2QQ2Q2q")
+_REFUSED = -1  # MUSA_AITER_HIP_REFUSED
+_REPORT_WORDS = 64
+
+
+class _CheckSet:
+    """Verdict words (pinned host memory), guard word (device memory) and stamp of the checked calls on one
+    (device, stream), which issue one at a time under the lock: a check kernel, where there is one, and the
+    kernel it guards follow each other on the stream."""
+    __slots__ = ("lock", "report", "guard", "report_ptr", "guard_ptr", "stamp")
+
+    def __init__(self, device: torch.device):
+        self.lock = threading.Lock()
+        self.report = torch.zeros(_REPORT_WORDS, dtype=torch.int64, pin_memory=True)
+        self.guard = torch.zeros(1, dtype=torch.int64, device=device)
+        self.report_ptr, self.guard_ptr = self.report.data_ptr(), self.guard.data_ptr()
+        self.stamp = 0
+
+
+_check_sets: dict[tuple[int, int], _CheckSet] = {}
+_check_sets_lock = threading.Lock()
+
+
+def _check_set(device: torch.device, stream: int) -> _CheckSet:
+    key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
+    found = _check_sets.get(key)
+    if found is None:
+        with _check_sets_lock:
+            found = _check_sets.get(key)
+            if found is None:
+                found = _check_sets[key] = _CheckSet(device)
+    return found
+
+
+def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, lin_elt: int, lin_dtype: int,
+                        key_cache: torch.Tensor, value_cache: torch.Tensor, key_linear: torch.Tensor,
+                        value_linear: torch.Tensor, slots: torch.Tensor, num_layers: int, num_tokens: int,
+                        num_blocks: int, num_heads: int, head_dim: int, block_size: int, lin_token_stride: int,
+                        lin_layer_stride: int, k_scale: torch.Tensor | None = None,
+                        v_scale: torch.Tensor | None = None, scale_mode: int = 0, fill_zeros: bool = True) -> bool:
+    """paged_tiles for a call whose slots and scales are still unchecked: the device checks them, and False
+    means that one was refused (a slot past the cache, a scale that is not positive and finite) and
+    nothing was moved.  Needs at least one token and layer; not for a stream being captured."""
+    device = key_cache.device
+    with on_device(device):
+        stream = stream_ptr(device)
+        checks = _check_set(device, stream.value or 0)
+        with checks.lock:
+            claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter else (0, None))
+            checks.stamp += 1
+            call = _PAGED_TILES_CALL.pack(
+                scatter, codec, cache_elt, lin_elt, lin_dtype, scale_mode, fill_zeros, scatter,
+                key_cache.data_ptr(), value_cache.data_ptr(), key_linear.data_ptr(), value_linear.data_ptr(),
+                slots.data_ptr(), num_layers, num_tokens, num_blocks, num_heads, head_dim, block_size,
+                lin_token_stride, lin_layer_stride, _data(k_scale), _data(v_scale), claims, checks.report_ptr,
+                checks.guard_ptr, _REPORT_WORDS, checks.stamp)
+            rc = fn("musa_aiter_hip_paged_tiles_checked")(call, stream)
+            del keep
+    if rc == _REFUSED:
+        return False
+    check(rc, op)
+    return True
 
 
 def allocated_bytes() -> int:

@@ -152,6 +152,45 @@ def _check_slots_in_bounds(slots_long: torch.Tensor, nb: int, bs: int, name: str
         raise ValueError(f"{name}: slot index {max_slot} out of bounds for caches (max {nb * bs - 1})")
 
 
+class _ValueChecks:
+    """The checks of one call that read device values: slot bounds, then FP8 scales, in the reference's order.
+
+    Entered after the checks that come before them.  The launch makes them on the device (``moved``), so no
+    value is read by the host before it; ``run`` makes them one by one, raising the reference's error, and does
+    so where an error of a later check would otherwise overtake theirs."""
+
+    __slots__ = ("op", "slots", "nb", "bs", "scales", "done")
+
+    def __init__(self, op: str, slots: torch.Tensor, nb: int, bs: int):
+        self.op, self.slots, self.nb, self.bs = op, slots, nb, bs
+        self.scales: list[tuple[str, torch.Tensor]] = []
+        self.done = False
+
+    def __enter__(self) -> "_ValueChecks":
+        return self
+
+    def __exit__(self, exc_type, exc, tb) -> None:
+        if exc_type is not None and issubclass(exc_type, Exception) and not issubclass(exc_type, _hip.HipBackendError):
+            self.run()
+
+    def run(self) -> None:
+        if self.done:
+            return
+        self.done = True
+        _check_slots_in_bounds(self.slots, self.nb, self.bs, self.op)
+        for name, scale in self.scales:
+            _check_fp8_scale_values(scale, name)
+
+    def moved(self, caches: "_CachePair", call: dict) -> None:
+        """Makes the checks and the paged_tiles call."""
+        if self.slots.numel() and not caches.copied and not torch.cuda.is_current_stream_capturing():
+            if _hip.paged_tiles_checked(**call):
+                self.done = True
+                return
+        self.run()
+        _hip.paged_tiles(**call)
+
+
 def _float_elt(name: str, *tensors: torch.Tensor) -> int:
     dtype = tensors[0].dtype
     for t in tensors:
@@ -229,7 +268,8 @@ class _CachePair:
         self.user = (k, v)
         self.k = k if k.is_contiguous() else k.contiguous()
         self.v = v if v.is_contiguous() else v.contiguous()
-        self.copy_back = writable and (self.k is not k or self.v is not v)
+        self.copied = self.k is not k or self.v is not v
+        self.copy_back = writable and self.copied
 
     def finish(self) -> None:
         if self.copy_back:
@@ -267,24 +307,24 @@ def _fill_mode(fill_skipped: str, out_k: torch.Tensor | None, out_v: torch.Tenso
     return True
 
 
-def _paged_gather(op: str, key_cache: torch.Tensor, value_cache: torch.Tensor, slots: torch.Tensor, *, nl: int,
+def _paged_gather(checks: _ValueChecks, key_cache: torch.Tensor, value_cache: torch.Tensor, *, nl: int,
                   tcount: int, nb: int, nh: int, hd: int, bs: int, out_k: torch.Tensor, out_v: torch.Tensor,
                   token_dim: int, fill_zeros: bool) -> None:
     caches = _CachePair(key_cache, value_cache, writable=False)
     lin = _LinearPair(out_k, out_v, token_dim=token_dim, row=nh * hd, writable=True)
     elt = _ELT[key_cache.dtype]
-    _hip.paged_tiles(
-        op=op, scatter=False, codec=_CODEC_COPY, cache_elt=elt, lin_elt=elt, lin_dtype=0,
-        key_cache=caches.k, value_cache=caches.v, key_linear=lin.k, value_linear=lin.v, slots=slots,
+    checks.moved(caches, dict(
+        op=checks.op, scatter=False, codec=_CODEC_COPY, cache_elt=elt, lin_elt=elt, lin_dtype=0,
+        key_cache=caches.k, value_cache=caches.v, key_linear=lin.k, value_linear=lin.v, slots=checks.slots,
         num_layers=nl, num_tokens=tcount, num_blocks=nb, num_heads=nh, head_dim=hd, block_size=bs,
         lin_token_stride=lin.tok_stride, lin_layer_stride=lin.layer_stride, fill_zeros=fill_zeros,
-    )
+    ))
     lin.finish()
 
 
-def _paged_scatter(op: str, key_linear: torch.Tensor, value_linear: torch.Tensor, key_cache: torch.Tensor,
-                   value_cache: torch.Tensor, slots: torch.Tensor, *, nl: int, tcount: int, nb: int, nh: int, hd: int,
-                   bs: int, token_dim: int) -> None:
+def _paged_scatter(checks: _ValueChecks, key_linear: torch.Tensor, value_linear: torch.Tensor,
+                   key_cache: torch.Tensor, value_cache: torch.Tensor, *, nl: int, tcount: int, nb: int, nh: int,
+                   hd: int, bs: int, token_dim: int) -> None:
     if key_linear.dtype != key_cache.dtype:
         key_linear = key_linear.to(key_cache.dtype)
     if value_linear.dtype != value_cache.dtype:
@@ -292,12 +332,12 @@ def _paged_scatter(op: str, key_linear: torch.Tensor, value_linear: torch.Tensor
     caches = _CachePair(key_cache, value_cache, writable=True)
     lin = _LinearPair(key_linear, value_linear, token_dim=token_dim, row=nh * hd, writable=False)
     elt = _ELT[key_cache.dtype]
-    _hip.paged_tiles(
-        op=op, scatter=True, codec=_CODEC_COPY, cache_elt=elt, lin_elt=elt, lin_dtype=0,
-        key_cache=caches.k, value_cache=caches.v, key_linear=lin.k, value_linear=lin.v, slots=slots,
+    checks.moved(caches, dict(
+        op=checks.op, scatter=True, codec=_CODEC_COPY, cache_elt=elt, lin_elt=elt, lin_dtype=0,
+        key_cache=caches.k, value_cache=caches.v, key_linear=lin.k, value_linear=lin.v, slots=checks.slots,
         num_layers=nl, num_tokens=tcount, num_blocks=nb, num_heads=nh, head_dim=hd, block_size=bs,
         lin_token_stride=lin.tok_stride, lin_layer_stride=lin.layer_stride, fill_zeros=False,
-    )
+    ))
     caches.finish()
 
 
@@ -321,16 +361,16 @@ def kv_paged_to_linear(
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
     if key_cache.device != value_cache.device or slots.device != key_cache.device:
         raise ValueError("kv_paged_to_linear: all tensors must be on the same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    _float_elt(op, key_cache, value_cache)
-    _check_gather_out(out_k, (tcount, nh, hd), key_cache.dtype, key_cache.device, op)
-    _check_gather_out(out_v, (tcount, nh, hd), value_cache.dtype, value_cache.device, op)
-    fill_zeros = _fill_mode(fill_skipped, out_k, out_v, op)
-    _require_rocm(op, key_cache)
-    ok = out_k if out_k is not None else torch.empty((tcount, nh, hd), dtype=key_cache.dtype, device=key_cache.device)
-    ov = out_v if out_v is not None else torch.empty((tcount, nh, hd), dtype=value_cache.dtype, device=value_cache.device)
-    _paged_gather(op, key_cache, value_cache, slots, nl=1, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, out_k=ok,
-                  out_v=ov, token_dim=0, fill_zeros=fill_zeros)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        _float_elt(op, key_cache, value_cache)
+        _check_gather_out(out_k, (tcount, nh, hd), key_cache.dtype, key_cache.device, op)
+        _check_gather_out(out_v, (tcount, nh, hd), value_cache.dtype, value_cache.device, op)
+        fill_zeros = _fill_mode(fill_skipped, out_k, out_v, op)
+        _require_rocm(op, key_cache)
+        ok = out_k if out_k is not None else torch.empty((tcount, nh, hd), dtype=key_cache.dtype, device=key_cache.device)
+        ov = out_v if out_v is not None else torch.empty((tcount, nh, hd), dtype=value_cache.dtype, device=value_cache.device)
+        _paged_gather(checks, key_cache, value_cache, nl=1, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, out_k=ok,
+                      out_v=ov, token_dim=0, fill_zeros=fill_zeros)
     _emit(op, key_cache, "gfx950 paged->linear tile gather")
     return ok, ov
 
@@ -351,25 +391,25 @@ def kv_paged_to_linear_multi_layer(
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
     if value_cache.device != key_cache.device or slots.device != key_cache.device:
         raise ValueError("kv_paged_to_linear_multi_layer: all tensors must be on the same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    if out_k is not None and tuple(out_k.shape) != (nl, tcount, nh, hd):
-        raise ValueError(
-            f"kv_paged_to_linear_multi_layer: out_k must be [num_layers, T, kv_heads, head_dim], got {tuple(out_k.shape)}")
-    if out_v is not None and tuple(out_v.shape) != (nl, tcount, nh, hd):
-        raise ValueError(
-            f"kv_paged_to_linear_multi_layer: out_v must be [num_layers, T, kv_heads, head_dim], got {tuple(out_v.shape)}")
-    if fill_skipped == "preserve" and (out_k is None or out_v is None):
-        raise ValueError("kv_paged_to_linear_multi_layer: fill_skipped=preserve requires out_k and out_v")
-    _float_elt(op, key_cache, value_cache)
-    _check_gather_out(out_k, (nl, tcount, nh, hd), key_cache.dtype, key_cache.device, op)
-    _check_gather_out(out_v, (nl, tcount, nh, hd), value_cache.dtype, value_cache.device, op)
-    fill_zeros = _fill_mode(fill_skipped, out_k, out_v, op)
-    _require_rocm(op, key_cache)
-    shape = (nl, tcount, nh, hd)
-    ok = out_k if out_k is not None else torch.empty(shape, dtype=key_cache.dtype, device=key_cache.device)
-    ov = out_v if out_v is not None else torch.empty(shape, dtype=value_cache.dtype, device=value_cache.device)
-    _paged_gather(op, key_cache, value_cache, slots, nl=nl, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, out_k=ok,
-                  out_v=ov, token_dim=1, fill_zeros=fill_zeros)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        if out_k is not None and tuple(out_k.shape) != (nl, tcount, nh, hd):
+            raise ValueError(
+                f"kv_paged_to_linear_multi_layer: out_k must be [num_layers, T, kv_heads, head_dim], got {tuple(out_k.shape)}")
+        if out_v is not None and tuple(out_v.shape) != (nl, tcount, nh, hd):
+            raise ValueError(
+                f"kv_paged_to_linear_multi_layer: out_v must be [num_layers, T, kv_heads, head_dim], got {tuple(out_v.shape)}")
+        if fill_skipped == "preserve" and (out_k is None or out_v is None):
+            raise ValueError("kv_paged_to_linear_multi_layer: fill_skipped=preserve requires out_k and out_v")
+        _float_elt(op, key_cache, value_cache)
+        _check_gather_out(out_k, (nl, tcount, nh, hd), key_cache.dtype, key_cache.device, op)
+        _check_gather_out(out_v, (nl, tcount, nh, hd), value_cache.dtype, value_cache.device, op)
+        fill_zeros = _fill_mode(fill_skipped, out_k, out_v, op)
+        _require_rocm(op, key_cache)
+        shape = (nl, tcount, nh, hd)
+        ok = out_k if out_k is not None else torch.empty(shape, dtype=key_cache.dtype, device=key_cache.device)
+        ov = out_v if out_v is not None else torch.empty(shape, dtype=value_cache.dtype, device=value_cache.device)
+        _paged_gather(checks, key_cache, value_cache, nl=nl, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, out_k=ok,
+                      out_v=ov, token_dim=1, fill_zeros=fill_zeros)
     _emit(op, key_cache, f"gfx950 paged->linear tile gather ({nl} layers, one launch)")
     return ok, ov
 
@@ -400,11 +440,11 @@ def kv_linear_to_paged(
     dev = key_cache.device
     if any(x.device != dev for x in (key_linear, value_linear, key_cache, value_cache, slots)):
         raise ValueError("kv_linear_to_paged: all tensors must be on same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    _float_elt(op, key_cache, value_cache)
-    _require_rocm(op, key_cache)
-    _paged_scatter(op, key_linear, value_linear, key_cache, value_cache, slots, nl=1, tcount=int(tcount), nb=nb,
-                   nh=nh, hd=hd, bs=bs, token_dim=0)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        _float_elt(op, key_cache, value_cache)
+        _require_rocm(op, key_cache)
+        _paged_scatter(checks, key_linear, value_linear, key_cache, value_cache, nl=1, tcount=int(tcount), nb=nb,
+                       nh=nh, hd=hd, bs=bs, token_dim=0)
     _emit(op, key_linear, "gfx950 linear->paged tile scatter")
 
 
@@ -436,11 +476,11 @@ def kv_linear_to_paged_multi_layer(
     dev = key_cache.device
     if any(x.device != dev for x in (key_linear, value_linear, key_cache, value_cache, slots)):
         raise ValueError("kv_linear_to_paged_multi_layer: all tensors must be on same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    _float_elt(op, key_cache, value_cache)
-    _require_rocm(op, key_cache)
-    _paged_scatter(op, key_linear, value_linear, key_cache, value_cache, slots, nl=nl, tcount=tcount, nb=nb, nh=nh,
-                   hd=hd, bs=bs, token_dim=1)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        _float_elt(op, key_cache, value_cache)
+        _require_rocm(op, key_cache)
+        _paged_scatter(checks, key_linear, value_linear, key_cache, value_cache, nl=nl, tcount=tcount, nb=nb, nh=nh,
+                       hd=hd, bs=bs, token_dim=1)
     _emit(op, key_linear, f"gfx950 linear->paged tile scatter ({nl} layers, one launch)")
 
 
@@ -471,13 +511,13 @@ def kv_paged_to_merged_linear(
             raise ValueError("kv_paged_to_merged_linear: out dtype/device must match caches")
     if fill_skipped == "preserve" and out is None:
         raise ValueError("kv_paged_to_merged_linear: fill_skipped=preserve requires out")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    _float_elt(op, key_cache, value_cache)
-    fill_zeros = fill_skipped != "preserve"
-    _require_rocm(op, key_cache)
-    res = out if out is not None else torch.empty((tcount, 2, nh, hd), dtype=key_cache.dtype, device=key_cache.device)
-    _paged_gather(op, key_cache, value_cache, slots, nl=1, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs,
-                  out_k=res[:, 0], out_v=res[:, 1], token_dim=0, fill_zeros=fill_zeros)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        _float_elt(op, key_cache, value_cache)
+        fill_zeros = fill_skipped != "preserve"
+        _require_rocm(op, key_cache)
+        res = out if out is not None else torch.empty((tcount, 2, nh, hd), dtype=key_cache.dtype, device=key_cache.device)
+        _paged_gather(checks, key_cache, value_cache, nl=1, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs,
+                      out_k=res[:, 0], out_v=res[:, 1], token_dim=0, fill_zeros=fill_zeros)
     _emit(op, key_cache, "gfx950 paged->merged-linear tile gather")
     return res
 
@@ -499,11 +539,11 @@ def kv_merged_linear_to_paged(
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
     if any(x.device != key_cache.device for x in (merged_linear, key_cache, value_cache, slots)):
         raise ValueError("kv_merged_linear_to_paged: all tensors must be on same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    _float_elt(op, key_cache, value_cache)
-    _require_rocm(op, key_cache)
-    _paged_scatter(op, merged_linear[:, 0], merged_linear[:, 1], key_cache, value_cache, slots, nl=1, tcount=tcount,
-                   nb=nb, nh=nh, hd=hd, bs=bs, token_dim=0)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        _float_elt(op, key_cache, value_cache)
+        _require_rocm(op, key_cache)
+        _paged_scatter(checks, merged_linear[:, 0], merged_linear[:, 1], key_cache, value_cache, nl=1, tcount=tcount,
+                       nb=nb, nh=nh, hd=hd, bs=bs, token_dim=0)
     _emit(op, merged_linear, "gfx950 merged-linear->paged tile scatter")
 
 
@@ -529,14 +569,14 @@ def kv_paged_to_merged_linear_multi_layer(
             raise ValueError("kv_paged_to_merged_linear_multi_layer: out dtype/device must match caches")
     if fill_skipped == "preserve" and out is None:
         raise ValueError("kv_paged_to_merged_linear_multi_layer: fill_skipped=preserve requires out")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    _float_elt(op, key_cache, value_cache)
-    fill_zeros = fill_skipped != "preserve"
-    _require_rocm(op, key_cache)
-    res = out if out is not None else torch.empty((nl, tcount, 2, nh, hd), dtype=key_cache.dtype,
-                                                  device=key_cache.device)
-    _paged_gather(op, key_cache, value_cache, slots, nl=nl, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs,
-                  out_k=res[:, :, 0], out_v=res[:, :, 1], token_dim=1, fill_zeros=fill_zeros)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        _float_elt(op, key_cache, value_cache)
+        fill_zeros = fill_skipped != "preserve"
+        _require_rocm(op, key_cache)
+        res = out if out is not None else torch.empty((nl, tcount, 2, nh, hd), dtype=key_cache.dtype,
+                                                      device=key_cache.device)
+        _paged_gather(checks, key_cache, value_cache, nl=nl, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs,
+                      out_k=res[:, :, 0], out_v=res[:, :, 1], token_dim=1, fill_zeros=fill_zeros)
     _emit(op, key_cache, f"gfx950 paged->merged-linear tile gather ({nl} layers, one launch)")
     return res
 
@@ -560,11 +600,11 @@ def kv_merged_linear_to_paged_multi_layer(
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
     if any(x.device != key_cache.device for x in (merged_linear, key_cache, value_cache, slots)):
         raise ValueError("kv_merged_linear_to_paged_multi_layer: all tensors must be on same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    _float_elt(op, key_cache, value_cache)
-    _require_rocm(op, key_cache)
-    _paged_scatter(op, merged_linear[:, :, 0], merged_linear[:, :, 1], key_cache, value_cache, slots, nl=nl,
-                   tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=1)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        _float_elt(op, key_cache, value_cache)
+        _require_rocm(op, key_cache)
+        _paged_scatter(checks, merged_linear[:, :, 0], merged_linear[:, :, 1], key_cache, value_cache, nl=nl,
+                       tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=1)
     _emit(op, merged_linear, f"gfx950 merged-linear->paged tile scatter ({nl} layers, one launch)")
 
 
@@ -593,11 +633,21 @@ def _codec(fp8_format: str) -> int:
     return _CODEC_E4M3 if _normalize_fp8_format(fp8_format) == "e4m3" else _CODEC_E5M2
 
 
-def _ensure_fp8_scale(scale: torch.Tensor | float, *, device: torch.device, name: str, num_heads: int,
-                      num_layers: int | None = None) -> torch.Tensor:
-    scale_tensor = torch.as_tensor(scale, dtype=torch.float32, device=device)
-    if scale_tensor.numel() == 0 or not bool(((scale_tensor > 0) & torch.isfinite(scale_tensor)).all()):
+def _check_fp8_scale_values(scale: torch.Tensor, name: str) -> None:
+    if not bool(((scale > 0) & torch.isfinite(scale)).all()):
         raise ValueError(f"{name}: FP8 scale must be positive and finite")
+
+
+def _ensure_fp8_scale(scale: torch.Tensor | float, *, device: torch.device, name: str, num_heads: int,
+                      num_layers: int | None = None, checks: _ValueChecks | None = None) -> torch.Tensor:
+    """The scale as a float32 device tensor of an accepted shape; its values are checked here, or left to ``checks``."""
+    scale_tensor = torch.as_tensor(scale, dtype=torch.float32, device=device)
+    if scale_tensor.numel() == 0:
+        raise ValueError(f"{name}: FP8 scale must be positive and finite")
+    if checks is None:
+        _check_fp8_scale_values(scale_tensor, name)
+    else:
+        checks.scales.append((name, scale_tensor))
     if scale_tensor.numel() == 1:
         return scale_tensor.reshape(()).contiguous()
     if scale_tensor.dim() == 1 and int(scale_tensor.shape[0]) == num_heads:
@@ -638,8 +688,8 @@ def _fp8_linear_input(x: torch.Tensor) -> torch.Tensor:
     return x if x.dtype in _LIN_DTYPE else x.to(torch.float32)
 
 
-def _fp8_scatter(op: str, key_linear: torch.Tensor, value_linear: torch.Tensor, key_cache: torch.Tensor,
-                 value_cache: torch.Tensor, slots: torch.Tensor, k_scale: torch.Tensor, v_scale: torch.Tensor, *,
+def _fp8_scatter(checks: _ValueChecks, key_linear: torch.Tensor, value_linear: torch.Tensor, key_cache: torch.Tensor,
+                 value_cache: torch.Tensor, k_scale: torch.Tensor, v_scale: torch.Tensor, *,
                  fp8_format: str, nl: int, tcount: int, nb: int, nh: int, hd: int, bs: int, token_dim: int) -> None:
     key_linear = _fp8_linear_input(key_linear)
     value_linear = _fp8_linear_input(value_linear)
@@ -648,17 +698,17 @@ def _fp8_scatter(op: str, key_linear: torch.Tensor, value_linear: torch.Tensor, 
     k_scale, v_scale, mode = _scale_pair(k_scale, v_scale, nh)
     caches = _CachePair(_fp8_bytes(key_cache), _fp8_bytes(value_cache), writable=True)
     lin = _LinearPair(key_linear, value_linear, token_dim=token_dim, row=nh * hd, writable=False)
-    _hip.paged_tiles(
-        op=op, scatter=True, codec=_codec(fp8_format), cache_elt=1, lin_elt=_ELT[key_linear.dtype],
+    checks.moved(caches, dict(
+        op=checks.op, scatter=True, codec=_codec(fp8_format), cache_elt=1, lin_elt=_ELT[key_linear.dtype],
         lin_dtype=_LIN_DTYPE[key_linear.dtype], key_cache=caches.k, value_cache=caches.v, key_linear=lin.k,
-        value_linear=lin.v, slots=slots, num_layers=nl, num_tokens=tcount, num_blocks=nb, num_heads=nh,
+        value_linear=lin.v, slots=checks.slots, num_layers=nl, num_tokens=tcount, num_blocks=nb, num_heads=nh,
         head_dim=hd, block_size=bs, lin_token_stride=lin.tok_stride, lin_layer_stride=lin.layer_stride,
         k_scale=k_scale, v_scale=v_scale, scale_mode=mode, fill_zeros=False,
-    )
+    ))
     caches.finish()
 
 
-def _fp8_gather(op: str, key_cache: torch.Tensor, value_cache: torch.Tensor, slots: torch.Tensor,
+def _fp8_gather(checks: _ValueChecks, key_cache: torch.Tensor, value_cache: torch.Tensor,
                 k_scale: torch.Tensor, v_scale: torch.Tensor, *, fp8_format: str, out_dtype: torch.dtype,
                 out_k: torch.Tensor, out_v: torch.Tensor, nl: int, tcount: int, nb: int, nh: int, hd: int, bs: int,
                 token_dim: int) -> None:
@@ -671,13 +721,13 @@ def _fp8_gather(op: str, key_cache: torch.Tensor, value_cache: torch.Tensor, slo
         tv = torch.empty(out_v.shape, dtype=work_dtype, device=out_v.device)
     caches = _CachePair(_fp8_bytes(key_cache), _fp8_bytes(value_cache), writable=False)
     lin = _LinearPair(tk, tv, token_dim=token_dim, row=nh * hd, writable=True)
-    _hip.paged_tiles(
-        op=op, scatter=False, codec=_codec(fp8_format), cache_elt=1, lin_elt=_ELT[work_dtype],
+    checks.moved(caches, dict(
+        op=checks.op, scatter=False, codec=_codec(fp8_format), cache_elt=1, lin_elt=_ELT[work_dtype],
         lin_dtype=_LIN_DTYPE[work_dtype], key_cache=caches.k, value_cache=caches.v, key_linear=lin.k,
-        value_linear=lin.v, slots=slots, num_layers=nl, num_tokens=tcount, num_blocks=nb, num_heads=nh,
+        value_linear=lin.v, slots=checks.slots, num_layers=nl, num_tokens=tcount, num_blocks=nb, num_heads=nh,
         head_dim=hd, block_size=bs, lin_token_stride=lin.tok_stride, lin_layer_stride=lin.layer_stride,
         k_scale=k_scale, v_scale=v_scale, scale_mode=mode, fill_zeros=True,
-    )
+    ))
     lin.finish()
     if tk is not out_k:
         out_k.copy_(tk)
@@ -717,12 +767,12 @@ def kv_linear_to_paged_fp8(
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
     if slots.device != key_linear.device:
         raise ValueError("kv_linear_to_paged_fp8: slot_mapping must be on the same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    ks = _ensure_fp8_scale(k_scale, device=key_linear.device, name="k_scale", num_heads=nh)
-    vs = _ensure_fp8_scale(v_scale, device=value_linear.device, name="v_scale", num_heads=nh)
-    _require_rocm(op, key_linear)
-    _fp8_scatter(op, key_linear, value_linear, key_cache_fp8, value_cache_fp8, slots, ks, vs, fp8_format=fp8_format,
-                 nl=1, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=0)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        ks = _ensure_fp8_scale(k_scale, device=key_linear.device, name="k_scale", num_heads=nh, checks=checks)
+        vs = _ensure_fp8_scale(v_scale, device=value_linear.device, name="v_scale", num_heads=nh, checks=checks)
+        _require_rocm(op, key_linear)
+        _fp8_scatter(checks, key_linear, value_linear, key_cache_fp8, value_cache_fp8, ks, vs, fp8_format=fp8_format,
+                     nl=1, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=0)
     _emit(op, key_linear, f"gfx950 fused {fp8_format.upper()} quantize scatter")
 
 
@@ -748,18 +798,18 @@ def kv_paged_fp8_to_linear(
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
     if slots.device != key_cache_fp8.device:
         raise ValueError("kv_paged_fp8_to_linear: slot_mapping must be on the same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    ks = _ensure_fp8_scale(k_scale, device=key_cache_fp8.device, name="k_scale", num_heads=nh)
-    vs = _ensure_fp8_scale(v_scale, device=value_cache_fp8.device, name="v_scale", num_heads=nh)
-    ok = out_k if out_k is not None else torch.empty(tcount, nh, hd, dtype=out_dtype, device=key_cache_fp8.device)
-    ov = out_v if out_v is not None else torch.empty(tcount, nh, hd, dtype=out_dtype, device=value_cache_fp8.device)
-    if ok.shape != (tcount, nh, hd) or ov.shape != (tcount, nh, hd):
-        raise ValueError("kv_paged_fp8_to_linear: output shape mismatch")
-    if ok.dtype is not out_dtype or ov.dtype is not out_dtype:
-        raise ValueError("kv_paged_fp8_to_linear: output dtype mismatch")
-    _require_rocm(op, key_cache_fp8)
-    _fp8_gather(op, key_cache_fp8, value_cache_fp8, slots, ks, vs, fp8_format=fp8_format, out_dtype=out_dtype,
-                out_k=ok, out_v=ov, nl=1, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=0)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        ks = _ensure_fp8_scale(k_scale, device=key_cache_fp8.device, name="k_scale", num_heads=nh, checks=checks)
+        vs = _ensure_fp8_scale(v_scale, device=value_cache_fp8.device, name="v_scale", num_heads=nh, checks=checks)
+        ok = out_k if out_k is not None else torch.empty(tcount, nh, hd, dtype=out_dtype, device=key_cache_fp8.device)
+        ov = out_v if out_v is not None else torch.empty(tcount, nh, hd, dtype=out_dtype, device=value_cache_fp8.device)
+        if ok.shape != (tcount, nh, hd) or ov.shape != (tcount, nh, hd):
+            raise ValueError("kv_paged_fp8_to_linear: output shape mismatch")
+        if ok.dtype is not out_dtype or ov.dtype is not out_dtype:
+            raise ValueError("kv_paged_fp8_to_linear: output dtype mismatch")
+        _require_rocm(op, key_cache_fp8)
+        _fp8_gather(checks, key_cache_fp8, value_cache_fp8, ks, vs, fp8_format=fp8_format, out_dtype=out_dtype,
+                    out_k=ok, out_v=ov, nl=1, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=0)
     _emit(op, key_cache_fp8, f"gfx950 fused {fp8_format.upper()} dequantize gather")
     return ok, ov
 
@@ -793,12 +843,14 @@ def kv_linear_to_paged_fp8_multi_layer(
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
     if slots.device != key_linear.device:
         raise ValueError("kv_linear_to_paged_fp8_multi_layer: slot_mapping must be on the same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    ks = _ensure_fp8_scale(k_scale, device=key_linear.device, name="k_scale", num_heads=nh, num_layers=nl)
-    vs = _ensure_fp8_scale(v_scale, device=value_linear.device, name="v_scale", num_heads=nh, num_layers=nl)
-    _require_rocm(op, key_linear)
-    _fp8_scatter(op, key_linear, value_linear, key_cache_fp8, value_cache_fp8, slots, ks, vs, fp8_format=fp8_format,
-                 nl=nl, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=1)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        ks = _ensure_fp8_scale(k_scale, device=key_linear.device, name="k_scale", num_heads=nh, num_layers=nl,
+                               checks=checks)
+        vs = _ensure_fp8_scale(v_scale, device=value_linear.device, name="v_scale", num_heads=nh, num_layers=nl,
+                               checks=checks)
+        _require_rocm(op, key_linear)
+        _fp8_scatter(checks, key_linear, value_linear, key_cache_fp8, value_cache_fp8, ks, vs, fp8_format=fp8_format,
+                     nl=nl, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=1)
     _emit(op, key_linear, f"gfx950 fused {fp8_format.upper()} quantize scatter ({nl} layers)")
 
 
@@ -824,19 +876,21 @@ def kv_paged_fp8_to_linear_multi_layer(
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
     if slots.device != key_cache_fp8.device:
         raise ValueError("kv_paged_fp8_to_linear_multi_layer: slot_mapping must be on the same device")
-    _check_slots_in_bounds(slots, nb, bs, op)
-    ks = _ensure_fp8_scale(k_scale, device=key_cache_fp8.device, name="k_scale", num_heads=nh, num_layers=nl)
-    vs = _ensure_fp8_scale(v_scale, device=value_cache_fp8.device, name="v_scale", num_heads=nh, num_layers=nl)
-    shape = (nl, tcount, nh, hd)
-    ok = out_k if out_k is not None else torch.empty(shape, dtype=out_dtype, device=key_cache_fp8.device)
-    ov = out_v if out_v is not None else torch.empty(shape, dtype=out_dtype, device=value_cache_fp8.device)
-    if ok.shape != shape or ov.shape != shape:
-        raise ValueError("kv_paged_fp8_to_linear_multi_layer: output shape mismatch")
-    if ok.dtype is not out_dtype or ov.dtype is not out_dtype:
-        raise ValueError("kv_paged_fp8_to_linear_multi_layer: output dtype mismatch")
-    _require_rocm(op, key_cache_fp8)
-    _fp8_gather(op, key_cache_fp8, value_cache_fp8, slots, ks, vs, fp8_format=fp8_format, out_dtype=out_dtype,
-                out_k=ok, out_v=ov, nl=nl, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=1)
+    with _ValueChecks(op, slots, nb, bs) as checks:
+        ks = _ensure_fp8_scale(k_scale, device=key_cache_fp8.device, name="k_scale", num_heads=nh, num_layers=nl,
+                               checks=checks)
+        vs = _ensure_fp8_scale(v_scale, device=value_cache_fp8.device, name="v_scale", num_heads=nh, num_layers=nl,
+                               checks=checks)
+        shape = (nl, tcount, nh, hd)
+        ok = out_k if out_k is not None else torch.empty(shape, dtype=out_dtype, device=key_cache_fp8.device)
+        ov = out_v if out_v is not None else torch.empty(shape, dtype=out_dtype, device=value_cache_fp8.device)
+        if ok.shape != shape or ov.shape != shape:
+            raise ValueError("kv_paged_fp8_to_linear_multi_layer: output shape mismatch")
+        if ok.dtype is not out_dtype or ov.dtype is not out_dtype:
+            raise ValueError("kv_paged_fp8_to_linear_multi_layer: output dtype mismatch")
+        _require_rocm(op, key_cache_fp8)
+        _fp8_gather(checks, key_cache_fp8, value_cache_fp8, ks, vs, fp8_format=fp8_format, out_dtype=out_dtype,
+                    out_k=ok, out_v=ov, nl=nl, tcount=tcount, nb=nb, nh=nh, hd=hd, bs=bs, token_dim=1)
     _emit(op, key_cache_fp8, f"gfx950 fused {fp8_format.upper()} dequantize gather ({nl} layers)")
     return ok, ov
 
