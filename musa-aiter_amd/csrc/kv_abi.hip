@@ -1711,12 +1711,12 @@ int musa_aiter_hip_cachegen_encode(const void* input, int input_dtype, int64_t n
                                    int64_t workspace_bytes, void* stream) {
   if (numel <= 0) return hipSuccess;
   if (input == nullptr || encoded == nullptr || codebook == nullptr || cdf == nullptr || workspace == nullptr ||
-      num_bins < 2 || num_bins > 256 || workspace_bytes < kvhip::kCacheGenWorkspaceBytes ||
+      num_bins < 2 || num_bins > 256 || workspace_bytes < kvhip::kCacheGenMinWorkspaceBytes ||
       (native_rounding != 0 && input_dtype != kvhip::kCgF32))
     return hipErrorInvalidValue;
   return kvhip::launch_cachegen_encode(input, input_dtype, numel, static_cast<int>(num_bins), native_rounding != 0,
                                        static_cast<uint8_t*>(encoded), static_cast<float*>(codebook),
-                                       static_cast<float*>(cdf), workspace, as_stream(stream));
+                                       static_cast<float*>(cdf), workspace, workspace_bytes, as_stream(stream));
 }
 
 int musa_aiter_hip_cachegen_decode(const void* encoded, int64_t numel, const void* table, int64_t table_len,

@@ -82,11 +82,22 @@ __device__ __forceinline__ void for_chunk(int64_t c, int64_t per_chunk, int64_t 
   }
 }
 
-// Workspace layout: the 256 bin counters, the per-workgroup (min, max) pairs.
-constexpr int64_t kCgCountsOffset = 0;
+// Workspace layout: copies of the 256 bin counters and the per-workgroup (min,
+// max) pairs.  Workgroup g of the bin pass adds its counts to copy g % copies:
+// with a single copy every workgroup's 256 atomics met on the same 16 lines,
+// one after another, which took the bin pass of a 256-token chunk (16.8 M
+// values) 30 us against 15 us with 32 copies.
+constexpr int64_t kCgCountBytes = 256 * 8;
 constexpr int64_t kCgPairsOffset = 4096;
-static_assert(kCgCountsOffset + 256 * 8 <= kCgPairsOffset, "workspace layout");
-static_assert(kCgPairsOffset + int64_t{kCgMinmaxGroups} * 8 <= kCacheGenWorkspaceBytes, "workspace too small");
+constexpr int64_t kCgCopiesOffset = kCgPairsOffset + int64_t{kCgMinmaxGroups} * 8;  // copies 1, 2, ...
+constexpr int kCgMaxCopies = 32;
+static_assert(kCgCountBytes <= kCgPairsOffset, "workspace layout");
+static_assert(kCgCopiesOffset + (kCgMaxCopies - 1) * kCgCountBytes == kCacheGenWorkspaceBytes &&
+                  kCgCopiesOffset <= kCacheGenMinWorkspaceBytes, "workspace size");
+
+__device__ __forceinline__ uint64_t* cg_counts(uint8_t* ws, int copy) {
+  return reinterpret_cast<uint64_t*>(copy == 0 ? ws : ws + kCgCopiesOffset + (copy - 1) * kCgCountBytes);
+}
 
 template <int IN>
 struct CgIn;
@@ -168,8 +179,7 @@ __device__ __forceinline__ MinMax block_minmax(MinMax m) {
 
 template <int IN, bool VEC>
 __global__ __launch_bounds__(kBlockThreads) void cg_minmax_kernel(const uint8_t* __restrict__ x, int64_t n,
-                                                                  float2* __restrict__ pairs,
-                                                                  uint64_t* __restrict__ counts) {
+                                                                  uint8_t* __restrict__ ws, int32_t copies) {
   constexpr int kEps = 16 / CgIn<IN>::kBytes;
   const int64_t tid = static_cast<int64_t>(blockIdx.x) * kBlockThreads + threadIdx.x;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlockThreads;
@@ -192,8 +202,9 @@ __global__ __launch_bounds__(kBlockThreads) void cg_minmax_kernel(const uint8_t*
   }
   for (int64_t i = first_scalar + tid; i < n; i += stride) m.fold(cg_load1<IN>(x, i));
   const MinMax r = block_minmax(m);
-  if (threadIdx.x == 0) pairs[blockIdx.x] = make_float2(r.mn, r.mx);
-  if (blockIdx.x == 0) counts[threadIdx.x] = 0;  // kBlockThreads == 256 counters
+  if (threadIdx.x == 0) reinterpret_cast<float2*>(ws + kCgPairsOffset)[blockIdx.x] = make_float2(r.mn, r.mx);
+  if (static_cast<int>(blockIdx.x) < copies)  // (at most one copy per workgroup)
+    cg_counts(ws, static_cast<int>(blockIdx.x))[threadIdx.x] = 0;  // kBlockThreads == 256 counters
 }
 
 struct CgEncodeArgs {
@@ -202,7 +213,8 @@ struct CgEncodeArgs {
   int64_t n;
   const float2* pairs;  // null: min_arg / scale_arg given by the caller, no histogram
   int32_t num_pairs;
-  uint64_t* counts;
+  uint8_t* ws;
+  int32_t copies;
   float* codebook;
   int32_t num_bins;
   float min_arg;
@@ -235,20 +247,22 @@ __device__ __forceinline__ uint32_t cg_bin(float x, float mn, float scale, float
 // cdf[0] = 0, cdf[t + 1] = (prefix of float32(count)) / numel, for the workgroup's 256 threads
 // holding counts[t]: each count rounded to float32, prefix sums in double (exact: integers below
 // 2**53), rounded to float32, divided by numel in float32.
+// (Every sum is exact, so a wave's shuffles and the four wave totals add up in any order.)
 __device__ __forceinline__ void cg_write_cdf(uint64_t count, int nb, int64_t numel, float* cdf) {
-  __shared__ double scan[2][256];
+  __shared__ double totals[kWavesPerBlock];
   const int t = threadIdx.x;
-  scan[0][t] = t < nb ? static_cast<double>(static_cast<float>(count)) : 0.0;
-  __syncthreads();
-  int cur = 0;
-  for (int off = 1; off < 256; off <<= 1) {
-    const double v = scan[cur][t] + (t >= off ? scan[cur][t - off] : 0.0);
-    scan[cur ^ 1][t] = v;
-    cur ^= 1;
-    __syncthreads();
+  const int lane = lane_id();
+  double v = t < nb ? static_cast<double>(static_cast<float>(count)) : 0.0;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const double before = __shfl_up(v, off);
+    v += lane >= off ? before : 0.0;
   }
+  if (lane == kWave - 1) totals[wave_in_block()] = v;
+  __syncthreads();
+  for (int w = 0; w < wave_in_block(); ++w) v += totals[w];
   if (t == 0) cdf[0] = 0.0f;
-  if (t < nb) cdf[t + 1] = static_cast<float>(scan[cur][t]) / static_cast<float>(numel);
+  if (t < nb) cdf[t + 1] = static_cast<float>(v) / static_cast<float>(numel);
 }
 
 template <int IN, bool NATIVE, bool HIST, bool VEC>
@@ -351,7 +365,9 @@ __global__ __launch_bounds__(kBlockThreads) void cg_encode_kernel(CgEncodeArgs a
 #pragma unroll
         for (int c = 0; c < kCgHistCopies; ++c) sum += hist[w][t * kCgHistCopies + c];
       if (sum != 0)
-        atomicAdd(reinterpret_cast<unsigned long long*>(&a.counts[t]), static_cast<unsigned long long>(sum));
+        atomicAdd(reinterpret_cast<unsigned long long*>(
+                      &cg_counts(a.ws, static_cast<int>(blockIdx.x % static_cast<uint32_t>(a.copies)))[t]),
+                  static_cast<unsigned long long>(sum));
     }
   }
 }
@@ -359,10 +375,15 @@ __global__ __launch_bounds__(kBlockThreads) void cg_encode_kernel(CgEncodeArgs a
 // One workgroup, after cg_encode_kernel: the counters into cdf[num_bins + 1].  (Finishing in the
 // encode kernel's last workgroup would need a device-scope release fence in every workgroup,
 // which writes back L2 and costs far more than this launch.)
-__global__ __launch_bounds__(kBlockThreads) void cg_cdf_kernel(const uint64_t* __restrict__ counts, int32_t nb,
+__global__ __launch_bounds__(kBlockThreads) void cg_cdf_kernel(uint8_t* __restrict__ ws, int32_t copies, int32_t nb,
                                                                int64_t numel, float* __restrict__ cdf) {
-  const int t = threadIdx.x;
-  cg_write_cdf(t < nb ? counts[t] : 0, nb, numel, cdf);
+  uint64_t part[kCgMaxCopies];
+#pragma unroll
+  for (int c = 0; c < kCgMaxCopies; ++c) part[c] = c < copies ? cg_counts(ws, c)[threadIdx.x] : 0;
+  uint64_t count = 0;
+#pragma unroll
+  for (int c = 0; c < kCgMaxCopies; ++c) count += part[c];
+  cg_write_cdf(count, nb, numel, cdf);
 }
 
 struct CgDecodeArgs {
@@ -488,22 +509,24 @@ int cg_groups(int64_t units, int vecs, int cap) {
 
 template <int IN>
 hipError_t encode_typed(const uint8_t* x, int64_t n, int nb, bool native, uint8_t* enc, float* codebook, float* cdf,
-                        uint8_t* ws, hipStream_t stream) {
+                        uint8_t* ws, int64_t ws_bytes, hipStream_t stream) {
   constexpr int kEps = 16 / CgIn<IN>::kBytes;
   const bool vec = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(enc) % kEps) == 0;
   const int64_t units = vec ? n / kEps : n;
   const int mgroups = cg_groups(units, kCgMinmaxVecs, kCgMinmaxGroups);
   const int groups = cg_groups(units, kCgEncodeVecs, kCgEncodeGroups);
-  uint64_t* counts = reinterpret_cast<uint64_t*>(ws + kCgCountsOffset);
-  float2* pairs = reinterpret_cast<float2*>(ws + kCgPairsOffset);
+  int copies = kCgMaxCopies;
+  if (copies > 1 + (ws_bytes - kCgCopiesOffset) / kCgCountBytes)
+    copies = static_cast<int>(1 + (ws_bytes - kCgCopiesOffset) / kCgCountBytes);
+  if (copies > mgroups) copies = mgroups;
+  const float2* pairs = reinterpret_cast<const float2*>(ws + kCgPairsOffset);
   if (vec)
-    hipLaunchKernelGGL((cg_minmax_kernel<IN, true>), dim3(mgroups), dim3(kBlockThreads), 0, stream, x, n, pairs, counts);
+    hipLaunchKernelGGL((cg_minmax_kernel<IN, true>), dim3(mgroups), dim3(kBlockThreads), 0, stream, x, n, ws, copies);
   else
-    hipLaunchKernelGGL((cg_minmax_kernel<IN, false>), dim3(mgroups), dim3(kBlockThreads), 0, stream, x, n, pairs,
-                       counts);
+    hipLaunchKernelGGL((cg_minmax_kernel<IN, false>), dim3(mgroups), dim3(kBlockThreads), 0, stream, x, n, ws, copies);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
-  CgEncodeArgs a{x, enc, n, pairs, mgroups, counts, codebook, nb, 0.0f, 0.0f};
+  CgEncodeArgs a{x, enc, n, pairs, mgroups, ws, copies, codebook, nb, 0.0f, 0.0f};
   if (native) {
     if (vec) hipLaunchKernelGGL((cg_encode_kernel<IN, true, true, true>), dim3(groups), dim3(kBlockThreads), 0, stream, a);
     else hipLaunchKernelGGL((cg_encode_kernel<IN, true, true, false>), dim3(groups), dim3(kBlockThreads), 0, stream, a);
@@ -513,7 +536,7 @@ hipError_t encode_typed(const uint8_t* x, int64_t n, int nb, bool native, uint8_
   }
   err = hipGetLastError();
   if (err != hipSuccess) return err;
-  hipLaunchKernelGGL(cg_cdf_kernel, dim3(1), dim3(kBlockThreads), 0, stream, counts, nb, n, cdf);
+  hipLaunchKernelGGL(cg_cdf_kernel, dim3(1), dim3(kBlockThreads), 0, stream, ws, copies, nb, n, cdf);
   return hipGetLastError();
 }
 
@@ -538,15 +561,16 @@ hipError_t decode_typed(const uint8_t* codes, int64_t n, const uint8_t* table, i
 }  // namespace
 
 hipError_t launch_cachegen_encode(const void* x, int in_dtype, int64_t n, int num_bins, bool native, uint8_t* enc,
-                                  float* codebook, float* cdf, void* workspace, hipStream_t stream) {
+                                  float* codebook, float* cdf, void* workspace, int64_t workspace_bytes,
+                                  hipStream_t stream) {
   if (n <= 0) return hipSuccess;
   const uint8_t* xs = static_cast<const uint8_t*>(x);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   switch (in_dtype) {
-    case kCgF32: return encode_typed<kCgF32>(xs, n, num_bins, native, enc, codebook, cdf, ws, stream);
-    case kCgF16: return encode_typed<kCgF16>(xs, n, num_bins, false, enc, codebook, cdf, ws, stream);
-    case kCgBF16: return encode_typed<kCgBF16>(xs, n, num_bins, false, enc, codebook, cdf, ws, stream);
-    case kCgF64: return encode_typed<kCgF64>(xs, n, num_bins, false, enc, codebook, cdf, ws, stream);
+    case kCgF32: return encode_typed<kCgF32>(xs, n, num_bins, native, enc, codebook, cdf, ws, workspace_bytes, stream);
+    case kCgF16: return encode_typed<kCgF16>(xs, n, num_bins, false, enc, codebook, cdf, ws, workspace_bytes, stream);
+    case kCgBF16: return encode_typed<kCgBF16>(xs, n, num_bins, false, enc, codebook, cdf, ws, workspace_bytes, stream);
+    case kCgF64: return encode_typed<kCgF64>(xs, n, num_bins, false, enc, codebook, cdf, ws, workspace_bytes, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -556,7 +580,7 @@ hipError_t launch_cachegen_bins(const float* x, uint8_t* enc, float min_val, flo
   if (n <= 0) return hipSuccess;
   const uint8_t* xs = reinterpret_cast<const uint8_t*>(x);
   const bool vec = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(enc) & 3) == 0;
-  CgEncodeArgs a{xs, enc, n, nullptr, 0, nullptr, nullptr, num_bins, min_val, scale};
+  CgEncodeArgs a{xs, enc, n, nullptr, 0, nullptr, 1, nullptr, num_bins, min_val, scale};
   const int groups = cg_groups(vec ? n / 4 : n, kCgEncodeVecs, kCgEncodeGroups);
   if (vec) hipLaunchKernelGGL((cg_encode_kernel<kCgF32, true, false, true>), dim3(groups), dim3(kBlockThreads), 0, stream, a);
   else hipLaunchKernelGGL((cg_encode_kernel<kCgF32, true, false, false>), dim3(groups), dim3(kBlockThreads), 0, stream, a);

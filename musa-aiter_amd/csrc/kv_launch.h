@@ -55,10 +55,12 @@ struct PagedTileParams {
 hipError_t launch_paged_tiles(const PagedTileParams& p, hipStream_t stream);
 
 // One launch ahead of a checked call's kernel (kv_rows.hip): `groups`
-// workgroups check that every idx entry lies below `rows` and every scale is
-// positive and finite, claim the tokens' destinations as launch_claim does
-// (owner set), write their verdicts to check.report[0, groups) and, where
-// something is refused, the call's stamp to check.guard.
+// workgroups check that every entry of idx (and of `other`) lies in [low,
+// rows) (other_rows) and every scale is positive and finite, claim the
+// destinations idx as launch_claim does (owner set; a token whose `other`
+// entry, its source, is skipped claims nothing), write their verdicts to
+// check.report[0, groups) and, where something is refused, the call's stamp to
+// check.guard.
 struct CheckSource {
   const int64_t* idx;
   int64_t n;
@@ -202,14 +204,17 @@ hipError_t launch_block_pattern(const BlockPatternParams& p, hipStream_t stream)
 // Input element types of the encoder.
 enum CacheGenInput : int { kCgF32 = 0, kCgF16 = 1, kCgBF16 = 2, kCgF64 = 3 };
 
-// Device workspace the encoder needs (per-workgroup ranges and the bin counters).
-constexpr int64_t kCacheGenWorkspaceBytes = 16384;
+// Device workspace of the encoder (per-workgroup ranges and copies of the bin
+// counters): the size it uses in full, and the least it takes (fewer copies).
+constexpr int64_t kCacheGenWorkspaceBytes = 75776;
+constexpr int64_t kCacheGenMinWorkspaceBytes = 16384;
 
 // Bins of the `n` elements of `x` over their own [min, max] (torch-path rounding, or the
 // reference kernel's when `native`; float32 input only), the codebook[num_bins] and the
 // cdf[num_bins + 1]; three launches, no host synchronisation.
 hipError_t launch_cachegen_encode(const void* x, int in_dtype, int64_t n, int num_bins, bool native, uint8_t* enc,
-                                  float* codebook, float* cdf, void* workspace, hipStream_t stream);
+                                  float* codebook, float* cdf, void* workspace, int64_t workspace_bytes,
+                                  hipStream_t stream);
 
 // Bins of float32 `x` with a caller-given minimum and scale, the reference kernel's rounding.
 hipError_t launch_cachegen_bins(const float* x, uint8_t* enc, float min_val, float scale, int64_t n, int num_bins,
