@@ -370,17 +370,18 @@ int paged_tiles(int scatter, int codec, int cache_elt, int lin_elt, int lin_dtyp
   return kvhip::launch_paged_tiles(p, stream);
 }
 
-// Waits until each of `words` verdict words carries `stamp`; *refused tells
-// whether any of them refuses the call.  The words arrive as the checking
+// Waits until each of `words` verdict words, `pitch` words apart, carries
+// `stamp`; *refused tells whether any of them refuses the call.  The words arrive as the checking
 // kernel runs, so polling them returns sooner than a stream synchronisation; a
 // kernel that has not run after 0.2 s (the stream busy with earlier work) is
 // waited for by the synchronisation.
-hipError_t await_verdict(const int64_t* report, int64_t words, int64_t stamp, hipStream_t stream, bool* refused) {
+hipError_t await_verdict(const int64_t* report, int64_t words, int64_t stamp, hipStream_t stream, bool* refused,
+                         int64_t pitch = 1) {
   const auto deadline = std::chrono::steady_clock::now() + std::chrono::milliseconds(200);
   *refused = false;
   bool synced = false;
   for (int64_t w = 0; w < words;) {
-    const int64_t v = __atomic_load_n(&report[w], __ATOMIC_ACQUIRE);
+    const int64_t v = __atomic_load_n(&report[w * pitch], __ATOMIC_ACQUIRE);
     if ((v >> 1) == stamp) {
       *refused = *refused || (v & 1) != 0;
       ++w;
@@ -449,6 +450,7 @@ int paged_tiles_checked(const musa_aiter_hip_paged_tiles_call& c, hipStream_t st
   src.idx = c.slot_mapping;
   src.n = c.num_tokens;
   src.rows = c.num_blocks * c.block_size;
+  src.low = INT64_MIN;
   if (c.codec != kvhip::kCopy) {
     src.scale[0] = c.k_scale;
     src.scale[1] = c.v_scale != nullptr ? c.v_scale : c.k_scale;
@@ -791,6 +793,27 @@ int musa_aiter_hip_paged_tiles(int scatter, int codec, int cache_elt, int lin_el
 
 int musa_aiter_hip_paged_tiles_checked(const musa_aiter_hip_paged_tiles_call* call, void* stream) {
   return call == nullptr ? static_cast<int>(hipErrorInvalidValue) : paged_tiles_checked(*call, as_stream(stream));
+}
+
+int musa_aiter_hip_block_tables_check(const int64_t* block_tables, const int64_t* seq_lens, int64_t batch,
+                                      int64_t max_blocks, int64_t num_blocks, int64_t block_size, int64_t* report,
+                                      int64_t report_words, int64_t stamp, int64_t* out, void* stream) {
+  if (report == nullptr || report_words < 3 || stamp <= 0 || out == nullptr) return hipErrorInvalidValue;
+  const int64_t groups = batch < report_words / 3 ? batch : report_words / 3;
+  hipError_t err = kvhip::launch_table_check(block_tables, seq_lens, batch, max_blocks, num_blocks, block_size, report,
+                                             stamp, groups, as_stream(stream));
+  if (err != hipSuccess) return err;
+  bool refused = false;
+  err = await_verdict(report + 2, groups, stamp, as_stream(stream), &refused, 3);
+  if (err != hipSuccess) return err;
+  out[0] = report[0];
+  out[1] = report[1];
+  out[2] = refused ? 1 : 0;
+  for (int64_t g = 1; g < groups; ++g) {
+    out[0] = report[3 * g] < out[0] ? report[3 * g] : out[0];
+    out[1] = report[3 * g + 1] > out[1] ? report[3 * g + 1] : out[1];
+  }
+  return hipSuccess;
 }
 
 int musa_aiter_hip_paged_tiles_noalloc(int scatter, int codec, int cache_elt, int lin_elt, int lin_dtype,
@@ -1420,6 +1443,54 @@ int musa_aiter_hicache_transfer_abi_version() { return 1; }
 // the host; either side may use paged row addressing.  Tokens whose source or
 // destination index lies outside [0, rows) are skipped; with `dedupe` a
 // destination row named by several tokens keeps the last one.
+int musa_aiter_hip_copy_rows_paged_checked(const musa_aiter_hip_copy_rows_paged_call* call, void* stream) {
+  if (call == nullptr) return hipErrorInvalidValue;
+  const musa_aiter_hip_copy_rows_paged_call& c = *call;
+  if (c.num_tokens <= 0 || c.num_planes <= 0 || c.row_bytes <= 0 || c.src_idx == nullptr || c.dst_idx == nullptr ||
+      c.report == nullptr || c.guard == nullptr || c.report_words < 1 || c.stamp <= 0 || c.claims == nullptr ||
+      c.claims->tags == nullptr || c.claims->capacity < c.dst_rows || c.claims->epoch == 0)
+    return hipErrorInvalidValue;
+  RowCopyParams p{};
+  p.src_planes = c.src_planes;
+  p.dst_planes = c.dst_planes;
+  p.num_planes = c.num_planes;
+  p.src_idx = c.src_idx;
+  p.dst_idx = c.dst_idx;
+  p.num_tokens = c.num_tokens;
+  p.num_rows_out = c.num_tokens;
+  p.src_rows = c.src_rows;
+  p.dst_rows = c.dst_rows;
+  p.row_bytes = c.row_bytes;
+  p.src_stride = c.src_stride;
+  p.dst_stride = c.dst_stride;
+  p.src_page_rows = c.src_page_rows;
+  p.src_page_stride = c.src_page_stride;
+  p.dst_page_rows = c.dst_page_rows;
+  p.dst_page_stride = c.dst_page_stride;
+  kvhip::CheckSource src{};
+  src.idx = c.dst_idx;
+  src.rows = c.dst_rows;
+  src.other = c.src_idx;
+  src.other_rows = c.src_rows;
+  src.low = c.low;
+  src.n = c.num_tokens;
+  if (c.num_tokens > 1) {
+    p.owner = src.owner = c.claims->tags;
+    p.epoch = src.epoch = c.claims->epoch;
+    p.owner_exclusive = 1;
+  }
+  int64_t groups = (c.num_tokens + kCheckPerGroup - 1) / kCheckPerGroup;
+  if (groups > c.report_words) groups = c.report_words;
+  hipError_t err = kvhip::launch_check(src, kvhip::CallCheck{c.report, c.guard, c.stamp}, groups, as_stream(stream));
+  if (err != hipSuccess) return err;
+  p.check = kvhip::CallCheck{nullptr, c.guard, c.stamp};
+  const hipError_t moved = kvhip::launch_row_copy(p, as_stream(stream));
+  bool refused = false;
+  err = await_verdict(c.report, groups, c.stamp, as_stream(stream), &refused);
+  if (err != hipSuccess || refused) return err != hipSuccess ? static_cast<int>(err) : MUSA_AITER_HIP_REFUSED;
+  return moved;
+}
+
 int musa_aiter_hip_copy_rows_paged(const uint64_t* src_planes, const uint64_t* dst_planes, int64_t num_planes,
                                    const int64_t* src_idx, const int64_t* dst_idx, int64_t num_tokens,
                                    int64_t src_rows, int64_t dst_rows, int64_t row_bytes, int64_t src_stride,

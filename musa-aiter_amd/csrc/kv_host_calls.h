@@ -33,6 +33,31 @@ typedef struct musa_aiter_hip_paged_tiles_call {
 } musa_aiter_hip_paged_tiles_call;
 int musa_aiter_hip_paged_tiles_checked(const musa_aiter_hip_paged_tiles_call* call, void* stream);
 
+/* musa_aiter_hip_copy_rows_paged (same fields) whose index entries are checked on the device as above:
+ * one outside [low, src_rows) or [low, dst_rows) refuses the call (negative entries skip their row). */
+typedef struct musa_aiter_hip_copy_rows_paged_call {
+  const uint64_t *src_planes, *dst_planes;
+  int64_t num_planes;
+  const int64_t *src_idx, *dst_idx;
+  int64_t num_tokens, src_rows, dst_rows, row_bytes, src_stride, dst_stride;
+  int64_t src_page_rows, src_page_stride, dst_page_rows, dst_page_stride;
+  int64_t low;
+  const musa_aiter_hip_claims* claims;
+  int64_t* report;
+  int64_t* guard;
+  int64_t report_words, stamp;
+} musa_aiter_hip_copy_rows_paged_call;
+int musa_aiter_hip_copy_rows_paged_checked(const musa_aiter_hip_copy_rows_paged_call* call, void* stream);
+
+/* Block tables [batch, max_blocks] and seq_lens [batch] (device, int64) of a dense call, read on the
+ * device: out[0] / out[1] receive the smallest and largest length, out[2] is 1 when a sequence uses a
+ * block id outside [0, num_blocks) (ids past ceil(len / block_size), and columns the table does not
+ * have, are not read), else 0.  report: report_words (>= 3) words of pinned host memory; `stamp` > 0
+ * differs from every earlier call on the same words.  Returns when the values are there. */
+int musa_aiter_hip_block_tables_check(const int64_t* block_tables, const int64_t* seq_lens, int64_t batch,
+                                      int64_t max_blocks, int64_t num_blocks, int64_t block_size, int64_t* report,
+                                      int64_t report_words, int64_t stamp, int64_t* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -53,6 +53,7 @@ struct RowArgs {
   int64_t src_page_stride;
   int64_t dst_page_rows;
   int64_t dst_page_stride;
+  CallCheck check;
   int32_t plane_inner;        // 1: one grid over (row, plane, piece), planes inside rows
   int32_t dst_major;          // 1: rows are destination rows, their tokens read from the claim tags (plane-major)
 };
@@ -129,6 +130,7 @@ __global__ __launch_bounds__(kBlockThreads) void row_flat_kernel(const RowArgs a
   using V = typename VecType<VEC>::T;
   __shared__ int64_t s_src[kBlockRows];
   __shared__ int64_t s_dst[kBlockRows];
+  if (refused_ahead(a.check)) return;
   constexpr bool inner = INNER;
   const int pp = inner ? 0 : a.plane_base + static_cast<int>(blockIdx.y);
   const uint8_t* const sp =
@@ -305,6 +307,57 @@ __global__ __launch_bounds__(kBlockThreads) void slot_row_kernel(const SlotRowAr
 
 __global__ __launch_bounds__(kBlockThreads) void claim_kernel(const int64_t* idx, int64_t idx_stride,
                                                               const BlockTableSlots bt, const int64_t* src_idx,
+// ----- rows of whole KiB named by a pair of index vectors: one wave per KiB --------------
+// HiCache items (a 2 KiB K or V row of 8 heads x 128): wave w moves one KiB of
+// row src_idx[u] to row dst_idx[u] of one plane, both offsets resolved with
+// scalar loads, no LDS and no barrier, as slot_row_kernel does for one index
+// vector.  INNER walks planes inside rows (one grid, see launch_row_copy),
+// otherwise grid y is the plane.  Bound by HBM (random 2 KiB reads): the
+// 4,096-item, 32-layer backup (1.07 GB) 192 us (5.6 TB/s), 209 us with the
+// block-resolving kernel, whose 8 KiB workgroups wait for an LDS round trip;
+// two KiB per wave 212 us, non-temporal stores 198 us.  XCD: each XCD takes a
+// contiguous eighth of a large grid (195 -> 192 us; 390 against 397 us for a
+// call of 8,192 items; 1 % slower for 500 items, which keep the natural order).
+struct PairRowArgs {
+  const int64_t* src_idx;
+  const int64_t* dst_idx;
+  const uint64_t* owner;
+  int64_t num_tokens;
+  int64_t src_rows;
+  int64_t dst_rows;
+  int64_t src_stride;
+  int64_t dst_stride;
+  uint32_t epoch;
+  uint32_t num_planes;
+  uint32_t row_kib;      // KiB per row
+  CallCheck check;
+  uint64_t src_planes[kMaxPlanes];
+  uint64_t dst_planes[kMaxPlanes];
+};
+
+template <bool INNER, int STP, bool XCD = false>
+__global__ __launch_bounds__(kBlockThreads) void pair_row_kernel(const PairRowArgs a) {
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const WgXyz wg = xcd_contiguous_wg<XCD>();
+  const uint32_t w = wg.x * kWavesPerBlock + wave;
+  const uint32_t per_row = INNER ? a.num_planes * a.row_kib : a.row_kib;
+  const uint32_t u = w / per_row;
+  if (u >= a.num_tokens) return;
+  const uint32_t rem = w - u * per_row;
+  const uint32_t plane = INNER ? rem / a.row_kib : wg.y;
+  const int64_t part = static_cast<int64_t>(INNER ? rem - plane * a.row_kib : rem) << 10;
+  const int64_t srow = a.src_idx[u], drow = a.dst_idx[u];
+  const uint64_t sbase = a.src_planes[plane], dbase = a.dst_planes[plane];
+  if (refused_ahead(a.check)) return;
+  if (srow < 0 || srow >= a.src_rows || drow < 0 || drow >= a.dst_rows) return;
+  const buf_t sb = make_buf(reinterpret_cast<const uint8_t*>(sbase) + srow * a.src_stride + part);
+  const buf_t db = make_buf(reinterpret_cast<uint8_t*>(dbase) + drow * a.dst_stride + part);
+  const uint32_t off = static_cast<uint32_t>(lane_id()) * 16u;
+  const u32x4 v = buf_ld16(sb, off);  // in flight while the claim is read
+  if (a.owner != nullptr && a.owner[drow] != claim_tag(a.epoch, u)) return;
+  buf_st16_p<STP>(db, off, v);
+}
+
                                                               int64_t src_rows, int64_t n, int64_t rows,
                                                               uint64_t* owner, uint32_t epoch, int reset) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -371,16 +424,22 @@ __global__ __launch_bounds__(kBlockThreads) void check_kernel(const CheckArgs a)
   bool bad = false;
   for (int64_t base = static_cast<int64_t>(blockIdx.x) * kCheckTokens; base < c.n;
        base += static_cast<int64_t>(gridDim.x) * kCheckTokens) {
-    int64_t s[4];
+    int64_t s[4], o[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int64_t i = base + k * kBlockThreads + threadIdx.x;
       s[k] = i < c.n ? c.idx[i] : -1;
+      o[k] = i < c.n && c.other != nullptr ? c.other[i] : c.other != nullptr ? -1 : 0;
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      bad |= s[k] >= c.rows;
-      if (c.owner != nullptr && s[k] >= 0 && s[k] < c.rows)
+      bad |= s[k] >= c.rows || s[k] < c.low;
+      bool moves = s[k] >= 0 && s[k] < c.rows;
+      if (c.other != nullptr) {
+        bad |= o[k] >= c.other_rows || o[k] < c.low;
+        moves = moves && o[k] >= 0 && o[k] < c.other_rows;
+      }
+      if (c.owner != nullptr && moves)
         atomicMax(reinterpret_cast<unsigned long long*>(c.owner + s[k]),
                   static_cast<unsigned long long>(claim_tag(c.epoch, base + k * kBlockThreads + threadIdx.x)));
     }
@@ -397,6 +456,41 @@ __global__ __launch_bounds__(kBlockThreads) void check_kernel(const CheckArgs a)
   if (refused) *a.guard = a.check.stamp;
   __hip_atomic_store(a.check.report + blockIdx.x, 2 * a.check.stamp + refused, __ATOMIC_RELEASE,
                      __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Sequence lengths and used block ids of [batch, max_blocks] tables: workgroup g
+// takes sequences g, g + grid, ... and reads ceil(len / block_size) ids of each
+// (at most the table's columns).  One kernel and three words per workgroup to
+// pinned memory stand for two device-to-host copies and a dozen host tensor
+// operations.
+__global__ __launch_bounds__(kBlockThreads) void table_check_kernel(const int64_t* tables, const int64_t* seq_lens,
+                                                                    int64_t batch, int64_t max_blocks,
+                                                                    int64_t num_blocks, int64_t block_size,
+                                                                    int64_t* report, int64_t stamp) {
+  int64_t lo = INT64_MAX, hi = INT64_MIN;
+  bool bad = false;
+  for (int64_t b = blockIdx.x; b < batch; b += gridDim.x) {
+    const int64_t len = seq_lens[b];
+    lo = len < lo ? len : lo;
+    hi = len > hi ? len : hi;
+    // len / block_size rounded up, without overflow for any length.
+    const int64_t need = len <= 0 ? 0 : (len - 1) / block_size + 1;
+    const int64_t used = need < max_blocks ? need : max_blocks;
+    for (int64_t j = threadIdx.x; j < used; j += kBlockThreads) {
+      const int64_t id = tables[b * max_blocks + j];
+      bad |= id < 0 || id >= num_blocks;
+    }
+  }
+  __shared__ int refused;
+  if (threadIdx.x == 0) refused = 0;
+  __syncthreads();
+  if (bad) refused = 1;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  int64_t* const r = report + 3 * static_cast<int64_t>(blockIdx.x);
+  r[0] = lo;
+  r[1] = hi;
+  __hip_atomic_store(r + 2, 2 * stamp + refused, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ----- strided block transfer ------------------------------------------------------
@@ -576,6 +670,7 @@ hipError_t launch_row_copy(const RowCopyParams& p, hipStream_t stream) {
   if (vec == 16 && (int64_t{1024} << shift) == p.row_bytes && src_host && dst_host && p.src_indptr == nullptr &&
       p.src_page_rows == 0 && p.dst_page_rows == 0 && p.idx_stride <= 1 && !inner && one_indexed &&
       p.num_tokens >= 1) {
+    if (p.check.guard != nullptr) return hipErrorInvalidValue;  // no checked call takes this kernel
     const bool scatter = p.dst_idx != nullptr;
     const bool dm = scatter && dst_major(p);
     const int64_t rows = dm ? p.dst_rows : (scatter ? p.num_tokens : p.num_rows_out);
@@ -649,6 +744,7 @@ hipError_t launch_row_copy(const RowCopyParams& p, hipStream_t stream) {
     a.src_page_stride = p.src_page_stride;
     a.dst_page_rows = p.dst_page_rows;
     a.dst_page_stride = p.dst_page_stride;
+    a.check = p.check;
     a.plane_inner = inner ? 1 : 0;
     if (!inner && p.src_indptr == nullptr && dst_major(p)) {
       a.dst_major = 1;
@@ -660,6 +756,51 @@ hipError_t launch_row_copy(const RowCopyParams& p, hipStream_t stream) {
       case 8: err = launch_rows_vec<8>(a, n, stream); break;
       case 4: err = launch_rows_vec<4>(a, n, stream); break;
       case 2: err = launch_rows_vec<2>(a, n, stream); break;
+  // Rows of whole KiB named by two packed index vectors: the per-KiB pair kernel.
+  if (vec == 16 && p.row_bytes % 1024 == 0 && p.src_idx != nullptr && p.dst_idx != nullptr && src_host && dst_host &&
+      p.src_indptr == nullptr && p.src_page_rows == 0 && p.dst_page_rows == 0 && p.idx_stride <= 1 && (inner || !dst_major(p))) {
+    const int64_t kib = p.row_bytes / 1024;
+    const int64_t planes = p.num_planes < kMaxPlanes ? p.num_planes : kMaxPlanes;
+    const int64_t waves = p.num_tokens * kib * (inner ? planes : 1);
+    if (waves <= 0x7FFFFFFF) {
+      for (int64_t base = 0; base < p.num_planes; base += kMaxPlanes) {
+        const int64_t n = (p.num_planes - base) < kMaxPlanes ? (p.num_planes - base) : kMaxPlanes;
+        PairRowArgs a{};
+        bool lines = p.dst_stride % 128 == 0;
+        for (int64_t i = 0; i < n; ++i) {
+          a.src_planes[i] = p.src_planes[base + i];
+          a.dst_planes[i] = p.dst_planes[base + i];
+          lines = lines && a.dst_planes[i] % 128 == 0;
+        }
+        a.src_idx = p.src_idx;
+        a.dst_idx = p.dst_idx;
+        a.owner = p.owner;
+        a.num_tokens = p.num_tokens;
+        a.src_rows = p.src_rows;
+        a.dst_rows = p.dst_rows;
+        a.src_stride = p.src_stride;
+        a.dst_stride = p.dst_stride;
+        a.epoch = p.epoch;
+        a.num_planes = static_cast<uint32_t>(n);
+        a.row_kib = static_cast<uint32_t>(kib);
+        a.check = p.check;
+        const int64_t all = p.num_tokens * kib * (inner ? n : 1);
+        const dim3 grid(static_cast<uint32_t>((all + kWavesPerBlock - 1) / kWavesPerBlock),
+                        inner ? 1u : static_cast<uint32_t>(n));
+        constexpr uint32_t kXcdGroups = 32768;  // workgroups from which a plane-inner grid takes the XCD order
+        if (inner && lines && grid.x >= kXcdGroups)
+          hipLaunchKernelGGL((pair_row_kernel<true, kBufWT, true>), grid, dim3(kBlockThreads), 0, stream, a);
+        else if (inner && lines) hipLaunchKernelGGL((pair_row_kernel<true, kBufWT>), grid, dim3(kBlockThreads), 0, stream, a);
+        else if (inner) hipLaunchKernelGGL((pair_row_kernel<true, kBufNT>), grid, dim3(kBlockThreads), 0, stream, a);
+        else if (lines) hipLaunchKernelGGL((pair_row_kernel<false, kBufWT>), grid, dim3(kBlockThreads), 0, stream, a);
+        else hipLaunchKernelGGL((pair_row_kernel<false, kBufNT>), grid, dim3(kBlockThreads), 0, stream, a);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess) return err;
+      }
+      return hipSuccess;
+    }
+  }
+
       default: err = launch_rows_vec<1>(a, n, stream); break;
     }
     if (err != hipSuccess) return err;
@@ -690,6 +831,17 @@ hipError_t launch_check(const CheckSource& src, const CallCheck& check, int64_t 
     return hipErrorInvalidValue;
   const CheckArgs a{src, check, const_cast<int64_t*>(check.guard)};
   hipLaunchKernelGGL(check_kernel, dim3(static_cast<uint32_t>(groups)), dim3(kBlockThreads), 0, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_table_check(const int64_t* tables, const int64_t* seq_lens, int64_t batch, int64_t max_blocks,
+                              int64_t num_blocks, int64_t block_size, int64_t* report, int64_t stamp, int64_t groups,
+                              hipStream_t stream) {
+  if (seq_lens == nullptr || (tables == nullptr && max_blocks > 0) || batch < 1 || max_blocks < 0 || block_size < 1 ||
+      report == nullptr || groups < 1)
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(table_check_kernel, dim3(static_cast<uint32_t>(groups)), dim3(kBlockThreads), 0, stream, tables,
+                     seq_lens, batch, max_blocks, num_blocks, block_size, report, stamp);
   return hipGetLastError();
 }
 

@@ -15,6 +15,7 @@ import importlib.util
 import struct
 import sysconfig
 import threading
+from array import array
 from pathlib import Path
 
 import torch
@@ -91,6 +92,9 @@ _SIGNATURES: dict[str, list] = {
     #  head_dim, block_size, stream); the "_fp8_vec8" entry copies one-byte elements.
     "musa_aiter_kv_copy_paged_blocks_fp8_vec8": [_c_void_p] * 5 + [_i64] * 7 + [_c_void_p],
     "musa_aiter_hip_paged_tiles_checked": [ctypes.c_char_p, _c_void_p],  # musa_aiter_hip_paged_tiles_call, stream
+    # (block_tables, seq_lens, batch, max_blocks, blocks, block_size, report, report_words, stamp, out, stream)
+    "musa_aiter_hip_block_tables_check": [_c_void_p] * 2 + [_i64] * 4 + [_c_void_p, _i64, _i64, _c_void_p, _c_void_p],
+    "musa_aiter_hip_copy_rows_paged_checked": [ctypes.c_char_p, _c_void_p],  # musa_aiter_hip_copy_rows_paged_call, stream
     "musa_aiter_hip_error_string": [_i32],
     "musa_aiter_hip_backend_name": [],
     "musa_aiter_hip_graph_claim_arrays": [],
@@ -311,7 +315,8 @@ def index_max(idx: torch.Tensor) -> int:
 # scale pointers, the claims pointer, report and guard addresses, report words and stamp.
 _PAGED_TILES_CALL = struct.Struct("<8i5Q8q2QQ2Q2q")
 _REFUSED = -1  # MUSA_AITER_HIP_REFUSED
-_REPORT_WORDS = 64
+_REPORT_WORDS = 192      # 64 workgroups of a table check at three words each
+_SLOT_CHECK_WORDS = 64   # workgroups of a slot check
 
 
 class _CheckSet:
@@ -364,13 +369,61 @@ def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, l
                 key_cache.data_ptr(), value_cache.data_ptr(), key_linear.data_ptr(), value_linear.data_ptr(),
                 slots.data_ptr(), num_layers, num_tokens, num_blocks, num_heads, head_dim, block_size,
                 lin_token_stride, lin_layer_stride, _data(k_scale), _data(v_scale), claims, checks.report_ptr,
-                checks.guard_ptr, _REPORT_WORDS, checks.stamp)
+                checks.guard_ptr, _SLOT_CHECK_WORDS, checks.stamp)
             rc = fn("musa_aiter_hip_paged_tiles_checked")(call, stream)
             del keep
     if rc == _REFUSED:
         return False
     check(rc, op)
     return True
+
+
+# musa_aiter_hip_copy_rows_paged_call: plane lists, planes, two index pointers, eleven int64 sizes,
+# strides and the lowest index, claims, report and guard addresses, report words and stamp.
+_COPY_ROWS_PAGED_CALL = struct.Struct("<2Qq2Q11q3Q2q")
+
+
+def copy_rows_paged_checked(*, op: str, device: torch.device, src_planes: list[int], dst_planes: list[int],
+                            src_idx: torch.Tensor, dst_idx: torch.Tensor, src_rows: int, dst_rows: int,
+                            row_bytes: int, src_stride: int, dst_stride: int, low: int) -> bool:
+    """copy_rows_paged (deduplicated, plain rows) whose index entries the device checks: False means that one
+    lay outside [low, src_rows) or [low, dst_rows) and nothing was moved.  Needs at least one row and
+    plane; not for a stream being captured."""
+    src, dst = array("Q", src_planes), array("Q", dst_planes)
+    with on_device(device):
+        stream = stream_ptr(device)
+        checks = _check_set(device, stream.value or 0)
+        with checks.lock:
+            claims, keep = claims_for(device, stream, dst_rows)
+            checks.stamp += 1
+            call = _COPY_ROWS_PAGED_CALL.pack(
+                src.buffer_info()[0], dst.buffer_info()[0], len(src), src_idx.data_ptr(), dst_idx.data_ptr(),
+                src_idx.numel(), src_rows, dst_rows, row_bytes, src_stride, dst_stride, 0, 0, 0, 0, low, claims,
+                checks.report_ptr, checks.guard_ptr, _SLOT_CHECK_WORDS, checks.stamp)
+            rc = fn("musa_aiter_hip_copy_rows_paged_checked")(call, stream)
+            del keep
+    if rc == _REFUSED:
+        return False
+    check(rc, op)
+    return True
+
+
+def block_tables_check(*, op: str, block_tables: torch.Tensor, seq_lens: torch.Tensor, num_blocks: int,
+                       block_size: int) -> tuple[int, int, bool]:
+    """(smallest length, largest length, whether a sequence uses a block id outside [0, num_blocks)) of
+    contiguous int64 device tables with at least one sequence; not for a stream being captured."""
+    device = seq_lens.device
+    with on_device(device):
+        stream = stream_ptr(device)
+        checks = _check_set(device, stream.value or 0)
+        out = (_i64 * 3)()
+        with checks.lock:
+            checks.stamp += 1
+            rc = fn("musa_aiter_hip_block_tables_check")(
+                block_tables.data_ptr(), seq_lens.data_ptr(), seq_lens.numel(), block_tables.shape[1], num_blocks,
+                block_size, checks.report_ptr, _REPORT_WORDS, checks.stamp, out, stream)
+    check(rc, op)
+    return out[0], out[1], bool(out[2])
 
 
 def allocated_bytes() -> int:

@@ -201,13 +201,21 @@ def _transfer(
         src_k, dst_k, src_v, dst_v, src_indices, dst_indices, src_layout, dst_layout, start_layer, num_layers,
         mla=mla,
     )
-    src_idx, dst_idx = _validate_page_indices(src_indices, dst_indices, src_geometry[1], dst_geometry[1],
-                                              dst_k.device)
     planes = [(src_k, dst_k)] if src_v is None else [(src_k, dst_k), (src_v, dst_v)]
+    # The index checks run on the device, in the launch that claims the destinations; the host makes them
+    # (with their errors) for an index that the device refused and where it cannot: off the device, under
+    # capture and for an empty table.
+    on_device = dst_k.is_cuda and src_indices.numel() > 0 and not torch.cuda.is_current_stream_capturing()
+    if on_device:
+        src_idx, dst_idx = (t.to(device=dst_k.device, dtype=torch.long).contiguous()
+                            for t in (src_indices, dst_indices))
+    else:
+        src_idx, dst_idx = _validate_page_indices(src_indices, dst_indices, src_geometry[1], dst_geometry[1],
+                                                  dst_k.device)
     _require_rocm("hicache_transfer", *(t for pair in planes for t in pair))
     layers = range(start_layer, start_layer + num_layers)
     bases = [(s.data_ptr(), d.data_ptr()) for s, d in planes]
-    _hip.copy_rows_paged(
+    call = dict(
         op="hicache_transfer",
         device=dst_k.device,
         src_planes=[s + layer * src_geometry[4] for s, _ in bases for layer in layers],
@@ -220,6 +228,10 @@ def _transfer(
         src_stride=src_geometry[3],
         dst_stride=dst_geometry[3],
     )
+    if not on_device or not _hip.copy_rows_paged_checked(**call, low=-1):
+        if on_device:
+            _validate_page_indices(src_idx, dst_idx, src_geometry[1], dst_geometry[1], dst_k.device)
+        _hip.copy_rows_paged(**call)
     device, dtype = tensor_device_dtype(src_k)
     emit(DispatchRecord("hicache_transfer", BACKEND, device, dtype,
                         f"gfx950 byte-stride row copy ({src_layout}->{dst_layout}, {num_layers} layers)"))

@@ -1012,11 +1012,35 @@ def _first_bad_block(block_tables_cpu: torch.Tensor, seq_lens_cpu: torch.Tensor,
     return first // max_blocks, int(block_tables_cpu.reshape(-1)[first].item())
 
 
+class _Tables:
+    """Block tables and sequence lengths of a dense call: as int64 device tensors for the kernel, and what the
+    checks need of them, read on the device when they are there (one kernel, three numbers), else on the host."""
+
+    def __init__(self, op: str, block_tables: torch.Tensor, seq_lens: torch.Tensor, nb: int, bs: int):
+        self.tables, self.lens, self.nb, self.bs = _index_tensor(block_tables), _index_tensor(seq_lens), nb, bs
+        self.min_len, self.max_len, self._bad_block = 0, 0, False
+        if self.lens.numel() == 0:
+            return
+        if self.lens.is_cuda and self.tables.is_cuda and _hip.is_available() \
+                and not torch.cuda.is_current_stream_capturing():
+            self.min_len, self.max_len, self._bad_block = _hip.block_tables_check(
+                op=op, block_tables=self.tables, seq_lens=self.lens, num_blocks=nb, block_size=bs)
+        else:
+            lens = self.lens.cpu()
+            self.min_len, self.max_len, self._bad_block = int(lens.min().item()), int(lens.max().item()), True
+
+    def first_bad_block(self, accepted: torch.Tensor | None = None) -> tuple[int, int] | None:
+        """_first_bad_block of the tables; ``accepted`` (host lengths) in place of the call's own."""
+        if not self._bad_block:
+            return None
+        return _first_bad_block(self.tables.cpu(), self.lens.cpu() if accepted is None else accepted, self.bs, self.nb)
+
+
 def _flash_dense_len(op: str, cache: torch.Tensor, value_cache: torch.Tensor, block_tables: torch.Tensor,
-                     seq_lens: torch.Tensor, max_seq_len: int | None, bs: int, *,
-                     joint_dtype_message: bool) -> tuple[int, torch.Tensor, torch.Tensor]:
+                     seq_lens: torch.Tensor, max_seq_len: int | None, nb: int, bs: int, *,
+                     joint_dtype_message: bool) -> tuple[int, _Tables]:
     """Shared block_tables / seq_lens validation of the Flash-style loads, in the reference's order
-    (:1541-1564 and :1741-1763, whose dtype messages differ); returns (dense_len, seq_lens, tables) on the CPU."""
+    (:1541-1564 and :1741-1763, whose dtype messages differ); returns (dense_len, tables)."""
     if block_tables.dim() != 2:
         raise ValueError(f"{op}: block_tables must be [batch, max_blocks]")
     if seq_lens.dim() != 1 or seq_lens.shape[0] != block_tables.shape[0]:
@@ -1032,16 +1056,16 @@ def _flash_dense_len(op: str, cache: torch.Tensor, value_cache: torch.Tensor, bl
             raise ValueError(f"{op}: block_tables must use an integer dtype")
         if seq_lens.dtype not in _INDEX_DTYPES:
             raise ValueError(f"{op}: seq_lens must use an integer dtype")
-    seq_lens_cpu = seq_lens.to(device="cpu", dtype=torch.long)
-    if seq_lens_cpu.numel() > 0 and int(seq_lens_cpu.min().item()) < 0:
+    tables = _Tables(op, block_tables, seq_lens, nb, bs)
+    if tables.min_len < 0:
         raise ValueError(f"{op}: seq_lens must be non-negative")
-    inferred_max = int(seq_lens_cpu.max().item()) if seq_lens_cpu.numel() > 0 else 0
+    inferred_max = tables.max_len
     dense_len = inferred_max if max_seq_len is None else int(max_seq_len)
     if dense_len < inferred_max:
         raise ValueError(f"{op}: max_seq_len is smaller than seq_lens max")
     if (dense_len + bs - 1) // bs > int(block_tables.shape[1]):
         raise ValueError(f"{op}: block_tables does not contain enough columns")
-    return dense_len, seq_lens_cpu, block_tables.to(device="cpu", dtype=torch.long)
+    return dense_len, tables
 
 
 def _dense_out(op: str, out: torch.Tensor | None, which: str, shape: tuple[int, ...], dtype: torch.dtype,
@@ -1141,13 +1165,13 @@ def kv_load_and_reshape_flash(
     """
     op = "kv_load_and_reshape_flash"
     nb, nh, hd, bs = _validate_paged_shapes(key_cache, value_cache, name=op)
-    dense_len, seq_lens_cpu, tables_cpu = _flash_dense_len(op, key_cache, value_cache, block_tables, seq_lens,
-                                                           max_seq_len, bs, joint_dtype_message=False)
+    dense_len, tables = _flash_dense_len(op, key_cache, value_cache, block_tables, seq_lens, max_seq_len, nb, bs,
+                                         joint_dtype_message=False)
     batch = int(block_tables.shape[0])
     shape = (batch, dense_len, nh, hd)
     out_k = _dense_out(op, out_k, "out_k", shape, key_cache.dtype, key_cache.device)
     out_v = _dense_out(op, out_v, "out_v", shape, value_cache.dtype, value_cache.device)
-    bad = _first_bad_block(tables_cpu, seq_lens_cpu, bs, nb)
+    bad = tables.first_bad_block()
     if bad is not None:
         raise ValueError(f"{op}: invalid block id {bad[1]}")
     elt = _float_elt(op, key_cache, value_cache)
@@ -1157,7 +1181,7 @@ def kv_load_and_reshape_flash(
     _hip.paged_dense_tiles(
         op=op, scatter=False, codec=_CODEC_COPY, cache_elt=elt, lin_elt=elt, lin_dtype=0,
         key_cache=caches.k, value_cache=caches.v, dense_k=wk, dense_v=wv,
-        block_tables=_index_tensor(block_tables), seq_lens=_index_tensor(seq_lens), batch=batch,
+        block_tables=tables.tables, seq_lens=tables.lens, batch=batch,
         dense_len=dense_len, max_blocks=int(block_tables.shape[1]), num_blocks=nb, num_heads=nh, head_dim=hd,
         block_size=bs, dense_token_stride=nh * hd, fill_zeros=True,
     )
@@ -1209,31 +1233,33 @@ def kv_reshape_and_cache_back_flash(
         raise ValueError(f"{op}: block_tables must use an integer dtype")
     if seq_lens.dtype not in _INDEX_DTYPES:
         raise ValueError(f"{op}: seq_lens must use an integer dtype")
-    seq_lens_cpu = seq_lens.to(device="cpu", dtype=torch.long)
-    tables_cpu = block_tables.to(device="cpu", dtype=torch.long)
     batch, dense_len = int(dense_k.shape[0]), int(dense_k.shape[1])
     max_blocks = int(block_tables.shape[1])
-    # The reference checks each sequence in turn (:1660-1676): length, table width, block ids.
-    bad_len = (seq_lens_cpu < 0) | (seq_lens_cpu > dense_len)
-    bad_width = (seq_lens_cpu.clamp(min=0) + bs - 1) // bs > max_blocks
-    bad_block = _first_bad_block(tables_cpu, torch.where(bad_len | bad_width, 0, seq_lens_cpu), bs, nb)
-    first = [int(bad_len.nonzero()[0].item()) if bool(bad_len.any()) else batch,
-             int(bad_width.nonzero()[0].item()) if bool(bad_width.any()) else batch,
-             bad_block[0] if bad_block is not None else batch]
-    b = min(first)
-    if b < batch:
-        if first[0] == b:
-            raise ValueError(f"{op}: seq_lens exceeds dense sequence length")
-        if first[1] == b:
-            raise ValueError(f"{op}: block_tables does not contain enough columns")
-        raise ValueError(f"{op}: invalid block id {bad_block[1]}")
+    tables = _Tables(op, block_tables, seq_lens, nb, bs)
+    bad_block = tables.first_bad_block()
+    if tables.min_len < 0 or tables.max_len > dense_len or (tables.max_len + bs - 1) // bs > max_blocks or bad_block:
+        # The reference checks each sequence in turn (:1660-1676): length, table width, block ids.
+        lens = tables.lens.cpu()
+        bad_len = (lens < 0) | (lens > dense_len)
+        bad_width = (lens.clamp(min=0) + bs - 1) // bs > max_blocks
+        bad_block = tables.first_bad_block(torch.where(bad_len | bad_width, 0, lens))
+        first = [int(bad_len.nonzero()[0].item()) if bool(bad_len.any()) else batch,
+                 int(bad_width.nonzero()[0].item()) if bool(bad_width.any()) else batch,
+                 bad_block[0] if bad_block is not None else batch]
+        b = min(first)
+        if b < batch:
+            if first[0] == b:
+                raise ValueError(f"{op}: seq_lens exceeds dense sequence length")
+            if first[1] == b:
+                raise ValueError(f"{op}: block_tables does not contain enough columns")
+            raise ValueError(f"{op}: invalid block id {bad_block[1]}")
     elt = _float_elt(op, dense_k, key_cache)
     _require_rocm(op, dense_k)
     caches = _CachePair(key_cache, value_cache, writable=True)
     _hip.paged_dense_tiles(
         op=op, scatter=True, codec=_CODEC_COPY, cache_elt=elt, lin_elt=elt, lin_dtype=0,
         key_cache=caches.k, value_cache=caches.v, dense_k=dense_k.contiguous(), dense_v=dense_v.contiguous(),
-        block_tables=_index_tensor(block_tables), seq_lens=_index_tensor(seq_lens), batch=batch,
+        block_tables=tables.tables, seq_lens=tables.lens, batch=batch,
         dense_len=dense_len, max_blocks=max_blocks, num_blocks=nb, num_heads=nh, head_dim=hd, block_size=bs,
         dense_token_stride=nh * hd, fill_zeros=False,
     )
@@ -1264,13 +1290,13 @@ def kv_load_and_dequantize_fp8_flash(
     """
     op = "kv_load_and_dequantize_fp8_flash"
     nb, nh, hd, bs = _validate_paged_shapes(key_cache_fp8, value_cache_fp8, name=op)
-    dense_len, seq_lens_cpu, tables_cpu = _flash_dense_len(op, key_cache_fp8, value_cache_fp8, block_tables,
-                                                           seq_lens, max_seq_len, bs, joint_dtype_message=True)
+    dense_len, tables = _flash_dense_len(op, key_cache_fp8, value_cache_fp8, block_tables, seq_lens, max_seq_len, nb,
+                                         bs, joint_dtype_message=True)
     batch = int(block_tables.shape[0])
     shape = (batch, dense_len, nh, hd)
     out_k = _dense_out(op, out_k, "out_k", shape, out_dtype, key_cache_fp8.device, exact_dtype=True)
     out_v = _dense_out(op, out_v, "out_v", shape, out_dtype, value_cache_fp8.device, exact_dtype=True)
-    bad = _first_bad_block(tables_cpu, seq_lens_cpu, bs, nb)
+    bad = tables.first_bad_block()
     if bad is not None:
         raise ValueError(f"{op}: invalid block id {bad[1]}")
     if batch == 0:
@@ -1289,7 +1315,7 @@ def kv_load_and_dequantize_fp8_flash(
     _hip.paged_dense_tiles(
         op=op, scatter=False, codec=_codec(fp8_format), cache_elt=1, lin_elt=_ELT[work_dtype],
         lin_dtype=_LIN_DTYPE[work_dtype], key_cache=caches.k, value_cache=caches.v, dense_k=wk, dense_v=wv,
-        block_tables=_index_tensor(block_tables), seq_lens=_index_tensor(seq_lens), batch=batch,
+        block_tables=tables.tables, seq_lens=tables.lens, batch=batch,
         dense_len=dense_len, max_blocks=int(block_tables.shape[1]), num_blocks=nb, num_heads=nh, head_dim=hd,
         block_size=bs, dense_token_stride=nh * hd, k_scale=ks, v_scale=vs, scale_mode=mode, fill_zeros=True,
     )

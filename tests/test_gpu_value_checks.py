@@ -126,3 +126,90 @@ def test_threads_on_streams_of_their_own():
     for t in threads:
         t.join()
     assert errors == []
+
+
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+@pytest.mark.parametrize("batch", [1, 3, 200])
+def test_block_tables_are_checked_on_the_device(index, batch):
+    bs, cols = 16, 5
+    nb = batch * cols + 3
+    gen = torch.Generator(device=DEV).manual_seed(batch)
+    caches = [torch.randn((nb, NH, HD, bs), generator=gen, device=DEV).to(torch.bfloat16) for _ in range(2)]
+    before = [c.clone() for c in caches]
+    tables = torch.randperm(nb, generator=gen, device=DEV)[:batch * cols].view(batch, cols).to(index)
+    lens = torch.full((batch,), 33, device=DEV, dtype=index)  # three blocks; the last sequence one token less
+    lens[-1] = 32
+    load, back = musa_aiter.kv_load_and_reshape_flash, musa_aiter.kv_reshape_and_cache_back_flash
+    unused = tables.clone()
+    unused[-1, 2] = -7      # past ceil(32 / 16): never read
+    unused[0, 3:] = nb + 9  # past ceil(33 / 16)
+    k, v = load(*caches, unused, lens)
+    assert k.shape == (batch, int(lens.max()), NH, HD)
+    assert back(k.neg(), v.neg(), *caches, unused, lens)
+    assert not torch.equal(caches[0], before[0])
+    assert back(k, v, *caches, tables, lens)
+    for c, b in zip(caches, before):
+        assert torch.equal(c, b)
+    for at, value in ((0, nb), (1, -1)):
+        bad = tables.clone()
+        bad[-1, at] = value
+        with pytest.raises(ValueError, match=f"invalid block id {value}"):
+            load(*caches, bad, lens)
+        with pytest.raises(ValueError, match=f"invalid block id {value}"):
+            back(k.neg(), v.neg(), *caches, bad, lens)
+    short = lens.clone()
+    short[-1] = -2
+    with pytest.raises(ValueError, match="seq_lens must be non-negative"):
+        load(*caches, tables, short)
+    with pytest.raises(ValueError, match="seq_lens exceeds dense sequence length"):
+        back(k.neg(), v.neg(), *caches, tables, short)
+    with pytest.raises(ValueError, match="smaller than seq_lens max"):
+        load(*caches, tables, lens, max_seq_len=31)
+    with pytest.raises(ValueError, match="enough columns"):
+        load(*caches, tables, lens, max_seq_len=cols * bs + 1)
+    wide = torch.zeros((batch, cols * bs + 1, NH, HD), device=DEV, dtype=torch.bfloat16)
+    long = lens.clone()
+    long[-1] = cols * bs + 1
+    with pytest.raises(ValueError, match="enough columns"):
+        back(wide, wide, *caches, tables, long)
+    for c, b in zip(caches, before):
+        assert torch.equal(c, b)
+
+
+@pytest.mark.parametrize("row", [512, 1024, 1536])  # 2-byte elements: rows of 1, 2 and 3 KiB
+@pytest.mark.parametrize("items,name", [(1, "per_layer"), (300, "all_layer"), (300, "all_layer_lf_pf"),
+                                        (2500, "all_layer_lf_pf"), (2500, "per_layer_pf_lf")])
+def test_hicache_page_indices_are_checked_on_the_device(row, items, name):
+    layers, pages = 3, items + 9
+    gen = torch.Generator(device=DEV).manual_seed(items + row)
+    call = getattr(musa_aiter, f"hicache_transfer_kv_{name}")
+    lf, pf = (layers, pages, row), (pages, layers, row)
+    shapes = {"per_layer": (lf, lf), "all_layer": (lf, lf), "all_layer_lf_pf": (lf, pf), "per_layer_pf_lf": (pf, lf)}
+    src, dst = ([torch.randn(shape, generator=gen, device=DEV).to(torch.bfloat16) for _ in range(2)]
+                for shape in shapes[name])
+    before = [d.clone() for d in dst]
+    src_idx, dst_idx = (torch.randperm(pages, generator=gen, device=DEV)[:items] for _ in range(2))
+    for at in (0, items - 1):
+        for which in (0, 1):
+            for value, text in ((pages, "out of range"), (-2, "must be -1 or non-negative")):
+                idx = [src_idx.clone(), dst_idx.clone()]
+                idx[which][at] = value
+                with pytest.raises(ValueError, match=text):
+                    call(src[0], dst[0], src[1], dst[1], *idx)
+    for d, b in zip(dst, before):
+        assert torch.equal(d, b)
+    if items > 4:
+        src_idx[3], dst_idx[2] = -1, -1       # skipped pairs
+        dst_idx[1] = dst_idx[items - 1]       # the later pair wins
+    call(src[0], dst[0], src[1], dst[1], src_idx, dst_idx)
+    moved = [(int(s), int(d)) for s, d in zip(src_idx, dst_idx) if s >= 0 and d >= 0]
+    from_to = dict((d, s) for s, d in moved)
+    s_i = torch.tensor([from_to[d] for d in from_to], device=DEV)
+    d_i = torch.tensor(list(from_to), device=DEV)
+    only = slice(0, 1) if name.startswith("per_layer") else slice(None)
+    for s, d, b in zip(src, dst, before):
+        s_lf = s if shapes[name][0] is lf else s.transpose(0, 1)
+        want = b.clone()
+        want_lf = want if shapes[name][1] is lf else want.transpose(0, 1)
+        want_lf[only, d_i] = s_lf[only, s_i]
+        assert torch.equal(d, want)
