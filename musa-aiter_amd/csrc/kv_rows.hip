@@ -358,57 +358,6 @@ __global__ __launch_bounds__(kBlockThreads) void pair_row_kernel(const PairRowAr
 
 __global__ __launch_bounds__(kBlockThreads) void claim_kernel(const int64_t* idx, int64_t idx_stride,
                                                               const BlockTableSlots bt, const int64_t* src_idx,
-// ----- rows of whole KiB named by a pair of index vectors: one wave per KiB --------------
-// HiCache items (a 2 KiB K or V row of 8 heads x 128): wave w moves one KiB of
-// row src_idx[u] to row dst_idx[u] of one plane, both offsets resolved with
-// scalar loads, no LDS and no barrier, as slot_row_kernel does for one index
-// vector.  INNER walks planes inside rows (one grid, see launch_row_copy),
-// otherwise grid y is the plane.  Bound by HBM (random 2 KiB reads): the
-// 4,096-item, 32-layer backup (1.07 GB) 192 us (5.6 TB/s), 209 us with the
-// block-resolving kernel, whose 8 KiB workgroups wait for an LDS round trip;
-// two KiB per wave 212 us, non-temporal stores 198 us.  XCD: each XCD takes a
-// contiguous eighth of a large grid (195 -> 192 us; 390 against 397 us for a
-// call of 8,192 items; 1 % slower for 500 items, which keep the natural order).
-struct PairRowArgs {
-  const int64_t* src_idx;
-  const int64_t* dst_idx;
-  const uint64_t* owner;
-  int64_t num_tokens;
-  int64_t src_rows;
-  int64_t dst_rows;
-  int64_t src_stride;
-  int64_t dst_stride;
-  uint32_t epoch;
-  uint32_t num_planes;
-  uint32_t row_kib;      // KiB per row
-  CallCheck check;
-  uint64_t src_planes[kMaxPlanes];
-  uint64_t dst_planes[kMaxPlanes];
-};
-
-template <bool INNER, int STP, bool XCD = false>
-__global__ __launch_bounds__(kBlockThreads) void pair_row_kernel(const PairRowArgs a) {
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const WgXyz wg = xcd_contiguous_wg<XCD>();
-  const uint32_t w = wg.x * kWavesPerBlock + wave;
-  const uint32_t per_row = INNER ? a.num_planes * a.row_kib : a.row_kib;
-  const uint32_t u = w / per_row;
-  if (u >= a.num_tokens) return;
-  const uint32_t rem = w - u * per_row;
-  const uint32_t plane = INNER ? rem / a.row_kib : wg.y;
-  const int64_t part = static_cast<int64_t>(INNER ? rem - plane * a.row_kib : rem) << 10;
-  const int64_t srow = a.src_idx[u], drow = a.dst_idx[u];
-  const uint64_t sbase = a.src_planes[plane], dbase = a.dst_planes[plane];
-  if (refused_ahead(a.check)) return;
-  if (srow < 0 || srow >= a.src_rows || drow < 0 || drow >= a.dst_rows) return;
-  const buf_t sb = make_buf(reinterpret_cast<const uint8_t*>(sbase) + srow * a.src_stride + part);
-  const buf_t db = make_buf(reinterpret_cast<uint8_t*>(dbase) + drow * a.dst_stride + part);
-  const uint32_t off = static_cast<uint32_t>(lane_id()) * 16u;
-  const u32x4 v = buf_ld16(sb, off);  // in flight while the claim is read
-  if (a.owner != nullptr && a.owner[drow] != claim_tag(a.epoch, u)) return;
-  buf_st16_p<STP>(db, off, v);
-}
-
                                                               int64_t src_rows, int64_t n, int64_t rows,
                                                               uint64_t* owner, uint32_t epoch, int reset) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -852,51 +801,6 @@ hipError_t launch_row_copy(const RowCopyParams& p, hipStream_t stream) {
       case 8: err = launch_rows_vec<8>(a, n, stream); break;
       case 4: err = launch_rows_vec<4>(a, n, stream); break;
       case 2: err = launch_rows_vec<2>(a, n, stream); break;
-  // Rows of whole KiB named by two packed index vectors: the per-KiB pair kernel.
-  if (vec == 16 && p.row_bytes % 1024 == 0 && p.src_idx != nullptr && p.dst_idx != nullptr && src_host && dst_host &&
-      p.src_indptr == nullptr && p.src_page_rows == 0 && p.dst_page_rows == 0 && p.idx_stride <= 1 && (inner || !dst_major(p))) {
-    const int64_t kib = p.row_bytes / 1024;
-    const int64_t planes = p.num_planes < kMaxPlanes ? p.num_planes : kMaxPlanes;
-    const int64_t waves = p.num_tokens * kib * (inner ? planes : 1);
-    if (waves <= 0x7FFFFFFF) {
-      for (int64_t base = 0; base < p.num_planes; base += kMaxPlanes) {
-        const int64_t n = (p.num_planes - base) < kMaxPlanes ? (p.num_planes - base) : kMaxPlanes;
-        PairRowArgs a{};
-        bool lines = p.dst_stride % 128 == 0;
-        for (int64_t i = 0; i < n; ++i) {
-          a.src_planes[i] = p.src_planes[base + i];
-          a.dst_planes[i] = p.dst_planes[base + i];
-          lines = lines && a.dst_planes[i] % 128 == 0;
-        }
-        a.src_idx = p.src_idx;
-        a.dst_idx = p.dst_idx;
-        a.owner = p.owner;
-        a.num_tokens = p.num_tokens;
-        a.src_rows = p.src_rows;
-        a.dst_rows = p.dst_rows;
-        a.src_stride = p.src_stride;
-        a.dst_stride = p.dst_stride;
-        a.epoch = p.epoch;
-        a.num_planes = static_cast<uint32_t>(n);
-        a.row_kib = static_cast<uint32_t>(kib);
-        a.check = p.check;
-        const int64_t all = p.num_tokens * kib * (inner ? n : 1);
-        const dim3 grid(static_cast<uint32_t>((all + kWavesPerBlock - 1) / kWavesPerBlock),
-                        inner ? 1u : static_cast<uint32_t>(n));
-        constexpr uint32_t kXcdGroups = 32768;  // workgroups from which a plane-inner grid takes the XCD order
-        if (inner && lines && grid.x >= kXcdGroups)
-          hipLaunchKernelGGL((pair_row_kernel<true, kBufWT, true>), grid, dim3(kBlockThreads), 0, stream, a);
-        else if (inner && lines) hipLaunchKernelGGL((pair_row_kernel<true, kBufWT>), grid, dim3(kBlockThreads), 0, stream, a);
-        else if (inner) hipLaunchKernelGGL((pair_row_kernel<true, kBufNT>), grid, dim3(kBlockThreads), 0, stream, a);
-        else if (lines) hipLaunchKernelGGL((pair_row_kernel<false, kBufWT>), grid, dim3(kBlockThreads), 0, stream, a);
-        else hipLaunchKernelGGL((pair_row_kernel<false, kBufNT>), grid, dim3(kBlockThreads), 0, stream, a);
-        const hipError_t err = hipGetLastError();
-        if (err != hipSuccess) return err;
-      }
-      return hipSuccess;
-    }
-  }
-
       default: err = launch_rows_vec<1>(a, n, stream); break;
     }
     if (err != hipSuccess) return err;
