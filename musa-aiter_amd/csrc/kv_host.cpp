@@ -11,12 +11,14 @@
 // For host <-> device copy batches, int64_column reads the caller's lists of
 // offsets and sizes (thousands of ints) into int64 columns and object_index
 // numbers the few distinct tensors its entries name.
+#include <torch/csrc/Dtype.h>
 #include <torch/extension.h>
 
 #include <cstdint>
 #include <unordered_map>
 #include <vector>
 
+#include "kv_host_calls.h"
 #include "musa_aiter_kv_hip.h"
 
 namespace py = pybind11;
@@ -218,6 +220,125 @@ int64_t two_x_nl_rows(const py::handle& kvcaches, const py::handle& memory_obj, 
   return reinterpret_cast<Entry>(entry)(&call, reinterpret_cast<void*>(stream));
 }
 
+// ----- one checked paged call --------------------------------------------------------------
+// kv_paged_to_linear / kv_linear_to_paged, their _multi_layer and FP8 forms:
+// the argument checks of the Python layer and the packed call in one pass.
+// Takes the common arguments as they are (plain contiguous tensors on the
+// current device, int64 slots, float32 scales of one mode) and returns
+// kNotTaken, with nothing launched, for everything else: the Python layer then
+// runs the reference's checks in their order, which convert or raise.  A
+// decode step's 64-token scatter spent 11.5 us of its 19.8 us in those checks.
+constexpr int64_t kNotTaken = -2;
+
+bool plain_tensor(const py::handle& h) { return THPVariable_CheckExact(h.ptr()); }
+
+bool float_kind(at::ScalarType t) { return t == at::kFloat || t == at::kHalf || t == at::kBFloat16; }
+
+// Scale mode of a plain float32 scale: 0 scalar, 1 [heads], 2 [layers, heads]; -1 anything else.
+int scale_mode_of(const py::handle& h, int64_t layers, int64_t heads, bool layered, const at::Device& device) {
+  if (!plain_tensor(h)) return -1;
+  const at::Tensor& s = THPVariable_Unpack(h.ptr());
+  if (s.scalar_type() != at::kFloat || s.device() != device || !s.is_contiguous()) return -1;
+  if (s.numel() == 1) return 0;
+  if (s.dim() == 1 && s.size(0) == heads) return 1;
+  if (layered && s.dim() == 2 && s.size(0) == layers && s.size(1) == heads) return 2;
+  return -1;
+}
+
+// `linear_k` / `linear_v`: the rows of a scatter; None for a gather, which allocates them (of `out_dtype`, or
+// the caches' type when that is None).  codec: 0 copy, 1 FP8 E4M3, 2 FP8 E5M2.  `claims`: the caller's
+// musa_aiter_hip_claims (scatters), its epoch already advanced.  Returns (status, k rows, v rows).
+py::tuple paged_call(const py::handle& key_cache, const py::handle& value_cache, const py::handle& linear_k,
+                     const py::handle& linear_v, const py::handle& slot_mapping, const py::handle& k_scale,
+                     const py::handle& v_scale, bool scatter, bool layered, int codec, const py::handle& out_dtype,
+                     uint64_t entry, uint64_t claims, uint64_t report, uint64_t guard, int64_t report_words,
+                     int64_t stamp, uint64_t stream, int64_t device) {
+  const auto no = [] { return py::make_tuple(kNotTaken, py::none(), py::none()); };
+  if (!plain_tensor(key_cache) || !plain_tensor(value_cache) || !plain_tensor(slot_mapping)) return no();
+  const at::Tensor& kc = THPVariable_Unpack(key_cache.ptr());
+  const at::Tensor& vc = THPVariable_Unpack(value_cache.ptr());
+  const at::Tensor& slots = THPVariable_Unpack(slot_mapping.ptr());
+  const int64_t lead = layered ? 1 : 0;
+  if (!kc.is_cuda() || kc.device().index() != device || vc.device() != kc.device() || slots.device() != kc.device())
+    return no();
+  if (kc.dim() != 4 + lead || vc.sizes() != kc.sizes() || !kc.is_contiguous() || !vc.is_contiguous() ||
+      kc.numel() == 0 || slots.dim() != 1 || slots.scalar_type() != at::kLong || !slots.is_contiguous() ||
+      slots.size(0) == 0)
+    return no();
+  const int64_t layers = layered ? kc.size(0) : 1;
+  const int64_t blocks = kc.size(lead), heads = kc.size(lead + 1), dim = kc.size(lead + 2), page = kc.size(lead + 3);
+  const int64_t tokens = slots.size(0), row = heads * dim;
+  const auto fp8_kind = [](at::ScalarType t) {
+    return t == at::kByte || t == at::kFloat8_e4m3fn || t == at::kFloat8_e5m2;
+  };
+  if (codec == 0 ? !float_kind(kc.scalar_type()) || vc.scalar_type() != kc.scalar_type()
+                 : !fp8_kind(kc.scalar_type()) || !fp8_kind(vc.scalar_type()))
+    return no();
+  musa_aiter_hip_paged_tiles_call call{};
+  if (codec != 0) {
+    const int mk = scale_mode_of(k_scale, layers, heads, layered, kc.device());
+    if (mk < 0 || scale_mode_of(v_scale, layers, heads, layered, kc.device()) != mk) return no();
+    call.scale_mode = mk;
+    call.k_scale = static_cast<const float*>(THPVariable_Unpack(k_scale.ptr()).data_ptr());
+    call.v_scale = static_cast<const float*>(THPVariable_Unpack(v_scale.ptr()).data_ptr());
+  }
+  const int64_t want_sizes[4] = {layers, tokens, heads, dim};
+  const at::IntArrayRef want(want_sizes + 1 - lead, 3 + lead);
+  at::Tensor lk, lv;
+  if (scatter) {
+    if (!plain_tensor(linear_k) || !plain_tensor(linear_v)) return no();
+    lk = THPVariable_Unpack(linear_k.ptr());
+    lv = THPVariable_Unpack(linear_v.ptr());
+    if (lk.sizes() != want || lv.sizes() != want || lk.device() != kc.device() || lv.device() != kc.device() ||
+        !lk.is_contiguous() || !lv.is_contiguous() || lv.scalar_type() != lk.scalar_type() ||
+        (codec == 0 ? lk.scalar_type() != kc.scalar_type() : !float_kind(lk.scalar_type())))
+      return no();
+    const auto* c = reinterpret_cast<const musa_aiter_hip_claims*>(claims);
+    if (c == nullptr || c->tags == nullptr || c->epoch == 0 || c->capacity < blocks * page) return no();
+    call.claims = c;
+  } else {
+    at::ScalarType dt = kc.scalar_type();
+    if (!out_dtype.is_none()) {
+      if (!THPDtype_Check(out_dtype.ptr())) return no();
+      dt = reinterpret_cast<THPDtype*>(out_dtype.ptr())->scalar_type;
+    }
+    if (!float_kind(dt)) return no();
+    lk = at::empty(want, kc.options().dtype(dt));
+    lv = at::empty(want, kc.options().dtype(dt));
+  }
+  call.scatter = call.dedupe = scatter ? 1 : 0;
+  call.codec = codec;
+  call.cache_elt = static_cast<int32_t>(kc.element_size());
+  call.lin_elt = static_cast<int32_t>(lk.element_size());
+  call.lin_dtype = lk.scalar_type() == at::kFloat ? 0 : lk.scalar_type() == at::kHalf ? 1 : 2;
+  call.fill_zeros = scatter ? 0 : 1;
+  call.key_cache = kc.data_ptr();
+  call.value_cache = vc.data_ptr();
+  call.key_linear = lk.data_ptr();
+  call.value_linear = lv.data_ptr();
+  call.slot_mapping = static_cast<const int64_t*>(slots.data_ptr());
+  call.num_layers = layers;
+  call.num_tokens = tokens;
+  call.num_blocks = blocks;
+  call.num_heads = heads;
+  call.head_dim = dim;
+  call.block_size = page;
+  call.lin_token_stride = row;
+  call.lin_layer_stride = row * tokens;
+  call.report = reinterpret_cast<int64_t*>(report);
+  call.guard = reinterpret_cast<int64_t*>(guard);
+  call.report_words = report_words;
+  call.stamp = stamp;
+  const auto fn = reinterpret_cast<decltype(&musa_aiter_hip_paged_tiles_checked)>(entry);
+  int64_t status;
+  {
+    py::gil_scoped_release unlocked;  // the entry waits for the device's verdict
+    status = fn(&call, reinterpret_cast<void*>(stream));
+  }
+  if (scatter || status != 0) return py::make_tuple(status, py::none(), py::none());
+  return py::make_tuple(status, lk, lv);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_kv_host, m) {
@@ -227,6 +348,8 @@ PYBIND11_MODULE(_kv_host, m) {
   m.def("int64_column", &int64_column, py::arg("items"));
   m.def("object_index", &object_index, py::arg("first"), py::arg("second"));
   m.def("two_x_nl_rows", &two_x_nl_rows);
+  m.def("paged_call", &paged_call);
+  m.attr("NOT_TAKEN") = kNotTaken;
   m.attr("OK") = static_cast<int>(kOk);
   m.attr("SHAPE") = static_cast<int>(kShape);
   m.attr("DTYPE") = static_cast<int>(kDtype);

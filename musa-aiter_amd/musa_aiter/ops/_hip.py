@@ -378,6 +378,48 @@ def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, l
     return True
 
 
+_paged_entry: list[int] = []  # address of musa_aiter_hip_paged_tiles_checked
+
+
+def paged_native(key_cache, value_cache, linear, slots, scales, *, layered: bool, codec: int, out_dtype=None):
+    """One checked paged call whose argument checks the host module makes too: a scatter of the rows ``linear``,
+    or with ``linear`` None a gather into new tensors (of ``out_dtype``, or the caches' type).
+
+    Returns None, with nothing launched, when the arguments are not all ones the module takes as they are
+    (see paged_call in kv_host.cpp) or the device refused a value; the caller then runs its own checks.
+    Otherwise returns the gathered (k, v) rows, or True for a scatter."""
+    if type(key_cache) is not torch.Tensor or not key_cache.is_cuda or torch._C._cuda_isCurrentStreamCapturing():
+        return None
+    index = torch._C._cuda_getDevice()
+    stream = torch._C._cuda_getCurrentRawStream(index)
+    checks = _check_sets.get((index, stream))
+    if checks is None:
+        return None  # the stream's first call makes its set
+    h = host()
+    if not _paged_entry:
+        _paged_entry.append(ctypes.cast(fn("musa_aiter_hip_paged_tiles_checked"), ctypes.c_void_p).value)
+    scatter = linear is not None
+    lin_k, lin_v = linear if scatter else (None, None)
+    k_scale, v_scale = scales if scales is not None else (None, None)
+    with checks.lock:
+        claims, entry = 0, None
+        if scatter:
+            entry = _claim_sets.get((index, stream))
+            if entry is None or entry[1].epoch == _EPOCH_LAST:
+                return None
+            entry[1].epoch += 1
+            claims = ctypes.addressof(entry[1])
+        checks.stamp += 1
+        rc, k, v = h.paged_call(key_cache, value_cache, lin_k, lin_v, slots, k_scale, v_scale, scatter, layered, codec,
+                                out_dtype, _paged_entry[0], claims, checks.report_ptr, checks.guard_ptr,
+                                _SLOT_CHECK_WORDS, checks.stamp, stream, index)
+        del entry
+    if rc == h.NOT_TAKEN or rc == _REFUSED:
+        return None
+    check(rc, "paged call")
+    return True if scatter else (k, v)
+
+
 # musa_aiter_hip_copy_rows_paged_call: plane lists, planes, two index pointers, eleven int64 sizes,
 # strides and the lowest index, claims, report and guard addresses, report words and stamp.
 _COPY_ROWS_PAGED_CALL = struct.Struct("<2Qq2Q11q3Q2q")

@@ -356,6 +356,11 @@ def kv_paged_to_linear(
     ``_kv_paged_to_linear_compute`` (:3047-3089).
     """
     op = "kv_paged_to_linear"
+    if out_k is None and out_v is None and fill_skipped == "zeros":
+        got = _hip.paged_native(key_cache, value_cache, None, slot_mapping, None, layered=False, codec=_CODEC_COPY)
+        if got is not None:
+            _emit(op, key_cache, "gfx950 paged->linear tile gather")
+            return got
     nb, nh, hd, bs = _validate_paged_shapes(key_cache, value_cache, name=op)
     tcount = slot_mapping.numel()
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
@@ -386,6 +391,11 @@ def kv_paged_to_linear_multi_layer(
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """Gather stacked caches ``[L, NB, H, D, BS]`` into ``[L, T, H, D]`` in one launch (reference :3209-3309)."""
     op = "kv_paged_to_linear_multi_layer"
+    if out_k is None and out_v is None and fill_skipped == "zeros":
+        got = _hip.paged_native(key_cache, value_cache, None, slot_mapping, None, layered=True, codec=_CODEC_COPY)
+        if got is not None:
+            _emit(op, key_cache, f"gfx950 paged->linear tile gather ({key_cache.shape[0]} layers, one launch)")
+            return got
     nl, nb, nh, hd, bs = _validate_stacked_paged_shapes(key_cache, value_cache, name=op)
     tcount = slot_mapping.numel()
     slots = _ensure_slotmapping_vector(slot_mapping, expected_len=tcount, name=op)
@@ -427,6 +437,10 @@ def kv_linear_to_paged(
     token in token order.
     """
     op = "kv_linear_to_paged"
+    if _hip.paged_native(key_cache, value_cache, (key_linear, value_linear), slot_mapping, None, layered=False,
+                         codec=_CODEC_COPY):
+        _emit(op, key_linear, "gfx950 linear->paged tile scatter")
+        return
     if key_linear.shape != value_linear.shape or key_linear.dim() != 3:
         raise ValueError("kv_linear_to_paged: key_linear/value_linear must be 3-D and match shapes")
     tcount = key_linear.shape[0]
@@ -457,6 +471,10 @@ def kv_linear_to_paged_multi_layer(
 ) -> None:
     """Scatter ``[L, T, H, D]`` into stacked caches in one launch (reference :3382-3457)."""
     op = "kv_linear_to_paged_multi_layer"
+    if _hip.paged_native(key_cache, value_cache, (key_linear, value_linear), slot_mapping, None, layered=True,
+                         codec=_CODEC_COPY):
+        _emit(op, key_linear, f"gfx950 linear->paged tile scatter ({key_cache.shape[0]} layers, one launch)")
+        return
     if key_linear.shape != value_linear.shape or key_linear.dim() != 4:
         raise ValueError(
             "kv_linear_to_paged_multi_layer: key_linear/value_linear must be 4-D "
@@ -629,6 +647,10 @@ def _fp8_format_params(fp8_format: str) -> tuple[int, int, int, int]:
     return 5, 2, 15, 16
 
 
+# Formats the native path takes by their plain names.
+_NATIVE_FORMATS = {"e4m3": _CODEC_E4M3, "e5m2": _CODEC_E5M2}
+
+
 def _codec(fp8_format: str) -> int:
     return _CODEC_E4M3 if _normalize_fp8_format(fp8_format) == "e4m3" else _CODEC_E5M2
 
@@ -752,6 +774,11 @@ def kv_linear_to_paged_fp8(
     normal, round half to even); scales are scalar or per kv-head.
     """
     op = "kv_linear_to_paged_fp8"
+    codec = _NATIVE_FORMATS.get(fp8_format)
+    if codec is not None and _hip.paged_native(key_cache_fp8, value_cache_fp8, (key_linear, value_linear),
+                                               slot_mapping, (k_scale, v_scale), layered=False, codec=codec):
+        _emit(op, key_linear, f"gfx950 fused {fp8_format.upper()} quantize scatter")
+        return
     fp8_format = _normalize_fp8_format(fp8_format)
     _validate_fp8_cache_tensor(key_cache_fp8, name="kv_linear_to_paged_fp8 key_cache_fp8")
     _validate_fp8_cache_tensor(value_cache_fp8, name="kv_linear_to_paged_fp8 value_cache_fp8")
@@ -790,6 +817,13 @@ def kv_paged_fp8_to_linear(
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """Gather FP8 cache slots, decode ``code * scale`` in fp32 and round to ``out_dtype`` (reference :2250-2301)."""
     op = "kv_paged_fp8_to_linear"
+    codec = _NATIVE_FORMATS.get(fp8_format)
+    if codec is not None and out_k is None and out_v is None:
+        got = _hip.paged_native(key_cache_fp8, value_cache_fp8, None, slot_mapping, (k_scale, v_scale),
+                                layered=False, codec=codec, out_dtype=out_dtype)
+        if got is not None:
+            _emit(op, key_cache_fp8, f"gfx950 fused {fp8_format.upper()} dequantize gather")
+            return got
     fp8_format = _normalize_fp8_format(fp8_format)
     _validate_fp8_cache_tensor(key_cache_fp8, name="kv_paged_fp8_to_linear key_cache_fp8")
     _validate_fp8_cache_tensor(value_cache_fp8, name="kv_paged_fp8_to_linear value_cache_fp8")
@@ -827,6 +861,11 @@ def kv_linear_to_paged_fp8_multi_layer(
 ) -> None:
     """Multi-layer FP8 quantize scatter; scales scalar, ``[H]`` or ``[L, H]`` (reference :2304-2347)."""
     op = "kv_linear_to_paged_fp8_multi_layer"
+    codec = _NATIVE_FORMATS.get(fp8_format)
+    if codec is not None and _hip.paged_native(key_cache_fp8, value_cache_fp8, (key_linear, value_linear),
+                                               slot_mapping, (k_scale, v_scale), layered=True, codec=codec):
+        _emit(op, key_linear, f"gfx950 fused {fp8_format.upper()} quantize scatter ({key_cache_fp8.shape[0]} layers)")
+        return
     fp8_format = _normalize_fp8_format(fp8_format)
     _validate_fp8_cache_tensor(key_cache_fp8, name="kv_linear_to_paged_fp8_multi_layer key_cache_fp8")
     _validate_fp8_cache_tensor(value_cache_fp8, name="kv_linear_to_paged_fp8_multi_layer value_cache_fp8")
@@ -868,6 +907,13 @@ def kv_paged_fp8_to_linear_multi_layer(
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """Multi-layer FP8 dequantize gather into ``[L, T, H, D]`` (reference :2350-2398)."""
     op = "kv_paged_fp8_to_linear_multi_layer"
+    codec = _NATIVE_FORMATS.get(fp8_format)
+    if codec is not None and out_k is None and out_v is None:
+        got = _hip.paged_native(key_cache_fp8, value_cache_fp8, None, slot_mapping, (k_scale, v_scale),
+                                layered=True, codec=codec, out_dtype=out_dtype)
+        if got is not None:
+            _emit(op, key_cache_fp8, f"gfx950 fused {fp8_format.upper()} dequantize gather ({key_cache_fp8.shape[0]} layers)")
+            return got
     fp8_format = _normalize_fp8_format(fp8_format)
     _validate_fp8_cache_tensor(key_cache_fp8, name="kv_paged_fp8_to_linear_multi_layer key_cache_fp8")
     _validate_fp8_cache_tensor(value_cache_fp8, name="kv_paged_fp8_to_linear_multi_layer value_cache_fp8")

@@ -213,3 +213,107 @@ def test_hicache_page_indices_are_checked_on_the_device(row, items, name):
         want_lf = want if shapes[name][1] is lf else want.transpose(0, 1)
         want_lf[only, d_i] = s_lf[only, s_i]
         assert torch.equal(d, want)
+
+
+@pytest.mark.parametrize("layers", [1, 3])
+def test_native_argument_checks_agree_with_the_python_layer(layers, monkeypatch):
+    """Every form of arguments gives one result and one error whether the host module takes the call or the
+    Python layer does: other dtypes, strides, shapes, scale kinds and devices among them."""
+    from musa_aiter.ops import _hip
+
+    bs, tokens = 16, 40
+    nb, slots, caches, linear = _setup(bs, tokens, layers)
+    _, _, codes, _ = _setup(bs, tokens, layers, torch.uint8)
+    head = torch.full((NH,), 0.5, device=DEV)
+    strided = torch.stack(linear, -1)
+    wide = [torch.cat([c, c], -1)[..., :bs] for c in caches]
+    per_layer = torch.full((layers, NH), 0.5, device=DEV)
+    empty = [x[..., :0, :, :] for x in linear]
+
+    def store(k, v, kc, vc, s):
+        got = [kc.clone(memory_format=torch.preserve_format), vc.clone(memory_format=torch.preserve_format)]
+        _names("kv_linear_to_paged", layers)(k, v, *got, s)
+        return got
+
+    def quant(k, v, s, ks, vs, kc=codes[0], vc=codes[1], **kw):
+        got = [kc.clone(), vc.clone()]
+        _names("kv_linear_to_paged_fp8", layers)(k, v, *got, s, ks, vs, **kw)
+        return [g.view(torch.uint8) for g in got]
+
+    load = _names("kv_paged_to_linear", layers)
+    dequant = _names("kv_paged_fp8_to_linear", layers)
+    calls = [
+        lambda: store(*linear, *caches, slots),
+        lambda: store(*linear, *caches, slots.to(torch.int32)),
+        lambda: store(*linear, *caches, slots.repeat_interleave(2)[::2]),
+        lambda: store(*linear, *caches, slots.cpu()),
+        lambda: store(*linear, *caches, slots[:-1]),
+        lambda: store(*linear, *caches, slots.view(1, -1)),
+        lambda: store(*linear, *caches, slots.float()),
+        lambda: store(*(x.float() for x in linear), *caches, slots),
+        lambda: store(linear[0], linear[1].float(), *caches, slots),
+        lambda: store(strided[..., 0], strided[..., 1], *caches, slots),
+        lambda: store(*linear, *wide, slots),
+        lambda: store(*linear, caches[0], caches[1].half(), slots),
+        lambda: store(*linear, caches[0], caches[1][..., :-1], slots),
+        lambda: store(*(x[..., :-1] for x in linear), *caches, slots),
+        lambda: store(*(x.double() for x in linear), *(c.double() for c in caches), slots),
+        lambda: store(*empty, *caches, slots[:0]),
+        lambda: load(*caches, slots),
+        lambda: load(*wide, slots),
+        lambda: load(*caches, slots[:0]),
+        lambda: load(caches[0], caches[1].half(), slots),
+        lambda: load(*(c.cpu() for c in caches), slots.cpu()),
+        lambda: load(*caches, slots, fill_skipped="preserve"),
+        lambda: load(*caches, torch.where(slots % 3 == 0, -1, slots)),
+        lambda: quant(*linear, slots, head, head),
+        lambda: quant(*linear, slots, 0.5, head),
+        lambda: quant(*linear, slots, head[:1], 0.25),
+        lambda: quant(*linear, slots, head.double(), head.cpu()),
+        lambda: quant(*linear, slots, head.repeat(2)[::2], head),
+        lambda: quant(*linear, slots, per_layer, head),
+        lambda: quant(*linear, slots, per_layer, per_layer),
+        lambda: quant(*linear, slots, head[:0], head),
+        lambda: quant(*linear, slots, head, head, fp8_format="FP8_E5M2"),
+        lambda: quant(*linear, slots, head, head, fp8_format="e5m2"),
+        lambda: quant(*linear, slots, head, head, fp8_format="e3m4"),
+        lambda: quant(*linear, slots, head, head, codes[0].view(torch.float8_e4m3fn), codes[1].view(torch.float8_e5m2)),
+        lambda: quant(*linear, slots, head, head, codes[0].view(torch.int8), codes[1]),
+        lambda: quant(*(x.double() for x in linear), slots, head, head),
+        lambda: quant(linear[0], linear[1].float(), slots, head, head),
+        lambda: quant(*empty, slots[:0], head, -head),
+        lambda: dequant(*codes, slots, head, head),
+        lambda: dequant(*codes, slots, per_layer, per_layer, out_dtype=torch.float32),
+        lambda: dequant(*codes, slots, head, 0.5, out_dtype=torch.float64),
+        lambda: dequant(*codes, slots, head, head, out_dtype=torch.float16, fp8_format="E4M3FN"),
+        lambda: dequant(*codes, slots[:0], head, head),
+        lambda: dequant(*codes, slots.to(torch.int16), head, head),
+    ]
+
+    def outcome(call):
+        try:
+            return [t.cpu() for t in call()]
+        except Exception as e:
+            return type(e), str(e)
+
+    native = []
+    real = _hip.paged_native
+    monkeypatch.setattr(_hip, "paged_native", lambda *a, **k: (native.append(real(*a, **k)), native[-1])[1])
+    outcome(calls[0]), outcome(calls[16])  # the stream's check and claim sets exist from here on
+    first = []
+    for call in calls:
+        native.clear()
+        first.append((outcome(call), bool(native) and native[-1] is not None))
+    monkeypatch.setattr(_hip, "paged_native", lambda *a, **k: None)
+    taken = 0
+    for k, (call, (got, was_native)) in enumerate(zip(calls, first)):
+        want = outcome(call)
+        taken += was_native
+        assert type(got) is type(want), (k, got, want)
+        if isinstance(got, tuple):
+            assert got == want, k
+            assert not was_native, k
+        else:
+            assert all(a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride() and
+                       torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(got, want)), k
+    assert taken >= 8  # the plain forms do take the native path
