@@ -270,6 +270,20 @@ __global__ __launch_bounds__(kBlockThreads) void cg_encode_kernel(CgEncodeArgs a
   constexpr int kEps = 16 / CgIn<IN>::kBytes;
   __shared__ uint32_t hist[kWavesPerBlock][256 * kCgHistCopies];
   const int nb = a.num_bins;
+  // The first chunk is loaded ahead of the range fold, which waits for the
+  // pairs, a workgroup reduction and the histogram's clearing: on small inputs
+  // (one or two chunks per workgroup) those waits and the load's own overlap:
+  // the whole call on 16.8 M bf16 values 25.5 -> 24.3 us.
+  constexpr int V = kCgEncodeVecs;
+  const int64_t slots = a.n / kEps;
+  const int64_t per_chunk = int64_t{kBlockThreads} * V;
+  const int64_t lane_off = int64_t{wave_in_block()} * kWave * V + lane_id();
+  auto load = [&](int64_t c, u32x4* v) {
+    for_chunk<V>(c, per_chunk, lane_off, slots, [&](int k, int64_t s) { v[k] = ld16(a.x + s * 16); });
+  };
+  [[maybe_unused]] u32x4 cur[V], nxt[V];
+  int64_t c = blockIdx.x;
+  if (VEC && c * per_chunk < slots) load(c, cur);
   float mn = a.min_arg, scale = a.scale_arg;
   if constexpr (HIST) {
     MinMax m;
@@ -302,7 +316,6 @@ __global__ __launch_bounds__(kBlockThreads) void cg_encode_kernel(CgEncodeArgs a
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlockThreads;
   int64_t first_scalar = 0;
   if constexpr (VEC) {
-    const int64_t slots = a.n / kEps;
     auto emit = [&](int64_t s, const u32x4& v) {
       uint32_t b[kEps];
       bool same = true;
@@ -332,15 +345,6 @@ __global__ __launch_bounds__(kBlockThreads) void cg_encode_kernel(CgEncodeArgs a
     };
     // Software-pipelined: the next chunk's vectors are loaded before this chunk's bins are
     // computed and stored, so each wave keeps 2 * V vectors in flight.
-    constexpr int V = kCgEncodeVecs;
-    const int64_t per_chunk = int64_t{kBlockThreads} * V;
-    const int64_t lane_off = int64_t{wave_in_block()} * kWave * V + lane_id();
-    auto load = [&](int64_t c, u32x4* v) {
-      for_chunk<V>(c, per_chunk, lane_off, slots, [&](int k, int64_t s) { v[k] = ld16(a.x + s * 16); });
-    };
-    u32x4 cur[V], nxt[V];
-    int64_t c = blockIdx.x;
-    if (c * per_chunk < slots) load(c, cur);
     for (; c * per_chunk < slots; c += gridDim.x) {
       const int64_t cn = c + gridDim.x;
       if (cn * per_chunk < slots) load(cn, nxt);
