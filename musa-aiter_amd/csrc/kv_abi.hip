@@ -446,6 +446,20 @@ int paged_tiles_checked(const musa_aiter_hip_paged_tiles_call& c, hipStream_t st
     p.scan_dupes = 0;
     p.check.report = nullptr;
   }
+  if (!c.scatter && c.discard && c.codec == kvhip::kCopy) {
+    // Nobody sees what a refused gather wrote: its own launch checks it, with none ahead of it.
+    const int64_t shares = (c.num_tokens + kvhip::kCheckSlice - 1) / kvhip::kCheckSlice;
+    p.check.report = c.report;
+    p.check.words = shares < c.report_words ? shares : c.report_words;
+    err = kvhip::launch_paged_tiles(p, stream);
+    if (err == hipSuccess) {
+      err = await_verdict(c.report, p.check.words, c.stamp, stream, &refused);
+      return err != hipSuccess ? err : refused ? MUSA_AITER_HIP_REFUSED : 0;
+    }
+    if (err != hipErrorNotSupported) return err;
+    p.check.report = nullptr;
+    p.check.words = 0;
+  }
   kvhip::CheckSource src{};
   src.idx = c.slot_mapping;
   src.n = c.num_tokens;
@@ -467,7 +481,7 @@ int paged_tiles_checked(const musa_aiter_hip_paged_tiles_call& c, hipStream_t st
   }
   int64_t groups = (c.num_tokens + kCheckPerGroup - 1) / kCheckPerGroup;
   if (groups > c.report_words) groups = c.report_words;
-  kvhip::CallCheck check{c.report, c.guard, c.stamp};
+  kvhip::CallCheck check{c.report, c.guard, c.stamp, 0};
   err = kvhip::launch_check(src, check, groups, stream);
   if (err != hipSuccess) return err;
   p.check.guard = c.guard;
@@ -1481,9 +1495,9 @@ int musa_aiter_hip_copy_rows_paged_checked(const musa_aiter_hip_copy_rows_paged_
   }
   int64_t groups = (c.num_tokens + kCheckPerGroup - 1) / kCheckPerGroup;
   if (groups > c.report_words) groups = c.report_words;
-  hipError_t err = kvhip::launch_check(src, kvhip::CallCheck{c.report, c.guard, c.stamp}, groups, as_stream(stream));
+  hipError_t err = kvhip::launch_check(src, kvhip::CallCheck{c.report, c.guard, c.stamp, 0}, groups, as_stream(stream));
   if (err != hipSuccess) return err;
-  p.check = kvhip::CallCheck{nullptr, c.guard, c.stamp};
+  p.check = kvhip::CallCheck{nullptr, c.guard, c.stamp, 0};
   const hipError_t moved = kvhip::launch_row_copy(p, as_stream(stream));
   bool refused = false;
   err = await_verdict(c.report, groups, c.stamp, as_stream(stream), &refused);

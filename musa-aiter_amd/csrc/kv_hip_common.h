@@ -197,15 +197,20 @@ __device__ __forceinline__ uint64_t claim_tag(uint32_t epoch, int64_t token) {
 // moves anything, a slot past the cache or an FP8 scale that is not positive
 // and finite does not wait for the host to read the values first: either its
 // own kernel checks them (report set: every workgroup reads them all and
-// workgroup 0 reports), or a check kernel ahead of it on the stream does, and
-// the kernel behind it returns at once if the guard holds its stamp.  The host
-// reads the verdict while the kernel runs.
+// workgroup 0 reports; or, where a refused call's output is thrown away, extra
+// waves of the launch check a share each and report), or a check kernel ahead
+// of it on the stream does, and the kernel behind it returns at once if the
+// guard holds its stamp.  The host reads the verdict while the kernel runs.
 // ---------------------------------------------------------------------------
 struct CallCheck {
   int64_t* report;       // pinned host memory: verdict word(s), 2 * stamp + refused
   const int64_t* guard;  // device word: `stamp` when the call with that stamp is refused
   int64_t stamp;         // unique among the calls sharing the guard
+  int64_t words;         // report set: waves that check a share each, one report word per wave (0: workgroup 0 reports)
 };
+
+// Slots that a checking wave of a gather reads at a time: four per lane.
+constexpr int64_t kCheckSlice = 256;
 
 // True when a check kernel ahead of this one refused the call.
 __device__ __forceinline__ bool refused_ahead(const CallCheck& c) { return c.guard != nullptr && *c.guard == c.stamp; }

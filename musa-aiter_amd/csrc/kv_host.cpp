@@ -311,7 +311,7 @@ py::tuple paged_call(const py::handle& key_cache, const py::handle& value_cache,
   call.cache_elt = static_cast<int32_t>(kc.element_size());
   call.lin_elt = static_cast<int32_t>(lk.element_size());
   call.lin_dtype = lk.scalar_type() == at::kFloat ? 0 : lk.scalar_type() == at::kHalf ? 1 : 2;
-  call.fill_zeros = scatter ? 0 : 1;
+  call.fill_zeros = call.discard = scatter ? 0 : 1;  // a refused gather's new rows are dropped here
   call.key_cache = kc.data_ptr();
   call.value_cache = vc.data_ptr();
   call.key_linear = lk.data_ptr();

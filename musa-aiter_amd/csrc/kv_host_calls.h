@@ -22,6 +22,8 @@ extern "C" {
  * returns when the verdict is there, which does not wait for the copy. */
 typedef struct musa_aiter_hip_paged_tiles_call {
   int32_t scatter, codec, cache_elt, lin_elt, lin_dtype, scale_mode, fill_zeros, dedupe;
+  int32_t discard;  /* a gather whose rows the caller throws away if it is refused: they may be written then */
+  int32_t reserved;
   void *key_cache, *value_cache, *key_linear, *value_linear;
   const int64_t* slot_mapping;
   int64_t num_layers, num_tokens, num_blocks, num_heads, head_dim, block_size, lin_token_stride, lin_layer_stride;

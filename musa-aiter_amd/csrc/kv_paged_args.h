@@ -30,6 +30,7 @@ struct TileArgs {
   float inv_head_dim;          // 1 / head_dim, for small-integer division by head_dim
   BlockTableSlots bt;          // block_tables set: slots derived per dense token
   int32_t row_groups;          // tile kernel: row groups per block (grid x of a gather = tile * row_groups + group)
+  int32_t check_groups;        // gather: workgroups at the front of each plane for check_share (0: none)
   int32_t scan_dupes;          // scatter: resolve repeated slots with a ScanTable instead of claim tags
   CallCheck check;             // report set: this kernel checks the call's slots and scales; guard set: one ahead did
 };
@@ -109,7 +110,41 @@ __device__ __forceinline__ bool scales_refused(const TileArgs& a) {
 // Workgroup 0's verdict on a checked call, for the polling host.
 __device__ __forceinline__ void report_check(const CallCheck& c, bool refused) {
   if ((blockIdx.x | blockIdx.y | blockIdx.z | threadIdx.x) == 0)
-    __hip_atomic_store(c.report, 2 * c.stamp + (refused ? 1 : 0), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(c.report, 2 * c.stamp + (refused ? 1 : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A gather whose output is thrown away when the call is refused runs unguarded
+// (it skips the slots it cannot read anyway), so extra workgroups of its own
+// launch, ahead of plane 0's tiles, check the slots, kCheckSlice at a time, and
+// the call needs no check kernel ahead of it: one layer of 7,456 tokens (fp16,
+// 16-token pages) 17.2 -> 14.0 us a call, 16 layers of 9,001 tokens (64-token
+// pages) 213.8 -> 208.5.  (Behind plane 0's tiles they report so late that the
+// host's next call waits: 15.5 us; the first waves checking on their way to
+// their own tiles: 13.9 and 211.3 us.)  The word is all that a wave publishes,
+// so its store is relaxed: a release at system scope would write back the L2,
+// which holds the rows that other workgroups are storing.
+// FP8 gathers keep the check kernel: theirs took as much longer as it had taken
+// (6,007 tokens of 8 layers: 47.5 + 4.8 -> 51.6 us, the call 55 us both ways).
+// `group`: index among the extra workgroups of the plane.
+template <int NT>
+__device__ __forceinline__ void check_share(const TileArgs& a, uint32_t group, uint32_t plane) {
+  const int64_t word = static_cast<int64_t>(group) * (NT / kWave) + wave_in_block();
+  if (word >= a.check.words || plane != 0) return;
+  bool bad = false;
+  for (int64_t base = word * kCheckSlice; base < a.num_tokens; base += a.check.words * kCheckSlice) {
+    int64_t s[kCheckSlice / kWave];
+#pragma unroll
+    for (int k = 0; k < kCheckSlice / kWave; ++k) {
+      const int64_t j = base + k * kWave + lane_id();
+      s[k] = j < a.num_tokens ? a.slots[j] : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < kCheckSlice / kWave; ++k) bad |= s[k] >= a.num_slots;
+  }
+  const bool refused = ballot(bad) != 0;
+  if (lane_id() == 0)
+    __hip_atomic_store(a.check.report + word, 2 * a.check.stamp + (refused ? 1 : 0), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Checks a small call in the kernel that moves it (report set): every

@@ -267,7 +267,15 @@ void paged_tile_kernel(const TileArgs a) {
   // faster on random blocks than visiting each group of all tiles in turn).
   // Gathers over many planes give each XCD a contiguous eighth of the grid
   // (FEW false; chosen by the launcher).
-  const WgXyz wg = xcd_contiguous_wg<!SCATTER && !FEW>();
+  WgXyz wg = xcd_contiguous_wg<!SCATTER && !FEW>();
+  if constexpr (!SCATTER) {
+    const uint32_t ahead = static_cast<uint32_t>(a.check_groups);
+    if (wg.x < ahead) {
+      check_share<NT>(a, wg.x, wg.y);
+      return;
+    }
+    wg.x -= ahead;
+  }
   const int64_t tile_id = SCATTER ? static_cast<int64_t>(wg.x) : static_cast<int64_t>(wg.x) / a.row_groups;
   const int64_t group =
       SCATTER ? static_cast<int64_t>(wg.z) : static_cast<int64_t>(wg.x) - tile_id * a.row_groups;
@@ -290,7 +298,7 @@ void paged_tile_kernel(const TileArgs a) {
   if (t >= 0 && t < a.num_tokens) s = slot_at(a, t);
   if (refused_ahead(a.check)) return;
   if constexpr (!SCATTER && TOKG) {
-    if (a.check.report != nullptr && check_in_kernel<NT>(a)) return;
+    if (a.check.report != nullptr && a.check.words == 0 && check_in_kernel<NT>(a)) return;
   }
   bool valid = (s >= 0) && (s < a.num_slots);
   if constexpr (SCATTER) {
@@ -622,8 +630,10 @@ hipError_t tile_grid(const TileArgs& a0, int64_t planes, TileArgs* a, dim3* grid
     if (tiles > 0x7FFFFFFF) return hipErrorInvalidValue;
     *grid = dim3(static_cast<uint32_t>(tiles), static_cast<uint32_t>(planes), static_cast<uint32_t>(groups));
   } else {
-    if (tiles > 0x7FFFFFFF / groups) return hipErrorInvalidValue;
-    *grid = dim3(static_cast<uint32_t>(tiles * groups), static_cast<uint32_t>(planes), 1);
+    const int64_t extra = (a0.check.words + NT / kWave - 1) / (NT / kWave);
+    a->check_groups = static_cast<int32_t>(extra);
+    if (tiles > (0x7FFFFFFF - extra) / groups) return hipErrorInvalidValue;
+    *grid = dim3(static_cast<uint32_t>(tiles * groups + extra), static_cast<uint32_t>(planes), 1);
   }
   *workgroups = tiles * planes * groups;
   return hipSuccess;
@@ -640,9 +650,10 @@ bool linear_rows_whole_lines(const TileArgs& a, int elt) {
 
 template <int ELT, int BS, bool SCATTER>
 hipError_t launch_tile(const TileArgs& a0, int64_t planes, hipStream_t stream) {
-  // Checked by its own kernel: scatters with a duplicate table and the small
-  // gathers' instantiations.
-  if (a0.check.report != nullptr && (SCATTER ? a0.scan_dupes == 0 : a0.num_tokens > kTokenGatherTokens))
+  // Checked by its own kernel: scatters with a duplicate table, the small
+  // gathers' instantiations, and every gather in shares.
+  if (a0.check.report != nullptr &&
+      (SCATTER ? a0.scan_dupes == 0 : a0.check.words == 0 && a0.num_tokens > kTokenGatherTokens))
     return hipErrorNotSupported;
   if constexpr (SCATTER) {
     // Destination order when the claim tags form this call's inverse map and
@@ -720,8 +731,8 @@ hipError_t launch_tile(const TileArgs& a0, int64_t planes, hipStream_t stream) {
   // no faster with it.
   const bool few = SCATTER ? workgroups <= kFewGroups
                            : !(planes >= kXcdOrderPlanes && workgroups > kFewGroups &&
-                               workgroups <= int64_t{0xFFFFFFFF});
-  if (!SCATTER && a0.check.report != nullptr && !few) return hipErrorNotSupported;
+                               int64_t{grid.x} * planes <= int64_t{0xFFFFFFFF});
+  if (!SCATTER && a0.check.report != nullptr && a0.check.words == 0 && !few) return hipErrorNotSupported;
   if (few && !SCATTER && a0.num_tokens <= kTokenGatherTokens)
     hipLaunchKernelGGL((paged_tile_kernel<ELT, BS, SCATTER, true, kCoopThreads, kBufNT, !SCATTER>), grid,
                        dim3(kCoopThreads), 0, stream, a);

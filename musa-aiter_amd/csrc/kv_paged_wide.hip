@@ -215,7 +215,13 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wide_gather_kernel(const 
   using W = Wide<ELT>;
   constexpr int TT = W::UC;
   const int lane = lane_id();
-  const WgXyz wg = xcd_contiguous_wg<XCD>();
+  WgXyz wg = xcd_contiguous_wg<XCD>();
+  const uint32_t ahead = static_cast<uint32_t>(a.check_groups);
+  if (wg.x < ahead) {
+    check_share<kBlockThreads>(a, wg.x, wg.y);
+    return;
+  }
+  wg.x -= ahead;
   const uint32_t tile = wg.x / static_cast<uint32_t>(a.row_groups);
   const uint32_t group = wg.x - tile * static_cast<uint32_t>(a.row_groups);
   const int64_t t0 = static_cast<int64_t>(tile) * TT;
@@ -396,7 +402,7 @@ constexpr int64_t kWideXcdPlanes = 32;
 template <int ELT, bool SCATTER>
 hipError_t launch_wide(const TileArgs& a0, int64_t planes, bool lines, hipStream_t stream) {
   using W = Wide<ELT>;
-  if (a0.check.report != nullptr && !a0.scan_dupes) return hipErrorNotSupported;
+  if (a0.check.report != nullptr && (SCATTER ? a0.scan_dupes == 0 : a0.check.words == 0)) return hipErrorNotSupported;
   TileArgs a = a0;
   const int64_t chunks = (a.nrows + W::UC - 1) / W::UC;
   const int64_t groups = (chunks + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -409,9 +415,12 @@ hipError_t launch_wide(const TileArgs& a0, int64_t planes, bool lines, hipStream
   const int64_t tiles = by_unit ? a.num_slots / W::UC : (a.num_tokens + tt - 1) / tt;
   if (groups > 0x7FFFFFFF || tiles > 0x7FFFFFFF / groups) return hipErrorInvalidValue;
   a.row_groups = static_cast<int32_t>(groups);
-  const dim3 grid(static_cast<uint32_t>(tiles * groups), static_cast<uint32_t>(planes));
+  const int64_t extra = SCATTER ? 0 : (a.check.words + kWavesPerBlock - 1) / kWavesPerBlock;
+  a.check_groups = static_cast<int32_t>(extra);
+  if (tiles * groups > 0x7FFFFFFF - extra) return hipErrorInvalidValue;
+  const dim3 grid(static_cast<uint32_t>(tiles * groups + extra), static_cast<uint32_t>(planes));
   const dim3 block(kBlockThreads);
-  const bool xcd = planes >= kWideXcdPlanes && tiles * groups * planes <= int64_t{0xFFFFFFFF};
+  const bool xcd = planes >= kWideXcdPlanes && int64_t{grid.x} * planes <= int64_t{0xFFFFFFFF};
   if constexpr (SCATTER) {
     if (by_unit && xcd)
       hipLaunchKernelGGL((paged_wide_unit_scatter_kernel<ELT, true, kBufWT>), grid, block, 0, stream, a);

@@ -454,7 +454,7 @@ __global__ __launch_bounds__(kBlockThreads) void check_kernel(const CheckArgs a)
   __syncthreads();
   if (threadIdx.x != 0) return;
   if (refused) *a.guard = a.check.stamp;
-  __hip_atomic_store(a.check.report + blockIdx.x, 2 * a.check.stamp + refused, __ATOMIC_RELEASE,
+  __hip_atomic_store(a.check.report + blockIdx.x, 2 * a.check.stamp + refused, __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_SYSTEM);
 }
 

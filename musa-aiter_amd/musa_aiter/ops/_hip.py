@@ -311,9 +311,9 @@ def index_max(idx: torch.Tensor) -> int:
         return int(buf.numpy()[:parts].max())
 
 
-# musa_aiter_hip_paged_tiles_call: eight int32 flags, five tensors, eight int64 sizes and strides, two
-# scale pointers, the claims pointer, report and guard addresses, report words and stamp.
-_PAGED_TILES_CALL = struct.Struct("<8i5Q8q2QQ2Q2q")
+# musa_aiter_hip_paged_tiles_call: ten int32 flags (the last one unused), five tensors, eight int64 sizes and
+# strides, two scale pointers, the claims pointer, report and guard addresses, report words and stamp.
+_PAGED_TILES_CALL = struct.Struct("<10i5Q8q2QQ2Q2q")
 _REFUSED = -1  # MUSA_AITER_HIP_REFUSED
 _REPORT_WORDS = 192      # 64 workgroups of a table check at three words each
 _SLOT_CHECK_WORDS = 64   # workgroups of a slot check
@@ -365,7 +365,7 @@ def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, l
             claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter else (0, None))
             checks.stamp += 1
             call = _PAGED_TILES_CALL.pack(
-                scatter, codec, cache_elt, lin_elt, lin_dtype, scale_mode, fill_zeros, scatter,
+                scatter, codec, cache_elt, lin_elt, lin_dtype, scale_mode, fill_zeros, scatter, 0, 0,
                 key_cache.data_ptr(), value_cache.data_ptr(), key_linear.data_ptr(), value_linear.data_ptr(),
                 slots.data_ptr(), num_layers, num_tokens, num_blocks, num_heads, head_dim, block_size,
                 lin_token_stride, lin_layer_stride, _data(k_scale), _data(v_scale), claims, checks.report_ptr,

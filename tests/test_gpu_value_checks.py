@@ -1,7 +1,7 @@
 """Slots and FP8 scales that a call must refuse are found on the device, before anything is written.
 
-Calls of at most 256 tokens check them in the kernel that moves them, larger ones (and those whose kernel
-cannot) in a kernel ahead of it on the stream.  Either way the error, the untouched caches and outputs
+Calls of at most 256 tokens check them in the kernel that moves them, 16- and 32-bit gathers into new rows in
+extra workgroups of that kernel, the others in a kernel ahead of it on the stream.  Either way the error, the untouched caches and outputs
 and the next call on the stream are what a check on the host ahead of the launch would give.
 """
 
@@ -317,3 +317,37 @@ def test_native_argument_checks_agree_with_the_python_layer(layers, monkeypatch)
             assert all(a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride() and
                        torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(got, want)), k
     assert taken >= 8  # the plain forms do take the native path
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.uint8])
+@pytest.mark.parametrize("bs", [5, 8, 16, 32, 64])
+@pytest.mark.parametrize("tokens,layers", [(200, 20), (257, 1), (1500, 20), (16385, 2)])  # 16,385: a 65th share
+def test_gather_into_new_rows_checks_itself_in_shares(dtype, bs, tokens, layers):
+    # Without outputs of the caller's the launch that gathers (16- and 32-bit elements, aligned blocks) also
+    # checks: the error, and the rows of the next call, are as before.  Bad slots at the edges of the waves'
+    # shares of 256.
+    nb, slots, caches, _ = _setup(bs, tokens, layers, dtype)
+    fp8 = dtype is torch.uint8
+    gather = _names("kv_paged_fp8_to_linear" if fp8 else "kv_paged_to_linear", layers)
+    scales = [torch.full((NH,), s, device=DEV) for s in (0.5, 0.25)] if fp8 else []
+    good = slots.clone()
+    good[tokens // 3] = -1
+    outs = [torch.full(((layers,) if layers > 1 else ()) + (tokens, NH, HD), 7.0, device=DEV,
+                        dtype=torch.bfloat16 if fp8 else dtype) for _ in range(2)]
+    kwargs = {"out_dtype": torch.bfloat16} if fp8 else {}
+    want = gather(*caches, good, *scales, out_k=outs[0], out_v=outs[1], **kwargs)
+    for at in sorted({0, 255, 256, 64 * 256 - 1, 64 * 256, tokens - 1}):
+        if at >= tokens:
+            continue
+        bad = good.clone()
+        bad[at] = nb * bs
+        with pytest.raises(ValueError, match=f"slot index {nb * bs} out of bounds"):
+            gather(*caches, bad, *scales, **kwargs)
+    for k in range(2 * len(scales)):
+        bad_scales = [s.clone() for s in scales]
+        bad_scales[k // 2][-(k % 2)] = float("inf")
+        with pytest.raises(ValueError, match="FP8 scale must be positive and finite"):
+            gather(*caches, good, *bad_scales, **kwargs)
+    for x, y in zip(gather(*caches, good, *scales, **kwargs), want):
+        assert torch.equal(x.view(torch.int16 if x.element_size() == 2 else torch.int32),
+                           y.view(torch.int16 if y.element_size() == 2 else torch.int32))
