@@ -335,6 +335,7 @@ class _CheckSet:
 
 _check_sets: dict[tuple[int, int], _CheckSet] = {}
 _check_sets_lock = threading.Lock()
+_MAX_CHECK_SETS = 64  # torch hands out 32 streams per device; streams of other origin come and go
 
 
 def _check_set(device: torch.device, stream: int) -> _CheckSet:
@@ -344,6 +345,10 @@ def _check_set(device: torch.device, stream: int) -> _CheckSet:
         with _check_sets_lock:
             found = _check_sets.get(key)
             if found is None:
+                # A set that gives way is kept by the calls that hold it; its guard word goes back to the
+                # allocator of its own stream, behind the kernels that read it.
+                while len(_check_sets) >= _MAX_CHECK_SETS:
+                    _check_sets.pop(next(iter(_check_sets)))
                 found = _check_sets[key] = _CheckSet(device)
     return found
 

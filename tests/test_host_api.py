@@ -343,3 +343,14 @@ def test_dense_preload_cpu_tensors_are_rejected_not_computed():
                                                              torch.tensor([0, 2]), torch.tensor([1, 3]), max_seq_len=2)
     with pytest.raises(RuntimeError, match="ROCm GPU"):
         musa_aiter.kv_copy_paged_blocks(kc, kc.clone(), kc.clone(), kc.clone(), torch.tensor([[0, 1]]))
+
+
+def test_check_sets_of_many_streams_are_bounded(monkeypatch):
+    from musa_aiter.ops import _hip
+
+    monkeypatch.setattr(_hip, "_check_sets", {})
+    monkeypatch.setattr(_hip, "_CheckSet", lambda device: object())
+    device = torch.device("cuda", 0)
+    sets = [_hip._check_set(device, stream) for stream in range(3 * _hip._MAX_CHECK_SETS)]
+    assert len(_hip._check_sets) == _hip._MAX_CHECK_SETS
+    assert _hip._check_set(device, 3 * _hip._MAX_CHECK_SETS - 1) is sets[-1]
