@@ -370,18 +370,18 @@ int paged_tiles(int scatter, int codec, int cache_elt, int lin_elt, int lin_dtyp
   return kvhip::launch_paged_tiles(p, stream);
 }
 
-// Waits until each of `words` verdict words, `pitch` words apart, carries
-// `stamp`; *refused tells whether any of them refuses the call.  The words arrive as the checking
-// kernel runs, so polling them returns sooner than a stream synchronisation; a
-// kernel that has not run after 0.2 s (the stream busy with earlier work) is
-// waited for by the synchronisation.
-hipError_t await_verdict(const int64_t* report, int64_t words, int64_t stamp, hipStream_t stream, bool* refused,
-                         int64_t pitch = 1) {
+// Waits until each of `words` verdict words carries `stamp`; *refused tells
+// whether any of them refuses the call.  Nothing but verdicts is ever written
+// to these words, so a word that carries the stamp is this call's.  The words
+// arrive as the checking kernel runs, so polling them returns sooner than a
+// stream synchronisation; a kernel that has not run after 0.2 s (the stream
+// busy with earlier work) is waited for by the synchronisation.
+hipError_t await_verdict(const int64_t* report, int64_t words, int64_t stamp, hipStream_t stream, bool* refused) {
   const auto deadline = std::chrono::steady_clock::now() + std::chrono::milliseconds(200);
   *refused = false;
   bool synced = false;
   for (int64_t w = 0; w < words;) {
-    const int64_t v = __atomic_load_n(&report[w * pitch], __ATOMIC_ACQUIRE);
+    const int64_t v = __atomic_load_n(&report[w], __ATOMIC_ACQUIRE);
     if ((v >> 1) == stamp) {
       *refused = *refused || (v & 1) != 0;
       ++w;
@@ -811,21 +811,23 @@ int musa_aiter_hip_paged_tiles_checked(const musa_aiter_hip_paged_tiles_call* ca
 
 int musa_aiter_hip_block_tables_check(const int64_t* block_tables, const int64_t* seq_lens, int64_t batch,
                                       int64_t max_blocks, int64_t num_blocks, int64_t block_size, int64_t* report,
-                                      int64_t report_words, int64_t stamp, int64_t* out, void* stream) {
-  if (report == nullptr || report_words < 3 || stamp <= 0 || out == nullptr) return hipErrorInvalidValue;
-  const int64_t groups = batch < report_words / 3 ? batch : report_words / 3;
+                                      int64_t report_words, int64_t* values, int64_t stamp, int64_t* out,
+                                      void* stream) {
+  if (report == nullptr || report_words < 1 || values == nullptr || stamp <= 0 || out == nullptr)
+    return hipErrorInvalidValue;
+  const int64_t groups = batch < report_words ? batch : report_words;
   hipError_t err = kvhip::launch_table_check(block_tables, seq_lens, batch, max_blocks, num_blocks, block_size, report,
-                                             stamp, groups, as_stream(stream));
+                                             values, stamp, groups, as_stream(stream));
   if (err != hipSuccess) return err;
   bool refused = false;
-  err = await_verdict(report + 2, groups, stamp, as_stream(stream), &refused, 3);
+  err = await_verdict(report, groups, stamp, as_stream(stream), &refused);
   if (err != hipSuccess) return err;
-  out[0] = report[0];
-  out[1] = report[1];
+  out[0] = values[0];
+  out[1] = values[1];
   out[2] = refused ? 1 : 0;
   for (int64_t g = 1; g < groups; ++g) {
-    out[0] = report[3 * g] < out[0] ? report[3 * g] : out[0];
-    out[1] = report[3 * g + 1] > out[1] ? report[3 * g + 1] : out[1];
+    out[0] = values[2 * g] < out[0] ? values[2 * g] : out[0];
+    out[1] = values[2 * g + 1] > out[1] ? values[2 * g + 1] : out[1];
   }
   return hipSuccess;
 }

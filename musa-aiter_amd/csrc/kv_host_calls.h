@@ -17,9 +17,10 @@ extern "C" {
 /* musa_aiter_hip_paged_tiles (same fields) whose slots and scales are checked on the device: a slot
  * >= num_blocks * block_size or a scale that is not positive and finite refuses the call before
  * anything is written.  The verdict is read from `report`, `report_words` (>= 1) words of pinned
- * host memory; `guard` is a device word (0 at first), `stamp` > 0 differs from every earlier call on
- * the same guard, and calls sharing a guard are issued one after another on one stream.  The entry
- * returns when the verdict is there, which does not wait for the copy. */
+ * host memory, 0 at first, to which nothing but the verdicts of these entries is ever written; `guard`
+ * is a device word (0 at first), `stamp` > 0 differs from every earlier call on the same report words
+ * or guard, and calls sharing either are issued one after another on one stream.  The entry returns
+ * when the verdict is there, which does not wait for the copy. */
 typedef struct musa_aiter_hip_paged_tiles_call {
   int32_t scatter, codec, cache_elt, lin_elt, lin_dtype, scale_mode, fill_zeros, dedupe;
   int32_t discard;  /* a gather whose rows the caller throws away if it is refused: they may be written then */
@@ -54,11 +55,13 @@ int musa_aiter_hip_copy_rows_paged_checked(const musa_aiter_hip_copy_rows_paged_
 /* Block tables [batch, max_blocks] and seq_lens [batch] (device, int64) of a dense call, read on the
  * device: out[0] / out[1] receive the smallest and largest length, out[2] is 1 when a sequence uses a
  * block id outside [0, num_blocks) (ids past ceil(len / block_size), and columns the table does not
- * have, are not read), else 0.  report: report_words (>= 3) words of pinned host memory; `stamp` > 0
- * differs from every earlier call on the same words.  Returns when the values are there. */
+ * have, are not read), else 0.  report, report_words, stamp: as above (the words may be shared with
+ * the calls above); values: 2 * report_words further words of pinned host memory, for the lengths,
+ * in which no verdict is looked for.  Returns when the values are there. */
 int musa_aiter_hip_block_tables_check(const int64_t* block_tables, const int64_t* seq_lens, int64_t batch,
                                       int64_t max_blocks, int64_t num_blocks, int64_t block_size, int64_t* report,
-                                      int64_t report_words, int64_t stamp, int64_t* out, void* stream);
+                                      int64_t report_words, int64_t* values, int64_t stamp, int64_t* out,
+                                      void* stream);
 
 #ifdef __cplusplus
 }

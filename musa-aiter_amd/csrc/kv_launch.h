@@ -134,13 +134,13 @@ struct ClaimSource {
 // tokens write, so that a following claim pass needs no cleared array.
 hipError_t launch_claim(const ClaimSource& src, int64_t n, int64_t rows, uint64_t* owner, uint32_t epoch,
                         hipStream_t stream, bool reset = false);
-// Block tables of a dense call (kv_rows.hip): `groups` workgroups write the
-// smallest and largest sequence length they see and then the verdict word (2 *
-// stamp + 1 when a sequence uses a block id outside [0, num_blocks)) to
-// report[3 * g ...].
+// Block tables of a dense call (kv_rows.hip): workgroup g of `groups` writes the
+// smallest and largest sequence length it sees to values[2 * g ...] and then
+// the verdict word (2 * stamp + 1 when a sequence uses a block id outside [0,
+// num_blocks)) to report[g].
 hipError_t launch_table_check(const int64_t* tables, const int64_t* seq_lens, int64_t batch, int64_t max_blocks,
-                              int64_t num_blocks, int64_t block_size, int64_t* report, int64_t stamp, int64_t groups,
-                              hipStream_t stream);
+                              int64_t num_blocks, int64_t block_size, int64_t* report, int64_t* values, int64_t stamp,
+                              int64_t groups, hipStream_t stream);
 hipError_t launch_fill_u64(uint64_t* p, int64_t n, uint64_t value, hipStream_t stream);
 
 // Maxima of idx[0, n) per workgroup into partial[0, parts), then `stamp`

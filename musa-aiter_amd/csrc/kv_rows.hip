@@ -462,11 +462,12 @@ __global__ __launch_bounds__(kBlockThreads) void check_kernel(const CheckArgs a)
 // takes sequences g, g + grid, ... and reads ceil(len / block_size) ids of each
 // (at most the table's columns).  One kernel and three words per workgroup to
 // pinned memory stand for two device-to-host copies and a dozen host tensor
-// operations.
+// operations.  The lengths go to words of their own: in a verdict word a length
+// could equal the next call's verdict.
 __global__ __launch_bounds__(kBlockThreads) void table_check_kernel(const int64_t* tables, const int64_t* seq_lens,
                                                                     int64_t batch, int64_t max_blocks,
                                                                     int64_t num_blocks, int64_t block_size,
-                                                                    int64_t* report, int64_t stamp) {
+                                                                    int64_t* report, int64_t* values, int64_t stamp) {
   int64_t lo = INT64_MAX, hi = INT64_MIN;
   bool bad = false;
   for (int64_t b = blockIdx.x; b < batch; b += gridDim.x) {
@@ -487,10 +488,10 @@ __global__ __launch_bounds__(kBlockThreads) void table_check_kernel(const int64_
   if (bad) refused = 1;
   __syncthreads();
   if (threadIdx.x != 0) return;
-  int64_t* const r = report + 3 * static_cast<int64_t>(blockIdx.x);
+  int64_t* const r = values + 2 * static_cast<int64_t>(blockIdx.x);
   r[0] = lo;
   r[1] = hi;
-  __hip_atomic_store(r + 2, 2 * stamp + refused, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(report + blockIdx.x, 2 * stamp + refused, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ----- strided block transfer ------------------------------------------------------
@@ -835,13 +836,13 @@ hipError_t launch_check(const CheckSource& src, const CallCheck& check, int64_t 
 }
 
 hipError_t launch_table_check(const int64_t* tables, const int64_t* seq_lens, int64_t batch, int64_t max_blocks,
-                              int64_t num_blocks, int64_t block_size, int64_t* report, int64_t stamp, int64_t groups,
-                              hipStream_t stream) {
+                              int64_t num_blocks, int64_t block_size, int64_t* report, int64_t* values, int64_t stamp,
+                              int64_t groups, hipStream_t stream) {
   if (seq_lens == nullptr || (tables == nullptr && max_blocks > 0) || batch < 1 || max_blocks < 0 || block_size < 1 ||
-      report == nullptr || groups < 1)
+      report == nullptr || values == nullptr || groups < 1)
     return hipErrorInvalidValue;
   hipLaunchKernelGGL(table_check_kernel, dim3(static_cast<uint32_t>(groups)), dim3(kBlockThreads), 0, stream, tables,
-                     seq_lens, batch, max_blocks, num_blocks, block_size, report, stamp);
+                     seq_lens, batch, max_blocks, num_blocks, block_size, report, values, stamp);
   return hipGetLastError();
 }
 

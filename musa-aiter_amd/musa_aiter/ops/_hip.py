@@ -92,8 +92,9 @@ _SIGNATURES: dict[str, list] = {
     #  head_dim, block_size, stream); the "_fp8_vec8" entry copies one-byte elements.
     "musa_aiter_kv_copy_paged_blocks_fp8_vec8": [_c_void_p] * 5 + [_i64] * 7 + [_c_void_p],
     "musa_aiter_hip_paged_tiles_checked": [ctypes.c_char_p, _c_void_p],  # musa_aiter_hip_paged_tiles_call, stream
-    # (block_tables, seq_lens, batch, max_blocks, blocks, block_size, report, report_words, stamp, out, stream)
-    "musa_aiter_hip_block_tables_check": [_c_void_p] * 2 + [_i64] * 4 + [_c_void_p, _i64, _i64, _c_void_p, _c_void_p],
+    # (block_tables, seq_lens, batch, max_blocks, blocks, block_size, report, report_words, values, stamp, out, stream)
+    "musa_aiter_hip_block_tables_check": [_c_void_p] * 2 + [_i64] * 4 + [_c_void_p, _i64, _c_void_p, _i64, _c_void_p,
+                                                                        _c_void_p],
     "musa_aiter_hip_copy_rows_paged_checked": [ctypes.c_char_p, _c_void_p],  # musa_aiter_hip_copy_rows_paged_call, stream
     "musa_aiter_hip_error_string": [_i32],
     "musa_aiter_hip_backend_name": [],
@@ -315,21 +316,22 @@ def index_max(idx: torch.Tensor) -> int:
 # strides, two scale pointers, the claims pointer, report and guard addresses, report words and stamp.
 _PAGED_TILES_CALL = struct.Struct("<10i5Q8q2QQ2Q2q")
 _REFUSED = -1  # MUSA_AITER_HIP_REFUSED
-_REPORT_WORDS = 192      # 64 workgroups of a table check at three words each
-_SLOT_CHECK_WORDS = 64   # workgroups of a slot check
+_REPORT_WORDS = 64              # verdict words, one per workgroup of a check
+_VALUE_WORDS = 2 * _REPORT_WORDS  # two lengths per workgroup of a table check; no verdict is read from them
 
 
 class _CheckSet:
-    """Verdict words (pinned host memory), guard word (device memory) and stamp of the checked calls on one
-    (device, stream), which issue one at a time under the lock: a check kernel, where there is one, and the
-    kernel it guards follow each other on the stream."""
-    __slots__ = ("lock", "report", "guard", "report_ptr", "guard_ptr", "stamp")
+    """Verdict words and table-check values (pinned host memory), guard word (device memory) and stamp of the
+    checked calls on one (device, stream), which issue one at a time under the lock: a check kernel, where there
+    is one, and the kernel it guards follow each other on the stream."""
+    __slots__ = ("lock", "report", "guard", "report_ptr", "values_ptr", "guard_ptr", "stamp")
 
     def __init__(self, device: torch.device):
         self.lock = threading.Lock()
-        self.report = torch.zeros(_REPORT_WORDS, dtype=torch.int64, pin_memory=True)
+        self.report = torch.zeros(_REPORT_WORDS + _VALUE_WORDS, dtype=torch.int64, pin_memory=True)
         self.guard = torch.zeros(1, dtype=torch.int64, device=device)
         self.report_ptr, self.guard_ptr = self.report.data_ptr(), self.guard.data_ptr()
+        self.values_ptr = self.report_ptr + 8 * _REPORT_WORDS
         self.stamp = 0
 
 
@@ -374,7 +376,7 @@ def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, l
                 key_cache.data_ptr(), value_cache.data_ptr(), key_linear.data_ptr(), value_linear.data_ptr(),
                 slots.data_ptr(), num_layers, num_tokens, num_blocks, num_heads, head_dim, block_size,
                 lin_token_stride, lin_layer_stride, _data(k_scale), _data(v_scale), claims, checks.report_ptr,
-                checks.guard_ptr, _SLOT_CHECK_WORDS, checks.stamp)
+                checks.guard_ptr, _REPORT_WORDS, checks.stamp)
             rc = fn("musa_aiter_hip_paged_tiles_checked")(call, stream)
             del keep
     if rc == _REFUSED:
@@ -417,7 +419,7 @@ def paged_native(key_cache, value_cache, linear, slots, scales, *, layered: bool
         checks.stamp += 1
         rc, k, v = h.paged_call(key_cache, value_cache, lin_k, lin_v, slots, k_scale, v_scale, scatter, layered, codec,
                                 out_dtype, _paged_entry[0], claims, checks.report_ptr, checks.guard_ptr,
-                                _SLOT_CHECK_WORDS, checks.stamp, stream, index)
+                                _REPORT_WORDS, checks.stamp, stream, index)
         del entry
     if rc == h.NOT_TAKEN or rc == _REFUSED:
         return None
@@ -446,7 +448,7 @@ def copy_rows_paged_checked(*, op: str, device: torch.device, src_planes: list[i
             call = _COPY_ROWS_PAGED_CALL.pack(
                 src.buffer_info()[0], dst.buffer_info()[0], len(src), src_idx.data_ptr(), dst_idx.data_ptr(),
                 src_idx.numel(), src_rows, dst_rows, row_bytes, src_stride, dst_stride, 0, 0, 0, 0, low, claims,
-                checks.report_ptr, checks.guard_ptr, _SLOT_CHECK_WORDS, checks.stamp)
+                checks.report_ptr, checks.guard_ptr, _REPORT_WORDS, checks.stamp)
             rc = fn("musa_aiter_hip_copy_rows_paged_checked")(call, stream)
             del keep
     if rc == _REFUSED:
@@ -468,7 +470,7 @@ def block_tables_check(*, op: str, block_tables: torch.Tensor, seq_lens: torch.T
             checks.stamp += 1
             rc = fn("musa_aiter_hip_block_tables_check")(
                 block_tables.data_ptr(), seq_lens.data_ptr(), seq_lens.numel(), block_tables.shape[1], num_blocks,
-                block_size, checks.report_ptr, _REPORT_WORDS, checks.stamp, out, stream)
+                block_size, checks.report_ptr, _REPORT_WORDS, checks.values_ptr, checks.stamp, out, stream)
     check(rc, op)
     return out[0], out[1], bool(out[2])
 

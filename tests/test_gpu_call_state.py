@@ -1,0 +1,76 @@
+"""What checked calls share on a stream: verdict words, stamps and guard of one call say nothing about another."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import musa_aiter
+from musa_aiter.ops import _hip
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+NH, HD, BS = 2, 16, 16
+
+
+def _paged(tokens, dtype=torch.bfloat16):
+    nb = tokens // BS + 2
+    slots = torch.randperm(nb * BS, device=DEV)[:tokens]
+    caches = [torch.randn((nb, NH, HD, BS), device=DEV).to(dtype) for _ in range(2)]
+    rows = [torch.randn((tokens, NH, HD), device=DEV).to(torch.bfloat16) for _ in range(2)]
+    return nb, slots, caches, rows
+
+
+def _refused_call(kind, tokens):
+    """(an accepted call, the same call with one value to refuse, the error's text)."""
+    if kind == "page":
+        src, dst = (torch.randn((2, tokens + 2, 64), device=DEV) for _ in range(2))
+        idx = torch.randperm(tokens + 2, device=DEV)[:tokens]
+        bad = idx.clone()
+        bad[0] = tokens + 2
+
+        def move(i):
+            musa_aiter.hicache_transfer_kv_all_layer(src, dst, src, dst.clone(), i, idx)
+
+        return lambda: move(idx), lambda: move(bad), "page index is out of range"
+    nb, slots, caches, rows = _paged(tokens)
+    if kind == "scale":
+        codes = [torch.zeros((nb, NH, HD, BS), dtype=torch.uint8, device=DEV) for _ in range(2)]
+        good = torch.ones(NH, device=DEV)
+        return (lambda: musa_aiter.kv_linear_to_paged_fp8(*rows, *codes, slots, good, good),
+                lambda: musa_aiter.kv_linear_to_paged_fp8(*rows, *codes, slots, good, -good),
+                "v_scale: FP8 scale must be positive and finite")
+    bad = slots.clone()
+    bad[0] = nb * BS
+    if kind == "store":
+        return (lambda: musa_aiter.kv_linear_to_paged(*rows, *caches, slots),
+                lambda: musa_aiter.kv_linear_to_paged(*rows, *caches, bad), "out of bounds")
+    return (lambda: musa_aiter.kv_paged_to_linear(*caches, slots),
+            lambda: musa_aiter.kv_paged_to_linear(*caches, bad), "out of bounds")
+
+
+# Calls of one verdict word (the moving kernel's own), and of several (a check kernel's, a gather's shares).
+@pytest.mark.parametrize("tokens", [200, 1500, 5000])
+@pytest.mark.parametrize("kind", ["store", "gather", "scale", "page"])
+@pytest.mark.parametrize("which", ["shortest", "longest"])
+def test_lengths_of_a_dense_call_are_no_verdict(which, kind, tokens):
+    # A dense call's table check leaves sequence lengths in host memory; one that equals the next call's
+    # "accepted" word (twice its stamp) must not be taken for that call's verdict.
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        accepted, refused, text = _refused_call(kind, tokens)
+        accepted()  # the stream's state exists from here on
+        checks = _hip._check_set(torch.device(DEV, torch.cuda.current_device()), stream.cuda_stream)
+        word = 2 * (checks.stamp + 2)  # the dense call takes the next stamp
+        lens = [word, word + 9] if which == "shortest" else [word - 1, word]
+        cols = (max(lens) + BS - 1) // BS
+        caches = [torch.zeros((cols, 1, 8, BS), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        # Both lengths in every workgroup of the table check (at most 64), so in every word it writes.
+        lens = torch.tensor(lens, device=DEV).repeat_interleave(64)
+        tables = torch.arange(cols, device=DEV).repeat(128, 1)
+        musa_aiter.kv_load_and_reshape_flash(*caches, tables, lens)
+        assert 2 * (checks.stamp + 1) == word
+        with pytest.raises(ValueError, match=text):
+            refused()
+        accepted()
+    torch.cuda.synchronize()
