@@ -285,6 +285,11 @@ def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int):
     return ctypes.addressof(c), entry
 
 
+def _pinned_words(n: int) -> torch.Tensor:
+    """``n`` zeroed words of pinned host memory (the device is named: torch.set_default_device must not move them)."""
+    return torch.zeros(n, dtype=torch.int64, device="cpu", pin_memory=True)
+
+
 _INDEX_MAX_PARTS = 64
 _index_max_lock = threading.Lock()
 _index_max_bufs: dict[int, list] = {}
@@ -303,7 +308,7 @@ def index_max(idx: torch.Tensor) -> int:
     with on_device(device), _index_max_lock:
         entry = _index_max_bufs.get(index)
         if entry is None:
-            entry = [torch.zeros(2 * _INDEX_MAX_PARTS, dtype=torch.int64, pin_memory=True), 0]
+            entry = [_pinned_words(2 * _INDEX_MAX_PARTS), 0]
             _index_max_bufs[index] = entry
         buf = entry[0]
         entry[1] += 1  # the stamp of this call (nonzero, never repeated)
@@ -328,7 +333,7 @@ class _CheckSet:
 
     def __init__(self, device: torch.device):
         self.lock = threading.Lock()
-        self.report = torch.zeros(_REPORT_WORDS + _VALUE_WORDS, dtype=torch.int64, pin_memory=True)
+        self.report = _pinned_words(_REPORT_WORDS + _VALUE_WORDS)
         self.guard = torch.zeros(1, dtype=torch.int64, device=device)
         self.report_ptr, self.guard_ptr = self.report.data_ptr(), self.guard.data_ptr()
         self.values_ptr = self.report_ptr + 8 * _REPORT_WORDS

@@ -1050,7 +1050,7 @@ def _first_bad_block(block_tables_cpu: torch.Tensor, seq_lens_cpu: torch.Tensor,
     if batch == 0 or max_blocks == 0:
         return None
     needed = (seq_lens_cpu.clamp(min=0) + bs - 1) // bs
-    used = torch.arange(max_blocks).unsqueeze(0) < needed.unsqueeze(1)
+    used = torch.arange(max_blocks, device=needed.device).unsqueeze(0) < needed.unsqueeze(1)
     bad = used & ((block_tables_cpu < 0) | (block_tables_cpu >= nb))
     if not bool(bad.any()):
         return None

@@ -74,3 +74,20 @@ def test_lengths_of_a_dense_call_are_no_verdict(which, kind, tokens):
             refused()
         accepted()
     torch.cuda.synchronize()
+
+
+def test_calls_under_a_default_device():
+    # torch.device / set_default_device redirects factory functions; the host words of a stream's first call
+    # are host memory all the same.
+    idx = torch.tensor([2, 0, 1], device=DEV)
+    src, dst = torch.randn((2, 3, 64), device=DEV), torch.zeros((2, 3, 64), device=DEV)
+    with torch.cuda.stream(torch.cuda.Stream()), torch.device(DEV), pytest.MonkeyPatch.context() as patch:
+        patch.setattr(_hip, "_check_sets", {})
+        musa_aiter.hicache_transfer_kv_all_layer(src, dst, src, dst.clone(), idx, idx)
+        caches = [torch.ones((2, 1, 8, BS), dtype=torch.bfloat16) for _ in range(2)]
+        k, _ = musa_aiter.kv_load_and_reshape_flash(*caches, torch.tensor([[0, 1]]), torch.tensor([20]))
+        with pytest.raises(ValueError, match="invalid block id 2"):
+            musa_aiter.kv_load_and_reshape_flash(*caches, torch.tensor([[0, 2]]), torch.tensor([20]))
+    torch.cuda.synchronize()
+    assert torch.equal(src, dst)
+    assert k.shape == (1, 20, 1, 8) and bool((k == 1).all())
