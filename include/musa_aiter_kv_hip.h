@@ -57,7 +57,9 @@ int64_t musa_aiter_hip_allocated_bytes(void);
  * visits to partial[w] (INT64_MIN if none) and then `stamp` (nonzero, a value the caller changes per
  * call) to partial[parts + w].  `partial` (2 * parts entries) is pinned host memory the caller owns;
  * the call returns once every stamp is there (after at most 0.2 s of polling it synchronises the
- * stream instead), so the maxima can be read right after it; n >= 1. */
+ * stream instead), so the maxima can be read right after it; n >= 1.  A caller that reuses memory for
+ * calls of different `parts` keeps the words of earlier maxima out of later stamps (by a `partial`
+ * whose entry [parts] is always the same word): a maximum may equal a stamp. */
 int musa_aiter_hip_index_max(const int64_t* idx, int64_t n, int64_t* partial, int64_t parts, int64_t stamp,
                              void* stream);
 /* No reference counterpart: the access-pattern ceiling of a paged copy, timed by bench.py.  Copies

@@ -312,9 +312,12 @@ def index_max(idx: torch.Tensor) -> int:
             _index_max_bufs[index] = entry
         buf = entry[0]
         entry[1] += 1  # the stamp of this call (nonzero, never repeated)
-        check(fn("musa_aiter_hip_index_max")(ptr(idx), n, ptr(buf), parts, entry[1], stream_ptr(device)),
-              "index_max")
-        return int(buf.numpy()[:parts].max())
+        # The entry puts `parts` maxima in front of `parts` stamps: they end and begin in the middle of the
+        # words, so that no word holds a maximum of one call and is looked at for another's stamp.
+        first = _INDEX_MAX_PARTS - parts
+        check(fn("musa_aiter_hip_index_max")(ptr(idx), n, buf.data_ptr() + 8 * first, parts, entry[1],
+                                             stream_ptr(device)), "index_max")
+        return int(buf.numpy()[first:_INDEX_MAX_PARTS].max())
 
 
 # musa_aiter_hip_paged_tiles_call: ten int32 flags (the last one unused), five tensors, eight int64 sizes and

@@ -91,3 +91,16 @@ def test_calls_under_a_default_device():
     torch.cuda.synchronize()
     assert torch.equal(src, dst)
     assert k.shape == (1, 20, 1, 8) and bool((k == 1).all())
+
+
+def test_index_max_of_a_short_vector_after_a_long_one():
+    # The maxima of a long vector's 64 workgroups fill words in which a short vector's single stamp must not be
+    # looked for: a maximum equal to the next stamp would be taken for that call's.
+    long = torch.empty(64 * 4096, dtype=torch.int64, device=DEV)
+    short = torch.tensor([12345678], device=DEV)
+    assert _hip.index_max(short) == 12345678
+    entry = _hip._index_max_bufs[torch.cuda.current_device()]
+    for _ in range(2):
+        long.fill_(entry[1] + 2)  # the stamp of the call after the long vector's
+        assert _hip.index_max(long) == int(long[0])
+        assert _hip.index_max(short) == 12345678
