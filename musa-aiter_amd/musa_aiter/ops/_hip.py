@@ -217,13 +217,13 @@ def check(rc: int, op: str) -> None:
         raise HipBackendError(f"{op}: HIP launch failed with error {rc} ({text})")
 
 
-_SAME_DEVICE = contextlib.nullcontext()
+_NOTHING = contextlib.nullcontext()
 
 
 def on_device(device: torch.device):
     """Context making ``device`` the current device; a no-op (no device exchange) when it already is."""
     if device.index is None or device.index == torch._C._cuda_getDevice():
-        return _SAME_DEVICE
+        return _NOTHING
     return torch.cuda.device(device)
 
 
@@ -256,9 +256,28 @@ _MIN_CLAIM_TAGS = 1 << 16
 _claim_sets: dict[tuple[int, int], tuple[torch.Tensor, _Claims]] = {}
 
 
+# Scatters and checked calls on one (device, stream) issue one at a time, from the advance of the epoch to
+# the last launch.  Otherwise another thread's call could advance the epoch before the library has read it
+# (two calls claiming under one epoch lose rows), or claim between a call's claim pass and its copy.  A lock
+# stays for good, as the claim tags do: stream handles recur.
+_stream_locks: dict[tuple[int, int], threading.Lock] = {}
+
+
+def _stream_key(device: torch.device, stream: ctypes.c_void_p) -> tuple[int, int]:
+    return (device.index if device.index is not None else torch.cuda.current_device(), stream.value or 0)
+
+
+def stream_lock(device: torch.device, stream: ctypes.c_void_p) -> threading.Lock:
+    """The lock to hold from claims_for to the return of the call that uses the claims."""
+    key = _stream_key(device, stream)
+    found = _stream_locks.get(key)
+    return found if found is not None else _stream_locks.setdefault(key, threading.Lock())
+
+
 def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int):
     """The claims of one scatter with ``rows`` destination rows on ``stream``: returns the address of a
-    musa_aiter_hip_claims to pass and the objects to keep alive until the call has returned.
+    musa_aiter_hip_claims to pass and the objects to keep alive until the call has returned.  The caller
+    holds the stream's lock.
 
     Eager calls share one tag array per (device, stream), zeroed when allocated, with an epoch that
     advances per call (no clearing pass; the array is re-zeroed when the 32-bit epoch runs out).
@@ -269,7 +288,7 @@ def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int):
         tags = torch.empty(rows, dtype=torch.int64, device=device)
         c = _Claims(tags.data_ptr(), rows, 0, 0)
         return ctypes.addressof(c), (tags, c)
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream.value or 0)
+    key = _stream_key(device, stream)
     entry = _claim_sets.get(key)
     if entry is None or entry[1].capacity < rows:
         have = entry[1].capacity if entry is not None else 0
@@ -330,12 +349,11 @@ _VALUE_WORDS = 2 * _REPORT_WORDS  # two lengths per workgroup of a table check; 
 
 class _CheckSet:
     """Verdict words and table-check values (pinned host memory), guard word (device memory) and stamp of the
-    checked calls on one (device, stream), which issue one at a time under the lock: a check kernel, where there
-    is one, and the kernel it guards follow each other on the stream."""
-    __slots__ = ("lock", "report", "guard", "report_ptr", "values_ptr", "guard_ptr", "stamp")
+    checked calls on one (device, stream), which issue one at a time under the stream's lock: a check kernel, where
+    there is one, and the kernel it guards follow each other on the stream."""
+    __slots__ = ("report", "guard", "report_ptr", "values_ptr", "guard_ptr", "stamp")
 
     def __init__(self, device: torch.device):
-        self.lock = threading.Lock()
         self.report = _pinned_words(_REPORT_WORDS + _VALUE_WORDS)
         self.guard = torch.zeros(1, dtype=torch.int64, device=device)
         self.report_ptr, self.guard_ptr = self.report.data_ptr(), self.guard.data_ptr()
@@ -375,8 +393,8 @@ def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, l
     device = key_cache.device
     with on_device(device):
         stream = stream_ptr(device)
-        checks = _check_set(device, stream.value or 0)
-        with checks.lock:
+        with stream_lock(device, stream):
+            checks = _check_set(device, stream.value or 0)
             claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter else (0, None))
             checks.stamp += 1
             call = _PAGED_TILES_CALL.pack(
@@ -407,16 +425,19 @@ def paged_native(key_cache, value_cache, linear, slots, scales, *, layered: bool
         return None
     index = torch._C._cuda_getDevice()
     stream = torch._C._cuda_getCurrentRawStream(index)
-    checks = _check_sets.get((index, stream))
-    if checks is None:
-        return None  # the stream's first call makes its set
+    lock = _stream_locks.get((index, stream))
+    if lock is None:
+        return None  # the stream's first call makes its lock, check set and claims
     h = host()
     if not _paged_entry:
         _paged_entry.append(ctypes.cast(fn("musa_aiter_hip_paged_tiles_checked"), ctypes.c_void_p).value)
     scatter = linear is not None
     lin_k, lin_v = linear if scatter else (None, None)
     k_scale, v_scale = scales if scales is not None else (None, None)
-    with checks.lock:
+    with lock:
+        checks = _check_sets.get((index, stream))
+        if checks is None:
+            return None
         claims, entry = 0, None
         if scatter:
             entry = _claim_sets.get((index, stream))
@@ -449,8 +470,8 @@ def copy_rows_paged_checked(*, op: str, device: torch.device, src_planes: list[i
     src, dst = array("Q", src_planes), array("Q", dst_planes)
     with on_device(device):
         stream = stream_ptr(device)
-        checks = _check_set(device, stream.value or 0)
-        with checks.lock:
+        with stream_lock(device, stream):
+            checks = _check_set(device, stream.value or 0)
             claims, keep = claims_for(device, stream, dst_rows)
             checks.stamp += 1
             call = _COPY_ROWS_PAGED_CALL.pack(
@@ -472,9 +493,9 @@ def block_tables_check(*, op: str, block_tables: torch.Tensor, seq_lens: torch.T
     device = seq_lens.device
     with on_device(device):
         stream = stream_ptr(device)
-        checks = _check_set(device, stream.value or 0)
         out = (_i64 * 3)()
-        with checks.lock:
+        with stream_lock(device, stream):
+            checks = _check_set(device, stream.value or 0)
             checks.stamp += 1
             rc = fn("musa_aiter_hip_block_tables_check")(
                 block_tables.data_ptr(), seq_lens.data_ptr(), seq_lens.numel(), block_tables.shape[1], num_blocks,
@@ -540,17 +561,18 @@ def paged_tiles(
     device = key_cache.device
     with on_device(device):
         stream = stream_ptr(device)
-        claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter and dedupe
-                        else (None, None))
-        rc = fn("musa_aiter_hip_paged_tiles")(
-            int(scatter), int(codec), int(cache_elt), int(lin_elt), int(lin_dtype),
-            ptr(key_cache), ptr(value_cache), ptr(key_linear), ptr(value_linear), ptr(slots),
-            int(num_layers), int(num_tokens), int(num_blocks), int(num_heads), int(head_dim), int(block_size),
-            int(lin_token_stride), int(lin_layer_stride),
-            ptr(k_scale), ptr(v_scale), int(scale_mode),
-            int(bool(fill_zeros)), int(bool(dedupe)), claims, stream,
-        )
-        del keep
+        with stream_lock(device, stream) if scatter and dedupe else _NOTHING:
+            claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter and dedupe
+                            else (None, None))
+            rc = fn("musa_aiter_hip_paged_tiles")(
+                int(scatter), int(codec), int(cache_elt), int(lin_elt), int(lin_dtype),
+                ptr(key_cache), ptr(value_cache), ptr(key_linear), ptr(value_linear), ptr(slots),
+                int(num_layers), int(num_tokens), int(num_blocks), int(num_heads), int(head_dim), int(block_size),
+                int(lin_token_stride), int(lin_layer_stride),
+                ptr(k_scale), ptr(v_scale), int(scale_mode),
+                int(bool(fill_zeros)), int(bool(dedupe)), claims, stream,
+            )
+            del keep
     check(rc, op)
 
 
@@ -583,16 +605,17 @@ def copy_rows(
     dst_arr = _as_u64(dst_planes)
     with on_device(device):
         stream = stream_ptr(device)
-        claims, keep = (claims_for(device, stream, dst_rows) if dedupe and dst_idx is not None
-                        else (0, None))
-        # One struct (musa_aiter_hip_copy_rows_call) instead of 19 converted ctypes arguments; the plane
-        # arrays stay referenced by src_arr / dst_arr until the call returns.
-        call = _COPY_ROWS_CALL.pack(
-            _address(src_arr), _address(dst_arr), _data(src_table), _data(dst_table), num_planes,
-            _data(src_idx), _data(dst_idx), num_tokens, num_rows_out, src_offset, dst_offset, src_rows, dst_rows,
-            row_bytes, src_stride, dst_stride, bool(zero_invalid), bool(dedupe), claims)
-        rc = fn("musa_aiter_hip_copy_rows_packed")(call, stream)
-        del keep
+        with stream_lock(device, stream) if dedupe and dst_idx is not None else _NOTHING:
+            claims, keep = (claims_for(device, stream, dst_rows) if dedupe and dst_idx is not None
+                            else (0, None))
+            # One struct (musa_aiter_hip_copy_rows_call) instead of 19 converted ctypes arguments; the plane
+            # arrays stay referenced by src_arr / dst_arr until the call returns.
+            call = _COPY_ROWS_CALL.pack(
+                _address(src_arr), _address(dst_arr), _data(src_table), _data(dst_table), num_planes,
+                _data(src_idx), _data(dst_idx), num_tokens, num_rows_out, src_offset, dst_offset, src_rows, dst_rows,
+                row_bytes, src_stride, dst_stride, bool(zero_invalid), bool(dedupe), claims)
+            rc = fn("musa_aiter_hip_copy_rows_packed")(call, stream)
+            del keep
     check(rc, op)
 
 
@@ -630,16 +653,17 @@ def paged_dense_tiles(
     device = key_cache.device
     with on_device(device):
         stream = stream_ptr(device)
-        claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter and dedupe
-                        else (None, None))
-        rc = fn("musa_aiter_hip_paged_dense_tiles")(
-            int(scatter), int(codec), int(cache_elt), int(lin_elt), int(lin_dtype),
-            ptr(key_cache), ptr(value_cache), ptr(dense_k), ptr(dense_v), ptr(block_tables), ptr(seq_lens),
-            int(batch), int(dense_len), int(max_blocks), int(num_blocks), int(num_heads), int(head_dim),
-            int(block_size), int(dense_token_stride), ptr(k_scale), ptr(v_scale), int(scale_mode),
-            int(bool(fill_zeros)), int(bool(dedupe)), claims, stream,
-        )
-        del keep
+        with stream_lock(device, stream) if scatter and dedupe else _NOTHING:
+            claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter and dedupe
+                            else (None, None))
+            rc = fn("musa_aiter_hip_paged_dense_tiles")(
+                int(scatter), int(codec), int(cache_elt), int(lin_elt), int(lin_dtype),
+                ptr(key_cache), ptr(value_cache), ptr(dense_k), ptr(dense_v), ptr(block_tables), ptr(seq_lens),
+                int(batch), int(dense_len), int(max_blocks), int(num_blocks), int(num_heads), int(head_dim),
+                int(block_size), int(dense_token_stride), ptr(k_scale), ptr(v_scale), int(scale_mode),
+                int(bool(fill_zeros)), int(bool(dedupe)), claims, stream,
+            )
+            del keep
     check(rc, op)
 
 
@@ -699,14 +723,15 @@ def copy_rows_paged(
         raise ValueError(f"{op}: source and destination plane lists differ in length")
     with on_device(device):
         stream = stream_ptr(device)
-        claims, keep = claims_for(device, stream, dst_rows) if dedupe else (None, None)
-        rc = fn("musa_aiter_hip_copy_rows_paged")(
-            u64_array(src_planes), u64_array(dst_planes), planes, ptr(src_idx), ptr(dst_idx), tokens,
-            int(src_rows), int(dst_rows), int(row_bytes), int(src_stride), int(dst_stride),
-            int(src_page_rows), int(src_page_stride), int(dst_page_rows), int(dst_page_stride),
-            int(bool(dedupe)), claims, stream,
-        )
-        del keep
+        with stream_lock(device, stream) if dedupe else _NOTHING:
+            claims, keep = claims_for(device, stream, dst_rows) if dedupe else (None, None)
+            rc = fn("musa_aiter_hip_copy_rows_paged")(
+                u64_array(src_planes), u64_array(dst_planes), planes, ptr(src_idx), ptr(dst_idx), tokens,
+                int(src_rows), int(dst_rows), int(row_bytes), int(src_stride), int(dst_stride),
+                int(src_page_rows), int(src_page_stride), int(dst_page_rows), int(dst_page_stride),
+                int(bool(dedupe)), claims, stream,
+            )
+            del keep
     check(rc, op)
 
 
@@ -735,12 +760,13 @@ def copy_blocks(
     device = dst_k.device
     with on_device(device):
         stream = stream_ptr(device)
-        claims, keep = claims_for(device, stream, dst_blocks)
-        rc = fn("musa_aiter_hip_copy_blocks")(
-            ptr(src_k), ptr(src_v), ptr(dst_k), ptr(dst_v), ptr(block_mapping), pairs, int(num_layers),
-            int(src_blocks), int(dst_blocks), int(block_bytes), claims, stream,
-        )
-        del keep
+        with stream_lock(device, stream):
+            claims, keep = claims_for(device, stream, dst_blocks)
+            rc = fn("musa_aiter_hip_copy_blocks")(
+                ptr(src_k), ptr(src_v), ptr(dst_k), ptr(dst_v), ptr(block_mapping), pairs, int(num_layers),
+                int(src_blocks), int(dst_blocks), int(block_bytes), claims, stream,
+            )
+            del keep
     check(rc, op)
 
 

@@ -372,15 +372,19 @@ def _two_x_nl_fast(op: str, kvcaches, memory_tensor, slot_mapping, skip: int, bl
         _COPY_ROWS_ENTRY.append(ctypes.cast(_hip.fn("musa_aiter_hip_copy_rows_packed"), ctypes.c_void_p).value)
     index = torch._C._cuda_getDevice()
     stream = torch._C._cuda_getCurrentRawStream(index)
-    claims, keep = 0, None
+    call = (kvcaches, memory_tensor, slot_mapping, int(skip), int(block_size), int(num_heads), int(head_size),
+            bool(scatter), _COPY_ROWS_ENTRY[0])
     if scatter:
-        if memory_tensor.device.index != index:
+        device = memory_tensor.device
+        if device.index != index:
             return False
-        claims, keep = _hip.claims_for(memory_tensor.device, ctypes.c_void_p(stream),
-                                       int(kvcaches[0][0].shape[0]) * int(block_size))
-    rc = h.two_x_nl_rows(kvcaches, memory_tensor, slot_mapping, int(skip), int(block_size), int(num_heads),
-                         int(head_size), bool(scatter), _COPY_ROWS_ENTRY[0], claims, stream, index)
-    del keep
+        with _hip.stream_lock(device, ctypes.c_void_p(stream)):
+            claims, keep = _hip.claims_for(device, ctypes.c_void_p(stream),
+                                           int(kvcaches[0][0].shape[0]) * int(block_size))
+            rc = h.two_x_nl_rows(*call, claims, stream, index)
+            del keep
+    else:
+        rc = h.two_x_nl_rows(*call, 0, stream, index)
     if rc < 0:
         return False
     _hip.check(rc, op)
