@@ -12,6 +12,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import importlib.util
+import itertools
 import struct
 import sysconfig
 import threading
@@ -363,21 +364,26 @@ class _CheckSet:
 
 _check_sets: dict[tuple[int, int], _CheckSet] = {}
 _check_sets_lock = threading.Lock()
-_MAX_CHECK_SETS = 64  # torch hands out 32 streams per device; streams of other origin come and go
+_MAX_CHECK_SETS = 64  # per device; torch hands out 32 streams each, streams of other origin come and go
+_uses = itertools.count(1)
+_last_use: dict[tuple[int, int], int] = {}
 
 
 def _check_set(device: torch.device, stream: int) -> _CheckSet:
+    """The check set of a (device, stream), whose lock the caller holds."""
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     found = _check_sets.get(key)
     if found is None:
         with _check_sets_lock:
-            found = _check_sets.get(key)
-            if found is None:
-                # A set that gives way is kept by the calls that hold it; its guard word goes back to the
-                # allocator of its own stream, behind the kernels that read it.
-                while len(_check_sets) >= _MAX_CHECK_SETS:
-                    _check_sets.pop(next(iter(_check_sets)))
-                found = _check_sets[key] = _CheckSet(device)
+            # The least recently used set gives way.  A call that still holds it keeps it; its guard word goes
+            # back to the allocator of its own stream, behind the kernels that read it.
+            own = [k for k in _check_sets if k[0] == key[0]]
+            if len(own) >= _MAX_CHECK_SETS:
+                oldest = min(own, key=lambda k: _last_use.get(k, 0))
+                del _check_sets[oldest]
+                _last_use.pop(oldest, None)
+            found = _check_sets[key] = _CheckSet(device)
+    _last_use[key] = next(_uses)
     return found
 
 
@@ -425,7 +431,8 @@ def paged_native(key_cache, value_cache, linear, slots, scales, *, layered: bool
         return None
     index = torch._C._cuda_getDevice()
     stream = torch._C._cuda_getCurrentRawStream(index)
-    lock = _stream_locks.get((index, stream))
+    key = (index, stream)
+    lock = _stream_locks.get(key)
     if lock is None:
         return None  # the stream's first call makes its lock, check set and claims
     h = host()
@@ -435,12 +442,13 @@ def paged_native(key_cache, value_cache, linear, slots, scales, *, layered: bool
     lin_k, lin_v = linear if scatter else (None, None)
     k_scale, v_scale = scales if scales is not None else (None, None)
     with lock:
-        checks = _check_sets.get((index, stream))
+        checks = _check_sets.get(key)
         if checks is None:
             return None
+        _last_use[key] = next(_uses)
         claims, entry = 0, None
         if scatter:
-            entry = _claim_sets.get((index, stream))
+            entry = _claim_sets.get(key)
             if entry is None or entry[1].epoch == _EPOCH_LAST:
                 return None
             entry[1].epoch += 1
