@@ -832,6 +832,14 @@ int musa_aiter_hip_block_tables_check(const int64_t* block_tables, const int64_t
   return hipSuccess;
 }
 
+int musa_aiter_hip_exchange_capture_mode(int* mode) {
+  if (mode == nullptr) return hipErrorInvalidValue;
+  auto m = static_cast<hipStreamCaptureMode>(*mode);
+  const hipError_t err = hipThreadExchangeStreamCaptureMode(&m);
+  *mode = static_cast<int>(m);
+  return err;
+}
+
 int musa_aiter_hip_paged_tiles_noalloc(int scatter, int codec, int cache_elt, int lin_elt, int lin_dtype,
                                        void* key_cache, void* value_cache, void* key_linear, void* value_linear,
                                        const int64_t* slot_mapping, int64_t num_layers, int64_t num_tokens,

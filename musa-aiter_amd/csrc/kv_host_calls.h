@@ -63,6 +63,9 @@ int musa_aiter_hip_block_tables_check(const int64_t* block_tables, const int64_t
                                       int64_t report_words, int64_t* values, int64_t stamp, int64_t* out,
                                       void* stream);
 
+/* hipThreadExchangeStreamCaptureMode: *mode becomes this thread's capture mode, and receives the one before. */
+int musa_aiter_hip_exchange_capture_mode(int* mode);
+
 #ifdef __cplusplus
 }
 #endif

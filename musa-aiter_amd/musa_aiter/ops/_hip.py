@@ -97,6 +97,7 @@ _SIGNATURES: dict[str, list] = {
     "musa_aiter_hip_block_tables_check": [_c_void_p] * 2 + [_i64] * 4 + [_c_void_p, _i64, _c_void_p, _i64, _c_void_p,
                                                                         _c_void_p],
     "musa_aiter_hip_copy_rows_paged_checked": [ctypes.c_char_p, _c_void_p],  # musa_aiter_hip_copy_rows_paged_call, stream
+    "musa_aiter_hip_exchange_capture_mode": [ctypes.POINTER(ctypes.c_int)],
     "musa_aiter_hip_error_string": [_i32],
     "musa_aiter_hip_backend_name": [],
     "musa_aiter_hip_graph_claim_arrays": [],
@@ -305,6 +306,18 @@ def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int):
     return ctypes.addressof(c), entry
 
 
+@contextlib.contextmanager
+def _relaxed_capture_mode():
+    """Allocations of this thread do not break a graph capture that another one has under way."""
+    mode = ctypes.c_int(2)  # hipStreamCaptureModeRelaxed
+    exchange = fn("musa_aiter_hip_exchange_capture_mode")
+    check(exchange(ctypes.byref(mode)), "exchange_capture_mode")
+    try:
+        yield
+    finally:
+        check(exchange(ctypes.byref(mode)), "exchange_capture_mode")
+
+
 def _pinned_words(n: int) -> torch.Tensor:
     """``n`` zeroed words of pinned host memory (the device is named: torch.set_default_device must not move them)."""
     return torch.zeros(n, dtype=torch.int64, device="cpu", pin_memory=True)
@@ -355,8 +368,9 @@ class _CheckSet:
     __slots__ = ("report", "guard", "report_ptr", "values_ptr", "guard_ptr", "stamp")
 
     def __init__(self, device: torch.device):
-        self.report = _pinned_words(_REPORT_WORDS + _VALUE_WORDS)
-        self.guard = torch.zeros(1, dtype=torch.int64, device=device)
+        with _relaxed_capture_mode():
+            self.report = _pinned_words(_REPORT_WORDS + _VALUE_WORDS)
+            self.guard = torch.zeros(1, dtype=torch.int64, device=device)
         self.report_ptr, self.guard_ptr = self.report.data_ptr(), self.guard.data_ptr()
         self.values_ptr = self.report_ptr + 8 * _REPORT_WORDS
         self.stamp = 0

@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import threading
+
 import pytest
 import torch
 
@@ -104,3 +106,39 @@ def test_index_max_of_a_short_vector_after_a_long_one():
         long.fill_(entry[1] + 2)  # the stamp of the call after the long vector's
         assert _hip.index_max(long) == int(long[0])
         assert _hip.index_max(short) == 12345678
+
+
+def test_first_checked_call_of_a_stream_leaves_another_threads_capture_alone():
+    _, slots, caches, rows = _paged(200)
+    musa_aiter.kv_linear_to_paged(*rows, *caches, slots)
+    outs = [torch.empty_like(r) for r in rows]
+    x = torch.zeros(8, device=DEV)
+    stream, errors = torch.cuda.Stream(), []
+    torch.cuda.synchronize()
+
+    def work():
+        try:
+            with torch.cuda.stream(stream):
+                musa_aiter.kv_paged_to_linear(*caches, slots, out_k=outs[0], out_v=outs[1])
+        except Exception as e:  # reported by the main thread
+            errors.append(repr(e))
+
+    saved = dict(_hip._check_sets)
+    _hip._check_sets.clear()
+    graph = torch.cuda.CUDAGraph()
+    try:
+        with torch.cuda.graph(graph):  # in global mode: an allocation by another thread invalidates it
+            x += 1
+            thread = threading.Thread(target=work)
+            thread.start()
+            thread.join(30)
+            x += 1
+    finally:
+        _hip._check_sets.update(saved)
+    assert errors == [] and not thread.is_alive()
+    for _ in range(2):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert x.tolist() == [4.0] * 8
+    for r, o in zip(rows, outs):
+        assert torch.equal(r, o)
