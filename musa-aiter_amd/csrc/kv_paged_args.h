@@ -32,6 +32,7 @@ struct TileArgs {
   int32_t row_groups;          // tile kernel: row groups per block (grid x of a gather = tile * row_groups + group)
   int32_t check_groups;        // gather: workgroups at the front of each plane for check_share (0: none)
   int32_t scan_dupes;          // scatter: resolve repeated slots with a ScanTable instead of claim tags
+  int32_t short_run;           // wide gather: tiles whose runs average fewer tokens move token by token
   CallCheck check;             // report set: this kernel checks the call's slots and scales; guard set: one ahead did
 };
 
@@ -287,27 +288,70 @@ hipError_t launch_wide(const TileArgs& a, int64_t planes, bool lines, hipStream_
 // rows (at most 64) at a row pitch of block_size elements.
 constexpr int64_t kWideMaxBlockSize = 65536;
 
-// Scatters into wide blocks (64-column units) of at most 2,048 tokens x planes,
-// or 128 tokens of any number of planes, take kWideFewScatterTile-token tiles:
-// more, shorter waves.  One layer, 64-token pages: 1,000 tokens of whole
-// sequences 12.1 us (FP8) and 11.3 us (bf16) with 8-token tiles, 12.6 and 11.5
-// with 16; 4,000 tokens 19.0 us with 16, 16.0 with 64.
-constexpr int kWideFewScatterTile = 8;
-constexpr bool wide_scatter_few(int64_t tokens, int64_t planes) { return tokens * planes <= 2048 || tokens <= 128; }
-
-// Small calls on wide blocks that stay with the element kernel, whose one
-// element per thread spreads single tokens over more waves (tokens x planes;
-// one layer, 64-token pages, element against wide kernels).  Scatters: 256
-// single tokens 11.6 us against 13.2 (bf16) and 11.9 against 15.3 (FP8), 500
-// level for bf16 and 19.7 against 20.8 for FP8; at 128 the wide kernels win
-// (11.4 -> 8.6 and 12.0 -> 9.8 us), past 600 both wait for the memory's
-// partial-line writes, and whole sequences are level at 600 and faster from
-// 1,000 (16.4 -> 11.3 us).  Gathers: 128 single tokens 7.2 us against 8.3
-// (bf16) and 7.3 against 9.8 (FP8), 300 tokens of whole sequences level at 7
-// us, 2,000 20.3 -> 7.0 us.
-constexpr bool wide_scatter_wins(int64_t tokens, int64_t planes) {
-  return tokens * planes <= 256 || tokens * planes > 1200;
+// Rules of the wide blocks (64-column units; 32-bit copies 32-column ones).
+// What a call costs depends on the elements it moves, tokens x rows x planes,
+// hardly on how they split up: rows of 64 to 4,096 elements and 1 or 16 layers
+// were timed with single tokens, runs of 4 and 16 and whole sequences of 200,
+// caches read from HBM, device time of the C entry, claim pass included.  The
+// pairs below are us with the element kernel -> the wide kernels, rows of
+// 1,024 | of 64 elements, one layer.
+//
+// Calls of fewer elements stay with the element kernel, whose one element per
+// thread spreads a few tokens over more waves:
+//   16-bit gather, 768 Ki: single 29.9 -> 30.2 | 32.1 -> 33.8, runs of 4 11.4 ->
+//     13.2 | 11.1 -> 13.7, of 16 9.0 -> 7.6 | 8.3 -> 8.0, sequences 7.7 -> 5.4 |
+//     6.9 -> 5.7 (at 512 Ki single tokens and runs of 4 lose 4 us);
+//   32-bit gather, 512 Ki: 21.3 -> 21.7 | 21.8 -> 22.6, 9.0 -> 8.7 | 8.3 -> 9.2,
+//     7.5 -> 5.5 | 6.5 -> 5.8, 6.9 -> 5.2 | 5.9 -> 5.6;
+//   FP8 gather, 1,250 Ki: 29.9 -> 31.7 | 32.0 -> 34.4, 13.0 -> 13.2 | 12.6 ->
+//     14.2, 10.4 -> 7.6 | 10.2 -> 8.5, 9.3 -> 8.1 | 9.1 -> 8.6;
+//   16- and 32-bit scatter, 256 Ki (16-bit): 16.0 -> 16.4 | 18.7 -> 19.9, 9.1 ->
+//     9.1 | 10.1 -> 11.0, 7.1 -> 5.9 | 8.7 -> 7.3, 6.5 -> 5.3 | 8.5 -> 6.9;
+//   FP8 scatter, 1 Mi: 36.4 -> 39.3 | 39.1 -> 41.7, 18.2 -> 19.4 | 18.6 -> 20.4,
+//     13.6 -> 12.8 | 16.5 -> 14.2, 11.9 -> 11.9 | 14.8 -> 12.5.
+// Scatters of at most 256 tokens x planes move in one launch with the wide
+// kernels, which find repeated slots themselves, and in two with the element
+// kernel: 128 tokens of a sequence 6.5 -> 5.3 us.  FP8 ones gain nothing by it
+// (32 tokens in runs of 16, 5.8 -> 10.3 us: a partial piece is stored byte by
+// byte), unless the kernel checks the call's values too and the host waits for
+// one launch instead of two (a call of 48 single tokens 10.9 -> 10.6 us, of runs
+// of 16 10.8 -> 11.7).
+constexpr bool wide_scatter_wins(int cache_elt, int64_t tokens, int64_t planes, int64_t elems, bool checks) {
+  return (tokens * planes <= 256 && (cache_elt != 1 || checks)) ||
+         elems >= (cache_elt == 1 ? int64_t{1} << 20 : int64_t{1} << 18);
 }
-constexpr bool wide_gather_wins(int64_t tokens, int64_t planes) { return tokens * planes > 600; }
+constexpr bool wide_gather_wins(int cache_elt, int64_t elems) {
+  return elems >= (cache_elt == 1 ? int64_t{5} << 18 : cache_elt == 2 ? int64_t{3} << 18 : int64_t{1} << 19);
+}
+
+// Past these limits with fewer workgroups than CUs a wave's 64 (32) tokens are
+// a long serial chain while CUs idle (16-bit gathers of 384 single tokens of
+// 1,024 rows: 51.8 us, 30.2 in one-wave workgroups; FP8 gathers of 625: 57.0 us,
+// 31.7 with 16-token tiles), so such calls take smaller pieces.  (The figures
+// below are with the caches' lines still in the memory-side cache.)
+constexpr int64_t kWideFewGroups = 256;  // CUs
+// 16- and 32-bit gathers, one-wave workgroups: 1,536 tokens of 1,024 rows of
+// 16 bits 9.5 us in runs of 16 and 24.8 in runs of 4, 10.4 and 27.4 with four
+// waves; level past 4 Mi elements.  32-bit ones are level from 1 Mi.
+constexpr bool wide_gather_few(int cache_elt, int64_t elems) {
+  return elems < (cache_elt == 2 ? int64_t{1} << 22 : int64_t{1} << 20);
+}
+// ... and their tiles of runs shorter than this move token by token: runs of 4
+// of 8,192 tokens of 64 rows of 16 bits take 12.3 us with 6, 20.2 with 3; from 2
+// Mi elements (32-bit: 1 Mi) 3 is the faster one (1,536 tokens of 1,024 rows
+// 24.8 us).
+constexpr int wide_gather_short_run(int cache_elt, int64_t elems) {
+  return elems < (cache_elt == 2 ? int64_t{1} << 21 : int64_t{1} << 20) ? 6 : 3;
+}
+// Scatters, 8-token tiles (`groups`: workgroups of 64- or 32-token tiles): 512
+// tokens of 1,024 rows of 16 bits in runs of 4 14.4 us, 26.0 with 64-token
+// tiles; 2,048 45 against 39 us.  Calls of few tokens always take them.
+constexpr int kWideFewScatterTile = 8;
+constexpr bool wide_scatter_few(int64_t tokens, int64_t groups) { return groups < kWideFewGroups || tokens <= 128; }
+// FP8 scatters: 1,536 tokens of 1,024 rows in runs of 16 22.4 us with 8-token
+// tiles and 26.2 with 64, whole sequences 14.8 and 12.7.
+constexpr bool wide_quant_few(int64_t tokens, int64_t elems) {
+  return elems < (int64_t{3} << 20) || tokens <= 128;
+}
 
 }  // namespace kvhip

@@ -749,6 +749,8 @@ hipError_t launch_tile(const TileArgs& a0, int64_t planes, hipStream_t stream) {
 template <int ELT_C, int ELT_L, int CODEC, int LDT, bool SCATTER>
 hipError_t dispatch_bs(const TileArgs& a, int64_t bs, bool fast, int64_t planes, hipStream_t stream) {
   if (fast) {
+    const int64_t elems = a.num_tokens * a.nrows * planes;
+    [[maybe_unused]] const bool checks = a.check.report != nullptr;
     if constexpr (CODEC == kCopy) {
       // 16- and 32-bit copies: workgroup-cooperative kernel.
       static_assert(ELT_C == ELT_L, "copies keep the element type");
@@ -756,7 +758,8 @@ hipError_t dispatch_bs(const TileArgs& a, int64_t bs, bool fast, int64_t planes,
       if (bs == 16) return launch_tile<ELT_C, 16, SCATTER>(a, planes, stream);
       if (bs == 32) return launch_tile<ELT_C, 32, SCATTER>(a, planes, stream);
       if (bs % (128 / ELT_C) == 0 && bs <= kWideMaxBlockSize && 
-          (SCATTER ? wide_scatter_wins(a.num_tokens, planes) : wide_gather_wins(a.num_tokens, planes)))
+          (SCATTER ? wide_scatter_wins(ELT_C, a.num_tokens, planes, elems, checks)
+                   : wide_gather_wins(ELT_C, elems)))
         return launch_wide<ELT_C, SCATTER>(a, planes, linear_rows_whole_lines(a, ELT_C), stream);
     } else if constexpr (!SCATTER) {
       // FP8 dequant-gather: per-wave kernel (kv_paged_waves.hip), unless a chunk
@@ -764,14 +767,14 @@ hipError_t dispatch_bs(const TileArgs& a, int64_t bs, bool fast, int64_t planes,
       hipError_t err = hipErrorNotSupported;
       if (bs == 16) err = launch_wave_gather<ELT_C, ELT_L, CODEC, LDT, 16>(a, planes, stream);
       if (bs == 32) err = launch_wave_gather<ELT_C, ELT_L, CODEC, LDT, 32>(a, planes, stream);
-      if (bs % 64 == 0 && bs <= kWideMaxBlockSize && wide_gather_wins(a.num_tokens, planes))
+      if (bs % 64 == 0 && bs <= kWideMaxBlockSize && wide_gather_wins(ELT_C, elems))
         err = launch_wave_gather<ELT_C, ELT_L, CODEC, LDT, 64>(a, planes, stream);
       if (err != hipErrorNotSupported) return err;
     } else {
       // FP8 quant-store: per-wave kernel (kv_paged_waves.hip).
       if (bs == 16) return launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 16>(a, planes, stream);
       if (bs == 32) return launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 32>(a, planes, stream);
-      if (bs % 64 == 0 && bs <= kWideMaxBlockSize && wide_scatter_wins(a.num_tokens, planes))
+      if (bs % 64 == 0 && bs <= kWideMaxBlockSize && wide_scatter_wins(ELT_C, a.num_tokens, planes, elems, checks))
         return launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 64>(a, planes, stream);
     }
   }

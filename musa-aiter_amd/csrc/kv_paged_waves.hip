@@ -161,9 +161,12 @@ __device__ __forceinline__ void dequant_token_rows(const TileArgs& a, const uint
 
 // Launches of at most this many tokens take the TOKG instantiation; there a
 // tile takes dequant_token_rows when its runs average fewer than
-// kShortDequantRunTokens tokens and none goes on past the tile.
+// kShortDequantRunTokens tokens and none goes on past the tile.  (Wide blocks,
+// which take it at every size: runs of 4 of 4,096 tokens of 1,024 rows 46.5 us
+// with 3, 32.7 with 6.)
 constexpr int64_t kTokenDequantTokens = 256;
-constexpr int kShortDequantRunTokens = 3;
+template <int BS>
+constexpr int kShortDequantRunTokens = BS < 64 ? 3 : 6;
 
 // Slot window of a tile of TT tokens.  Units of at most 32 columns: lane i holds
 // token t0 - 1 + i (LEAD = 1), and every run that starts in the tile ends inside
@@ -352,7 +355,7 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wave_gather_kernel(const 
     const uint64_t owned = heads | (((cmask + (heads << 1)) ^ cmask) & cmask);
     const int nr = __builtin_popcountll(heads);
     const bool goes_on = TT == 64 ? (win.hi & 1ull) : (owned & ~window) != 0;
-    if (nr > 0 && !goes_on && __builtin_popcountll(owned) < nr * kShortDequantRunTokens) {
+    if (nr > 0 && !goes_on && __builtin_popcountll(owned) < nr * kShortDequantRunTokens<BS>) {
       constexpr int M = kChunkRows / kWave;
       static_assert(kChunkRows % kWave == 0, "whole rows per lane");
       int lut_off[M];
@@ -1047,7 +1050,13 @@ hipError_t launch_wave_gather(const TileArgs& a, int64_t planes, hipStream_t str
   }
   // (The form costs 64-column units nothing; the others compile it apart.)
   const bool tok = BS == 64 || a.num_tokens <= kTokenDequantTokens;
-  constexpr int tt = BS < 64 ? kTileTokens : BS;
+  // Wide blocks take 16-token tiles where their 64-token ones would leave CUs
+  // idle: 2,048 tokens of 1,024 rows (128 workgroups) 60.7 us with the element
+  // kernel, 66.6 with 64-token tiles, 62.2 with 16 (single tokens; runs of 4
+  // 34.4, 49.6 and 30.6); whole sequences level, and 15 against 10 us at 4,096.
+  constexpr int kGroupTokens = kWavesPerBlock * BS;
+  const bool few = BS == 64 && (a.num_tokens + kGroupTokens - 1) / kGroupTokens * planes * chunks < kWideFewGroups;
+  const int tt = BS < 64 || few ? kTileTokens : BS;
   const int64_t tiles = (a.num_tokens + tt - 1) / tt;
   const int64_t blocks = (tiles + kWavesPerBlock - 1) / kWavesPerBlock;
   if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
@@ -1062,7 +1071,13 @@ hipError_t launch_wave_gather(const TileArgs& a, int64_t planes, hipStream_t str
   // FP8 preload -0.3-0.5 %;
   // 5 per CU was 2-5 % slower, and staging the tiles through LDS with
   // whole-line loads gained 1.6 % on cfg 3 but lost 6 % on the dense preload.
-  if (whole_line_rows(a, ELT_L) && tok)
+  if (whole_line_rows(a, ELT_L) && few)
+    hipLaunchKernelGGL((paged_wave_gather_kernel<ELT_C, ELT_L, CODEC, LDT, BS, kBufWT, true, kTileTokens>), grid,
+                       dim3(kBlockThreads), kGatherLdsPad, stream, a);
+  else if (few)
+    hipLaunchKernelGGL((paged_wave_gather_kernel<ELT_C, ELT_L, CODEC, LDT, BS, kBufNT, true, kTileTokens>), grid,
+                       dim3(kBlockThreads), kGatherLdsPad, stream, a);
+  else if (whole_line_rows(a, ELT_L) && tok)
     hipLaunchKernelGGL((paged_wave_gather_kernel<ELT_C, ELT_L, CODEC, LDT, BS, kBufWT, true>), grid,
                        dim3(kBlockThreads), kGatherLdsPad, stream, a);
   else if (whole_line_rows(a, ELT_L))
@@ -1086,7 +1101,7 @@ hipError_t launch_wave_scatter(const TileArgs& a, int64_t planes, hipStream_t st
   // Block order when the claim tags are this call's inverse map and the tokens
   // cover a good share of the slots (as for the 16- and 32-bit scatter).
   const bool bm = a.owner != nullptr && a.owner_exclusive && a.num_tokens * 4 >= a.num_slots;
-  const bool few = BS == 64 && wide_scatter_few(a.num_tokens, planes);
+  const bool few = BS == 64 && wide_quant_few(a.num_tokens, a.num_tokens * a.nrows * planes);
   constexpr int kFewTile = BS < 64 ? kTileTokens : kWideFewScatterTile;
   const int tt = few ? kFewTile : BS < 64 ? kTileTokens : BS;
   const int64_t blocks =

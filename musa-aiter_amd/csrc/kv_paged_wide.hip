@@ -189,8 +189,7 @@ __device__ __forceinline__ void wide_token_rows(const TileArgs& a, const WaveChu
 
 // Tiles whose runs average fewer than this many tokens move token by token.
 constexpr int kWideShortRun = 6;
-// Gather tiles do below this (as the narrow kernels' gathers).
-constexpr int kWideShortGatherRun = 3;
+// (Gather tiles do below TileArgs::short_run, see wide_gather_short_run.)
 
 __device__ __forceinline__ int64_t slot_or_none(const TileArgs& a, int64_t t) {
   return t >= 0 && t < a.num_tokens ? slot_at(a, t) : -1;
@@ -198,34 +197,35 @@ __device__ __forceinline__ int64_t slot_or_none(const TileArgs& a, int64_t t) {
 
 __device__ __forceinline__ uint64_t low_bits(int64_t n) { return n >= 64 ? ~0ull : (1ull << n) - 1ull; }
 
-// True when the runs of a tile average fewer than kWideShortGatherRun tokens:
-// `v` marks its valid tokens, `c` those that continue the token before them.
-__device__ __forceinline__ bool short_gather_tile(uint64_t v, uint64_t c) {
-  return __builtin_popcountll(v) < kWideShortGatherRun * __builtin_popcountll(v & ~c);
+// True when the runs of a tile average fewer than short_run tokens: `v` marks
+// its valid tokens, `c` those that continue the token before them.
+__device__ __forceinline__ bool short_gather_tile(const TileArgs& a, uint64_t v, uint64_t c) {
+  return __builtin_popcountll(v) < a.short_run * __builtin_popcountll(v & ~c);
 }
 
-// Gather.  Grid: x = tile * row_groups + group of 4 chunks, y = plane.  A run
+// Gather.  Grid: x = tile * row_groups + group of WPB chunks (4, or 1 in small
+// launches: wide_gather_few), y = plane.  A run
 // is every token of the window whose slot lies in the head's unit at the
 // head's distance from its token, so tokens skipped in between (slot < 0) do
 // not cut it; its first token's tile moves it.  A tile of short runs instead
 // moves its own tokens, no more, and the tile after it knows that from the
 // same slots.
-template <int ELT, bool XCD, int STP>
-__global__ __launch_bounds__(kBlockThreads) void paged_wide_gather_kernel(const TileArgs a) {
+template <int ELT, bool XCD, int STP, int WPB = kWavesPerBlock>
+__global__ __launch_bounds__(WPB * kWave) void paged_wide_gather_kernel(const TileArgs a) {
   using W = Wide<ELT>;
   constexpr int TT = W::UC;
   const int lane = lane_id();
   WgXyz wg = xcd_contiguous_wg<XCD>();
   const uint32_t ahead = static_cast<uint32_t>(a.check_groups);
   if (wg.x < ahead) {
-    check_share<kBlockThreads>(a, wg.x, wg.y);
+    check_share<WPB * kWave>(a, wg.x, wg.y);
     return;
   }
   wg.x -= ahead;
   const uint32_t tile = wg.x / static_cast<uint32_t>(a.row_groups);
   const uint32_t group = wg.x - tile * static_cast<uint32_t>(a.row_groups);
   const int64_t t0 = static_cast<int64_t>(tile) * TT;
-  const WaveChunk w = wave_chunk<ELT>(a, wg.y, static_cast<int64_t>(group) * kWavesPerBlock + wave_in_block());
+  const WaveChunk w = wave_chunk<ELT>(a, wg.y, static_cast<int64_t>(group) * WPB + wave_in_block());
   if (w.rows == 0) return;
 
   const int64_t s = slot_or_none(a, t0 + lane);
@@ -243,8 +243,8 @@ __global__ __launch_bounds__(kBlockThreads) void paged_wide_gather_kernel(const 
   auto continues = [&](int64_t slot, int64_t before) { return slot == before + 1 && (slot & (W::UC - 1)) != 0; };
   const uint64_t c = ballot(valid && lane > 0 && continues(s, s_prev));
   const uint64_t c_pre = ballot(valid_pre && lane > kWave - TT && continues(s_pre, s_pre_prev));
-  const bool pre_short = short_gather_tile(ballot(valid_pre) >> (kWave - TT), c_pre >> (kWave - TT));
-  if (short_gather_tile(pending, c)) {
+  const bool pre_short = short_gather_tile(a, ballot(valid_pre) >> (kWave - TT), c_pre >> (kWave - TT));
+  if (short_gather_tile(a, pending, c)) {
     wide_token_rows<ELT, false, TT>(a, w, s, pending, t0);
     pending = 0;
   }
@@ -405,9 +405,14 @@ hipError_t launch_wide(const TileArgs& a0, int64_t planes, bool lines, hipStream
   if (a0.check.report != nullptr && (SCATTER ? a0.scan_dupes == 0 : a0.check.words == 0)) return hipErrorNotSupported;
   TileArgs a = a0;
   const int64_t chunks = (a.nrows + W::UC - 1) / W::UC;
-  const int64_t groups = (chunks + kWavesPerBlock - 1) / kWavesPerBlock;
-  const bool few = SCATTER && wide_scatter_few(a.num_tokens, planes);
-  const int tt = few ? kWideFewScatterTile : W::UC;
+  const int64_t elems = a.num_tokens * a.nrows * planes;
+  const int64_t unit_tiles = (a.num_tokens + W::UC - 1) / W::UC;
+  const int64_t unit_groups = unit_tiles * ((chunks + kWavesPerBlock - 1) / kWavesPerBlock) * planes;
+  const bool few = SCATTER ? wide_scatter_few(a.num_tokens, unit_groups) : wide_gather_few(ELT, elems);
+  a.short_run = wide_gather_short_run(ELT, elems);
+  const int wpb = few && !SCATTER ? 1 : kWavesPerBlock;
+  const int64_t groups = (chunks + wpb - 1) / wpb;
+  const int tt = SCATTER && few ? kWideFewScatterTile : W::UC;
   // Destination order under the narrow scatter's rule: the claim tags are this
   // call's inverse map and the tokens cover a quarter of the slots.
   const bool by_unit = SCATTER && a.owner != nullptr && a.owner_exclusive && a.num_tokens * 4 >= a.num_slots &&
@@ -415,11 +420,11 @@ hipError_t launch_wide(const TileArgs& a0, int64_t planes, bool lines, hipStream
   const int64_t tiles = by_unit ? a.num_slots / W::UC : (a.num_tokens + tt - 1) / tt;
   if (groups > 0x7FFFFFFF || tiles > 0x7FFFFFFF / groups) return hipErrorInvalidValue;
   a.row_groups = static_cast<int32_t>(groups);
-  const int64_t extra = SCATTER ? 0 : (a.check.words + kWavesPerBlock - 1) / kWavesPerBlock;
+  const int64_t extra = SCATTER ? 0 : (a.check.words + wpb - 1) / wpb;
   a.check_groups = static_cast<int32_t>(extra);
   if (tiles * groups > 0x7FFFFFFF - extra) return hipErrorInvalidValue;
   const dim3 grid(static_cast<uint32_t>(tiles * groups + extra), static_cast<uint32_t>(planes));
-  const dim3 block(kBlockThreads);
+  const dim3 block(static_cast<uint32_t>(wpb * kWave));
   const bool xcd = planes >= kWideXcdPlanes && int64_t{grid.x} * planes <= int64_t{0xFFFFFFFF};
   if constexpr (SCATTER) {
     if (by_unit && xcd)
@@ -430,6 +435,9 @@ hipError_t launch_wide(const TileArgs& a0, int64_t planes, bool lines, hipStream
       hipLaunchKernelGGL((paged_wide_scatter_kernel<ELT, kWideFewScatterTile>), grid, block, 0, stream, a);
     else
       hipLaunchKernelGGL((paged_wide_scatter_kernel<ELT, W::UC>), grid, block, 0, stream, a);
+  } else if (few) {
+    if (lines) hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, false, kBufWT, 1>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, false, kBufNT, 1>), grid, block, 0, stream, a);
   } else {
     if (xcd && lines)
       hipLaunchKernelGGL((paged_wide_gather_kernel<ELT, true, kBufWT>), grid, block, 0, stream, a);

@@ -130,3 +130,49 @@ def test_wide_fp8_blocks_match_oracle(fmt, lin, bs, nh, hd, tokens, kind):
         want = cache.numpy().copy()
         ko.linear_to_paged_fp8(t.to(torch.float32).numpy(), want, slots, scale.numpy(), fmt)
         assert np.array_equal(cache_d.cpu().numpy(), want)
+
+
+def _fp8_round_trip(layers, nh, hd, bs, slots, nb):
+    gen = torch.Generator().manual_seed(layers + len(slots))
+    x = [(torch.randn((layers, len(slots), nh, hd), generator=gen) * 3).to(torch.bfloat16) for _ in range(2)]
+    scales = [torch.rand((layers, nh), generator=gen) * 0.02 + 0.001 for _ in range(2)]
+    caches = [torch.randint(0, 256, (layers, nb, nh, hd, bs), dtype=torch.uint8, generator=gen) for _ in range(2)]
+    s_d, scales_d, caches_d = torch.from_numpy(slots).to(DEV), [s.to(DEV) for s in scales], [c.to(DEV) for c in caches]
+    got = musa_aiter.kv_paged_fp8_to_linear_multi_layer(*caches_d, s_d, *scales_d, out_dtype=torch.bfloat16)
+    musa_aiter.kv_linear_to_paged_fp8_multi_layer(*(t.to(DEV) for t in x), *caches_d, s_d, *scales_d)
+    for out, t, cache, cache_d, scale in zip(got, x, caches, caches_d, scales):
+        for layer in range(layers):
+            assert np.array_equal(bits(out[layer]), ko.paged_fp8_to_linear(cache[layer].numpy(), slots,
+                                                                           scale[layer].numpy(), "e4m3", "bfloat16"))
+            want = cache[layer].numpy().copy()
+            ko.linear_to_paged_fp8(t[layer].to(torch.float32).numpy(), want, slots, scale[layer].numpy(), "e4m3")
+            assert np.array_equal(cache_d[layer].cpu().numpy(), want)
+
+
+# By elements moved (tokens x rows x planes) a call on wide blocks takes the element kernel, the wide kernels'
+# forms for small launches (one-wave workgroups or 16-token tiles for gathers, 8-token tiles for scatters) or
+# their large ones.  About 540 tokens of every run shape: with 2,048 rows the forms change between one and three
+# layers, 17 layers take the order of many planes; a cache of 12 blocks is scattered in destination order, one of
+# 40 in token order.
+@pytest.mark.parametrize("layers, nh, hd", [(1, 16, 128), (2, 16, 128), (3, 16, 128), (1, 17, 120), (2, 17, 120),
+                                            (3, 17, 120), (1, 8, 128), (17, 8, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.uint8])
+@pytest.mark.parametrize("nb", [12, 40])
+def test_wide_forms_by_elements_match_oracle(layers, nh, hd, dtype, nb):
+    slots = tricky_slots(np.random.default_rng(layers), 12, 64)
+    if dtype is torch.uint8:
+        _fp8_round_trip(layers, nh, hd, 64, slots, nb)
+    else:
+        _round_trip(dtype, layers, nh, hd, 64, slots, nb)
+
+
+# One layer of 1,024 rows: 128 tokens are 2**18 elements, the limits 128 to 2,048 tokens.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.uint8])
+@pytest.mark.parametrize("tokens", [128, 256, 384, 512, 640, 1024, 1536, 2048])
+@pytest.mark.parametrize("below", [0, 1])
+def test_wide_calls_at_the_limits_match_oracle(dtype, tokens, below):
+    slots, nb = make_slots("skips", np.random.default_rng(tokens), block_size=64, tokens=tokens - below)
+    if dtype is torch.uint8:
+        _fp8_round_trip(1, 8, 128, 64, slots, nb)
+    else:
+        _round_trip(dtype, 1, 8, 128, 64, slots, nb)
