@@ -774,8 +774,10 @@ hipError_t dispatch_bs(const TileArgs& a, int64_t bs, bool fast, int64_t planes,
       // FP8 quant-store: per-wave kernel (kv_paged_waves.hip).
       if (bs == 16) return launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 16>(a, planes, stream);
       if (bs == 32) return launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 32>(a, planes, stream);
-      if (bs % 64 == 0 && bs <= kWideMaxBlockSize && wide_scatter_wins(ELT_C, a.num_tokens, planes, elems, checks))
-        return launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 64>(a, planes, stream);
+      if (bs % 64 == 0 && bs <= kWideMaxBlockSize && wide_scatter_wins(ELT_C, a.num_tokens, planes, elems, checks)) {
+        const hipError_t err = launch_wave_scatter<ELT_C, ELT_L, CODEC, LDT, 64>(a, planes, stream);
+        if (err != hipErrorNotSupported) return err;
+      }
     }
   }
   // The element kernel checks claim tags only: a call without them takes the

@@ -1034,12 +1034,16 @@ static_assert(4 * (kGatherLdsPad + kLutHeads * 256 * 2) > 160 * 1024 &&
                   3 * (kGatherLdsPad + kLutHeads * 256 * 4 + 16) <= 160 * 1024,
               "3 workgroups per CU, not 4");
 
+// Row chunks are grid z.  Wide blocks with more (rows of millions of elements)
+// go to the element kernel.
+constexpr int64_t kMaxChunks = 65535;
+
 template <int ELT_C, int ELT_L, int CODEC, int LDT, int BS>
 hipError_t launch_wave_gather(const TileArgs& a, int64_t planes, hipStream_t stream) {
   using W = WaveShape<ELT_C, ELT_L, BS>;
   if (a.check.report != nullptr && (BS == 64 || a.num_tokens > kTokenDequantTokens)) return hipErrorNotSupported;
   const int64_t chunks = (a.nrows + W::kChunkRows - 1) / W::kChunkRows;
-  if (chunks > 65535) return hipErrorInvalidValue;
+  if (chunks > kMaxChunks) return BS == 64 ? hipErrorNotSupported : hipErrorInvalidValue;
   if (CODEC != kCopy && a.scale_mode != 0) {
     // Every chunk's heads must fit the workgroup's decode tables.
     for (int64_t z = 0; z < chunks; ++z) {
@@ -1097,7 +1101,7 @@ hipError_t launch_wave_scatter(const TileArgs& a, int64_t planes, hipStream_t st
   using W = ScatterShape<ELT_L, BS>;
   if (a.check.report != nullptr && !a.scan_dupes) return hipErrorNotSupported;
   const int64_t chunks = (a.nrows + W::kChunkRows * W::kWaveChunks - 1) / (W::kChunkRows * W::kWaveChunks);
-  if (chunks > 65535) return hipErrorInvalidValue;
+  if (chunks > kMaxChunks) return BS == 64 ? hipErrorNotSupported : hipErrorInvalidValue;
   // Block order when the claim tags are this call's inverse map and the tokens
   // cover a good share of the slots (as for the 16- and 32-bit scatter).
   const bool bm = a.owner != nullptr && a.owner_exclusive && a.num_tokens * 4 >= a.num_slots;

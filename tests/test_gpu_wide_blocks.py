@@ -176,3 +176,22 @@ def test_wide_calls_at_the_limits_match_oracle(dtype, tokens, below):
         _fp8_round_trip(1, 8, 128, 64, slots, nb)
     else:
         _round_trip(dtype, 1, 8, 128, 64, slots, nb)
+
+
+def test_wide_fp8_blocks_with_more_row_chunks_than_a_grid_holds():
+    # 32,769 heads of 128: 65,538 chunks of 64 rows, past the per-wave kernels' grid; the element kernel moves them.
+    nh, hd, slots = 32769, 128, np.array([5, 40])
+    gen = torch.Generator().manual_seed(1)
+    x = [torch.randn((2, nh, hd), generator=gen) for _ in range(2)]
+    scales = [torch.tensor(0.02), torch.tensor(0.03)]
+    caches_d = [torch.zeros((1, nh, hd, 64), dtype=torch.uint8, device=DEV) for _ in range(2)]
+    s_d, scales_d = torch.from_numpy(slots).to(DEV), [s.to(DEV) for s in scales]
+    musa_aiter.kv_linear_to_paged_fp8(*(t.to(DEV) for t in x), *caches_d, s_d, *scales_d)
+    got = musa_aiter.kv_paged_fp8_to_linear(*caches_d, s_d, *scales_d, out_dtype=torch.float32)
+    for t, cache_d, out, scale in zip(x, caches_d, got, scales):
+        # One-slot blocks: the same codes without the 62 columns that no token writes.
+        want = np.zeros((2, nh, hd, 1), np.uint8)
+        ko.linear_to_paged_fp8(t.numpy(), want, np.array([0, 1]), scale.numpy(), "e4m3")
+        assert np.array_equal(cache_d[0, :, :, slots].permute(2, 0, 1).cpu().numpy(), want[..., 0])
+        assert int((cache_d != 0).sum()) == int((want != 0).sum())
+        assert np.array_equal(bits(out), ko.paged_fp8_to_linear(want, np.array([0, 1]), scale.numpy(), "e4m3", "float32"))
