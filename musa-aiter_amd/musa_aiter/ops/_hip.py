@@ -434,7 +434,7 @@ def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, l
 _paged_entry: list[int] = []  # address of musa_aiter_hip_paged_tiles_checked
 
 
-def paged_native(key_cache, value_cache, linear, slots, scales, *, layered: bool, codec: int, out_dtype=None):
+def paged_native(op, key_cache, value_cache, linear, slots, scales, *, layered: bool, codec: int, out_dtype=None):
     """One checked paged call whose argument checks the host module makes too: a scatter of the rows ``linear``,
     or with ``linear`` None a gather into new tensors (of ``out_dtype``, or the caches' type).
 
@@ -474,7 +474,7 @@ def paged_native(key_cache, value_cache, linear, slots, scales, *, layered: bool
         del entry
     if rc == h.NOT_TAKEN or rc == _REFUSED:
         return None
-    check(rc, "paged call")
+    check(rc, op)
     return True if scatter else (k, v)
 
 

@@ -357,7 +357,7 @@ def kv_paged_to_linear(
     """
     op = "kv_paged_to_linear"
     if out_k is None and out_v is None and fill_skipped == "zeros":
-        got = _hip.paged_native(key_cache, value_cache, None, slot_mapping, None, layered=False, codec=_CODEC_COPY)
+        got = _hip.paged_native(op, key_cache, value_cache, None, slot_mapping, None, layered=False, codec=_CODEC_COPY)
         if got is not None:
             _emit(op, key_cache, "gfx950 paged->linear tile gather")
             return got
@@ -392,7 +392,7 @@ def kv_paged_to_linear_multi_layer(
     """Gather stacked caches ``[L, NB, H, D, BS]`` into ``[L, T, H, D]`` in one launch (reference :3209-3309)."""
     op = "kv_paged_to_linear_multi_layer"
     if out_k is None and out_v is None and fill_skipped == "zeros":
-        got = _hip.paged_native(key_cache, value_cache, None, slot_mapping, None, layered=True, codec=_CODEC_COPY)
+        got = _hip.paged_native(op, key_cache, value_cache, None, slot_mapping, None, layered=True, codec=_CODEC_COPY)
         if got is not None:
             _emit(op, key_cache, f"gfx950 paged->linear tile gather ({key_cache.shape[0]} layers, one launch)")
             return got
@@ -437,7 +437,7 @@ def kv_linear_to_paged(
     token in token order.
     """
     op = "kv_linear_to_paged"
-    if _hip.paged_native(key_cache, value_cache, (key_linear, value_linear), slot_mapping, None, layered=False,
+    if _hip.paged_native(op, key_cache, value_cache, (key_linear, value_linear), slot_mapping, None, layered=False,
                          codec=_CODEC_COPY):
         _emit(op, key_linear, "gfx950 linear->paged tile scatter")
         return
@@ -471,7 +471,7 @@ def kv_linear_to_paged_multi_layer(
 ) -> None:
     """Scatter ``[L, T, H, D]`` into stacked caches in one launch (reference :3382-3457)."""
     op = "kv_linear_to_paged_multi_layer"
-    if _hip.paged_native(key_cache, value_cache, (key_linear, value_linear), slot_mapping, None, layered=True,
+    if _hip.paged_native(op, key_cache, value_cache, (key_linear, value_linear), slot_mapping, None, layered=True,
                          codec=_CODEC_COPY):
         _emit(op, key_linear, f"gfx950 linear->paged tile scatter ({key_cache.shape[0]} layers, one launch)")
         return
@@ -775,7 +775,7 @@ def kv_linear_to_paged_fp8(
     """
     op = "kv_linear_to_paged_fp8"
     codec = _NATIVE_FORMATS.get(fp8_format)
-    if codec is not None and _hip.paged_native(key_cache_fp8, value_cache_fp8, (key_linear, value_linear),
+    if codec is not None and _hip.paged_native(op, key_cache_fp8, value_cache_fp8, (key_linear, value_linear),
                                                slot_mapping, (k_scale, v_scale), layered=False, codec=codec):
         _emit(op, key_linear, f"gfx950 fused {fp8_format.upper()} quantize scatter")
         return
@@ -819,7 +819,7 @@ def kv_paged_fp8_to_linear(
     op = "kv_paged_fp8_to_linear"
     codec = _NATIVE_FORMATS.get(fp8_format)
     if codec is not None and out_k is None and out_v is None:
-        got = _hip.paged_native(key_cache_fp8, value_cache_fp8, None, slot_mapping, (k_scale, v_scale),
+        got = _hip.paged_native(op, key_cache_fp8, value_cache_fp8, None, slot_mapping, (k_scale, v_scale),
                                 layered=False, codec=codec, out_dtype=out_dtype)
         if got is not None:
             _emit(op, key_cache_fp8, f"gfx950 fused {fp8_format.upper()} dequantize gather")
@@ -862,7 +862,7 @@ def kv_linear_to_paged_fp8_multi_layer(
     """Multi-layer FP8 quantize scatter; scales scalar, ``[H]`` or ``[L, H]`` (reference :2304-2347)."""
     op = "kv_linear_to_paged_fp8_multi_layer"
     codec = _NATIVE_FORMATS.get(fp8_format)
-    if codec is not None and _hip.paged_native(key_cache_fp8, value_cache_fp8, (key_linear, value_linear),
+    if codec is not None and _hip.paged_native(op, key_cache_fp8, value_cache_fp8, (key_linear, value_linear),
                                                slot_mapping, (k_scale, v_scale), layered=True, codec=codec):
         _emit(op, key_linear, f"gfx950 fused {fp8_format.upper()} quantize scatter ({key_cache_fp8.shape[0]} layers)")
         return
@@ -909,7 +909,7 @@ def kv_paged_fp8_to_linear_multi_layer(
     op = "kv_paged_fp8_to_linear_multi_layer"
     codec = _NATIVE_FORMATS.get(fp8_format)
     if codec is not None and out_k is None and out_v is None:
-        got = _hip.paged_native(key_cache_fp8, value_cache_fp8, None, slot_mapping, (k_scale, v_scale),
+        got = _hip.paged_native(op, key_cache_fp8, value_cache_fp8, None, slot_mapping, (k_scale, v_scale),
                                 layered=True, codec=codec, out_dtype=out_dtype)
         if got is not None:
             _emit(op, key_cache_fp8, f"gfx950 fused {fp8_format.upper()} dequantize gather ({key_cache_fp8.shape[0]} layers)")

@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import threading
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -142,3 +143,24 @@ def test_first_checked_call_of_a_stream_leaves_another_threads_capture_alone():
     assert x.tolist() == [4.0] * 8
     for r, o in zip(rows, outs):
         assert torch.equal(r, o)
+
+
+@pytest.mark.parametrize("layers", [1, 2])
+def test_failed_launches_name_the_operation(monkeypatch, layers):
+    # The host module's status is reported under the name of the call, as the Python layer's own launches are.
+    suffix = "_multi_layer" if layers > 1 else ""
+    lead = (layers,) if layers > 1 else ()
+    caches = [torch.zeros(lead + (4, NH, HD, BS), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    rows = [torch.zeros(lead + (5, NH, HD), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    codes = [torch.zeros(lead + (4, NH, HD, BS), dtype=torch.uint8, device=DEV) for _ in range(2)]
+    slots, scale = torch.arange(5, device=DEV), torch.ones(NH, device=DEV)
+    calls = {"kv_paged_to_linear": (*caches, slots), "kv_linear_to_paged": (*rows, *caches, slots),
+             "kv_paged_fp8_to_linear": (*codes, slots, scale, scale),
+             "kv_linear_to_paged_fp8": (*rows, *codes, slots, scale, scale)}
+    for name, args in calls.items():
+        getattr(musa_aiter, name + suffix)(*args)  # the stream's state exists from here on
+    failed = SimpleNamespace(paged_call=lambda *_: (1, None, None), NOT_TAKEN=_hip.host().NOT_TAKEN)
+    monkeypatch.setattr(_hip, "host", lambda: failed)
+    for name, args in calls.items():
+        with pytest.raises(_hip.HipBackendError, match=f"^{name + suffix}: HIP launch failed with error 1 "):
+            getattr(musa_aiter, name + suffix)(*args)
