@@ -258,3 +258,31 @@ def test_reference_c_entries_through_ctypes():
         assert dec_fn(out.data_ptr(), book.to(DEV).data_ptr(), dec.data_ptr(), n, None) == 0
         torch.cuda.synchronize()
         np.testing.assert_array_equal(_bits(dec.cpu().numpy()), _bits(book.numpy()[want.astype(np.int64)]))
+
+
+@pytest.mark.parametrize("numel", [1, 1000, 70_001, 5_000_000])  # one range workgroup, a few, the most
+@pytest.mark.parametrize("ws_bytes", [16384, 16384 + 2047, 40000, 75776 - 1])
+def test_encode_in_a_smaller_workspace(numel, ws_bytes):
+    # The entry takes any workspace from 16,384 bytes on, with fewer copies of the bin counters: the same codes,
+    # codebook and CDF, and nothing written past its end.
+    x = torch.randn(numel, device=DEV, dtype=torch.float32).to(torch.bfloat16)
+    want = musa_aiter.kv_cachegen_encode(x, num_bins=200)
+    guard = 4096
+    workspace = torch.full((ws_bytes + guard,), 0xA5, dtype=torch.uint8, device=DEV)
+    got = [torch.empty_like(t) for t in want]
+    rc = _hip.fn("musa_aiter_hip_cachegen_encode")(
+        x.data_ptr(), 2, numel, 200, 0, *(t.data_ptr() for t in got), workspace.data_ptr(), ws_bytes,
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
+    assert bool((workspace[ws_bytes:] == 0xA5).all())
+
+
+def test_encode_refuses_a_workspace_that_is_too_small():
+    x = torch.zeros(100, device=DEV)
+    out = torch.empty(1024, dtype=torch.uint8, device=DEV)
+    rc = _hip.fn("musa_aiter_hip_cachegen_encode")(
+        x.data_ptr(), 0, 100, 16, 0, out.data_ptr(), out.data_ptr(), out.data_ptr(), out.data_ptr(), 16383,
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 1  # hipErrorInvalidValue, before any launch
