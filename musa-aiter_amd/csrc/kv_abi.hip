@@ -1467,6 +1467,46 @@ int musa_aiter_hicache_transfer_abi_version() { return 1; }
 // the host; either side may use paged row addressing.  Tokens whose source or
 // destination index lies outside [0, rows) are skipped; with `dedupe` a
 // destination row named by several tokens keeps the last one.
+int musa_aiter_hip_copy_rows_paged(const uint64_t* src_planes, const uint64_t* dst_planes, int64_t num_planes,
+                                   const int64_t* src_idx, const int64_t* dst_idx, int64_t num_tokens,
+                                   int64_t src_rows, int64_t dst_rows, int64_t row_bytes, int64_t src_stride,
+                                   int64_t dst_stride, int64_t src_page_rows, int64_t src_page_stride,
+                                   int64_t dst_page_rows, int64_t dst_page_stride, int dedupe,
+                                   const musa_aiter_hip_claims* claims, void* stream) {
+  if (num_tokens <= 0 || num_planes <= 0 || row_bytes <= 0) return hipSuccess;
+  if (src_idx == nullptr || dst_idx == nullptr) return hipErrorInvalidValue;
+  RowCopyParams p{};
+  p.src_planes = src_planes;
+  p.dst_planes = dst_planes;
+  p.num_planes = num_planes;
+  p.src_idx = src_idx;
+  p.dst_idx = dst_idx;
+  p.num_tokens = num_tokens;
+  p.num_rows_out = num_tokens;
+  p.src_rows = src_rows;
+  p.dst_rows = dst_rows;
+  p.row_bytes = row_bytes;
+  p.src_stride = src_stride;
+  p.dst_stride = dst_stride;
+  p.src_page_rows = src_page_rows;
+  p.src_page_stride = src_page_stride;
+  p.dst_page_rows = dst_page_rows;
+  p.dst_page_stride = dst_page_stride;
+  if (dedupe) {
+    kvhip::ClaimSource src;
+    src.idx = dst_idx;
+    src.src_idx = src_idx;
+    src.src_rows = src_rows;
+    hipError_t err =
+        prepare_claims(src, num_tokens, dst_rows, as_stream(stream), claims, &p.owner, &p.epoch, &p.owner_exclusive);
+    if (err != hipSuccess) return err;
+  }
+  return kvhip::launch_row_copy(p, as_stream(stream));
+}
+
+// The same behind a check of both index vectors, for plain dedupe calls: an entry
+// outside [low, src_rows) or [low, dst_rows) refuses the whole call, and nothing
+// moves; negative entries skip their pair.
 int musa_aiter_hip_copy_rows_paged_checked(const musa_aiter_hip_copy_rows_paged_call* call, void* stream) {
   if (call == nullptr) return hipErrorInvalidValue;
   const musa_aiter_hip_copy_rows_paged_call& c = *call;
@@ -1513,43 +1553,6 @@ int musa_aiter_hip_copy_rows_paged_checked(const musa_aiter_hip_copy_rows_paged_
   err = await_verdict(c.report, groups, c.stamp, as_stream(stream), &refused);
   if (err != hipSuccess || refused) return err != hipSuccess ? static_cast<int>(err) : MUSA_AITER_HIP_REFUSED;
   return moved;
-}
-
-int musa_aiter_hip_copy_rows_paged(const uint64_t* src_planes, const uint64_t* dst_planes, int64_t num_planes,
-                                   const int64_t* src_idx, const int64_t* dst_idx, int64_t num_tokens,
-                                   int64_t src_rows, int64_t dst_rows, int64_t row_bytes, int64_t src_stride,
-                                   int64_t dst_stride, int64_t src_page_rows, int64_t src_page_stride,
-                                   int64_t dst_page_rows, int64_t dst_page_stride, int dedupe,
-                                   const musa_aiter_hip_claims* claims, void* stream) {
-  if (num_tokens <= 0 || num_planes <= 0 || row_bytes <= 0) return hipSuccess;
-  if (src_idx == nullptr || dst_idx == nullptr) return hipErrorInvalidValue;
-  RowCopyParams p{};
-  p.src_planes = src_planes;
-  p.dst_planes = dst_planes;
-  p.num_planes = num_planes;
-  p.src_idx = src_idx;
-  p.dst_idx = dst_idx;
-  p.num_tokens = num_tokens;
-  p.num_rows_out = num_tokens;
-  p.src_rows = src_rows;
-  p.dst_rows = dst_rows;
-  p.row_bytes = row_bytes;
-  p.src_stride = src_stride;
-  p.dst_stride = dst_stride;
-  p.src_page_rows = src_page_rows;
-  p.src_page_stride = src_page_stride;
-  p.dst_page_rows = dst_page_rows;
-  p.dst_page_stride = dst_page_stride;
-  if (dedupe) {
-    kvhip::ClaimSource src;
-    src.idx = dst_idx;
-    src.src_idx = src_idx;
-    src.src_rows = src_rows;
-    hipError_t err =
-        prepare_claims(src, num_tokens, dst_rows, as_stream(stream), claims, &p.owner, &p.epoch, &p.owner_exclusive);
-    if (err != hipSuccess) return err;
-  }
-  return kvhip::launch_row_copy(p, as_stream(stream));
 }
 
 // The reference kernel's contract: for every item whose two page indices are
