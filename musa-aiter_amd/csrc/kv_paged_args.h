@@ -9,6 +9,7 @@
 namespace kvhip {
 
 struct TileArgs {
+  CallCheck check;             // report set: this kernel checks the call's slots and scales; guard set: one ahead did
   uint8_t* cache[2];
   uint8_t* lin[2];
   const int64_t* slots;
@@ -33,7 +34,6 @@ struct TileArgs {
   int32_t check_groups;        // gather: workgroups at the front of each plane for check_share (0: none)
   int32_t scan_dupes;          // scatter: resolve repeated slots with a ScanTable instead of claim tags
   int32_t short_run;           // wide gather: tiles whose runs average fewer tokens move token by token
-  CallCheck check;             // report set: this kernel checks the call's slots and scales; guard set: one ahead did
 };
 
 // Slot of token t: the slot vector's entry, or the block-table slot of the
