@@ -266,17 +266,20 @@ _stream_locks: dict[tuple[int, int], threading.Lock] = {}
 
 
 def _stream_key(device: torch.device, stream: ctypes.c_void_p) -> tuple[int, int]:
-    return (device.index if device.index is not None else torch.cuda.current_device(), stream.value or 0)
+    index = device.index
+    return (torch.cuda.current_device() if index is None else index, stream.value or 0)
+
+
+def _key_lock(key: tuple[int, int]) -> threading.Lock:
+    return _stream_locks.get(key) or _stream_locks.setdefault(key, threading.Lock())
 
 
 def stream_lock(device: torch.device, stream: ctypes.c_void_p) -> threading.Lock:
     """The lock to hold from claims_for to the return of the call that uses the claims."""
-    key = _stream_key(device, stream)
-    found = _stream_locks.get(key)
-    return found if found is not None else _stream_locks.setdefault(key, threading.Lock())
+    return _key_lock(_stream_key(device, stream))
 
 
-def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int):
+def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int, key: tuple[int, int] | None = None):
     """The claims of one scatter with ``rows`` destination rows on ``stream``: returns the address of a
     musa_aiter_hip_claims to pass and the objects to keep alive until the call has returned.  The caller
     holds the stream's lock.
@@ -290,7 +293,7 @@ def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int):
         tags = torch.empty(rows, dtype=torch.int64, device=device)
         c = _Claims(tags.data_ptr(), rows, 0, 0)
         return ctypes.addressof(c), (tags, c)
-    key = _stream_key(device, stream)
+    key = key or _stream_key(device, stream)
     entry = _claim_sets.get(key)
     if entry is None or entry[1].capacity < rows:
         have = entry[1].capacity if entry is not None else 0
@@ -383,9 +386,9 @@ _uses = itertools.count(1)
 _last_use: dict[tuple[int, int], int] = {}
 
 
-def _check_set(device: torch.device, stream: int) -> _CheckSet:
+def _check_set(device: torch.device, stream: int, key: tuple[int, int] | None = None) -> _CheckSet:
     """The check set of a (device, stream), whose lock the caller holds."""
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
+    key = key or (device.index if device.index is not None else torch.cuda.current_device(), stream)
     found = _check_sets.get(key)
     if found is None:
         with _check_sets_lock:
@@ -413,9 +416,10 @@ def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, l
     device = key_cache.device
     with on_device(device):
         stream = stream_ptr(device)
-        with stream_lock(device, stream):
-            checks = _check_set(device, stream.value or 0)
-            claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter else (0, None))
+        key = _stream_key(device, stream)
+        with _key_lock(key):
+            checks = _check_set(device, key[1], key)
+            claims, keep = (claims_for(device, stream, num_blocks * block_size, key) if scatter else (0, None))
             checks.stamp += 1
             call = _PAGED_TILES_CALL.pack(
                 scatter, codec, cache_elt, lin_elt, lin_dtype, scale_mode, fill_zeros, scatter, 0, 0,
@@ -492,9 +496,10 @@ def copy_rows_paged_checked(*, op: str, device: torch.device, src_planes: list[i
     src, dst = array("Q", src_planes), array("Q", dst_planes)
     with on_device(device):
         stream = stream_ptr(device)
-        with stream_lock(device, stream):
-            checks = _check_set(device, stream.value or 0)
-            claims, keep = claims_for(device, stream, dst_rows)
+        key = _stream_key(device, stream)
+        with _key_lock(key):
+            checks = _check_set(device, key[1], key)
+            claims, keep = claims_for(device, stream, dst_rows, key)
             checks.stamp += 1
             call = _COPY_ROWS_PAGED_CALL.pack(
                 src.buffer_info()[0], dst.buffer_info()[0], len(src), src_idx.data_ptr(), dst_idx.data_ptr(),
@@ -516,8 +521,9 @@ def block_tables_check(*, op: str, block_tables: torch.Tensor, seq_lens: torch.T
     with on_device(device):
         stream = stream_ptr(device)
         out = (_i64 * 3)()
-        with stream_lock(device, stream):
-            checks = _check_set(device, stream.value or 0)
+        key = _stream_key(device, stream)
+        with _key_lock(key):
+            checks = _check_set(device, key[1], key)
             checks.stamp += 1
             rc = fn("musa_aiter_hip_block_tables_check")(
                 block_tables.data_ptr(), seq_lens.data_ptr(), seq_lens.numel(), block_tables.shape[1], num_blocks,
