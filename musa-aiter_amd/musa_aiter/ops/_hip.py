@@ -365,7 +365,7 @@ _VALUE_WORDS = 2 * _REPORT_WORDS  # two lengths per workgroup of a table check; 
 
 
 class _CheckSet:
-    """Verdict words and table-check values (pinned host memory), guard word (device memory) and stamp of the
+    """Verdict words and table-check values (pinned host memory), guard word (device memory) and last stamp of the
     checked calls on one (device, stream), which issue one at a time under the stream's lock: a check kernel, where
     there is one, and the kernel it guards follow each other on the stream."""
     __slots__ = ("report", "guard", "report_ptr", "values_ptr", "guard_ptr", "stamp")
@@ -382,8 +382,7 @@ class _CheckSet:
 _check_sets: dict[tuple[int, int], _CheckSet] = {}
 _check_sets_lock = threading.Lock()
 _MAX_CHECK_SETS = 64  # per device; torch hands out 32 streams each, streams of other origin come and go
-_uses = itertools.count(1)
-_last_use: dict[tuple[int, int], int] = {}
+_stamps = itertools.count(1)  # a call's stamp tells its verdict from every other's, and when its set was last used
 
 
 def _check_set(device: torch.device, stream: int, key: tuple[int, int] | None = None) -> _CheckSet:
@@ -396,11 +395,8 @@ def _check_set(device: torch.device, stream: int, key: tuple[int, int] | None = 
             # back to the allocator of its own stream, behind the kernels that read it.
             own = [k for k in _check_sets if k[0] == key[0]]
             if len(own) >= _MAX_CHECK_SETS:
-                oldest = min(own, key=lambda k: _last_use.get(k, 0))
-                del _check_sets[oldest]
-                _last_use.pop(oldest, None)
+                del _check_sets[min(own, key=lambda k: getattr(_check_sets[k], "stamp", 0))]
             found = _check_sets[key] = _CheckSet(device)
-    _last_use[key] = next(_uses)
     return found
 
 
@@ -420,7 +416,7 @@ def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, l
         with _key_lock(key):
             checks = _check_set(device, key[1], key)
             claims, keep = (claims_for(device, stream, num_blocks * block_size, key) if scatter else (0, None))
-            checks.stamp += 1
+            checks.stamp = next(_stamps)
             call = _PAGED_TILES_CALL.pack(
                 scatter, codec, cache_elt, lin_elt, lin_dtype, scale_mode, fill_zeros, scatter, 0, 0,
                 key_cache.data_ptr(), value_cache.data_ptr(), key_linear.data_ptr(), value_linear.data_ptr(),
@@ -463,7 +459,6 @@ def paged_native(op, key_cache, value_cache, linear, slots, scales, *, layered: 
         checks = _check_sets.get(key)
         if checks is None:
             return None
-        _last_use[key] = next(_uses)
         claims, entry = 0, None
         if scatter:
             entry = _claim_sets.get(key)
@@ -471,7 +466,7 @@ def paged_native(op, key_cache, value_cache, linear, slots, scales, *, layered: 
                 return None
             entry[1].epoch += 1
             claims = ctypes.addressof(entry[1])
-        checks.stamp += 1
+        checks.stamp = next(_stamps)
         rc, k, v = h.paged_call(key_cache, value_cache, lin_k, lin_v, slots, k_scale, v_scale, scatter, layered, codec,
                                 out_dtype, _paged_entry[0], claims, checks.report_ptr, checks.guard_ptr,
                                 _REPORT_WORDS, checks.stamp, stream, index)
@@ -500,7 +495,7 @@ def copy_rows_paged_checked(*, op: str, device: torch.device, src_planes: list[i
         with _key_lock(key):
             checks = _check_set(device, key[1], key)
             claims, keep = claims_for(device, stream, dst_rows, key)
-            checks.stamp += 1
+            checks.stamp = next(_stamps)
             call = _COPY_ROWS_PAGED_CALL.pack(
                 src.buffer_info()[0], dst.buffer_info()[0], len(src), src_idx.data_ptr(), dst_idx.data_ptr(),
                 src_idx.numel(), src_rows, dst_rows, row_bytes, src_stride, dst_stride, 0, 0, 0, 0, low, claims,
@@ -524,7 +519,7 @@ def block_tables_check(*, op: str, block_tables: torch.Tensor, seq_lens: torch.T
         key = _stream_key(device, stream)
         with _key_lock(key):
             checks = _check_set(device, key[1], key)
-            checks.stamp += 1
+            checks.stamp = next(_stamps)
             rc = fn("musa_aiter_hip_block_tables_check")(
                 block_tables.data_ptr(), seq_lens.data_ptr(), seq_lens.numel(), block_tables.shape[1], num_blocks,
                 block_size, checks.report_ptr, _REPORT_WORDS, checks.values_ptr, checks.stamp, out, stream)

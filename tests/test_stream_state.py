@@ -122,17 +122,20 @@ def test_claims_of_other_streams_do_not_wait(state):
     assert done == [1] and _epoch() == 1
 
 
-def test_check_sets_give_way_by_last_use(state, monkeypatch):
+def test_check_sets_give_way_by_last_use(state):
     # A program with more streams than sets keeps the sets of those it uses, however early they were made, and
     # another device's sets are no reason to give one up.
-    monkeypatch.setattr(_hip, "_last_use", {})
-    hot = _hip._check_set(CPU, 0)
-    elsewhere = _hip._check_set(torch.device("cuda", 1), 0)
-    second = _hip._check_set(CPU, 1)
+    def used(device, stream):
+        checks = _hip._check_set(device, stream)
+        checks.stamp = next(_hip._stamps)  # as a call on the stream does
+        return checks
+
+    hot = used(CPU, 0)
+    elsewhere = used(torch.device("cuda", 1), 0)
+    second = used(CPU, 1)
     for stream in range(2, 3 * _hip._MAX_CHECK_SETS):
-        _hip._check_set(CPU, stream)
-        assert _hip._check_set(CPU, 0) is hot
+        used(CPU, stream)
+        assert used(CPU, 0) is hot
     assert _hip._check_set(CPU, 1) is not second
     assert _hip._check_sets[(1, 0)] is elsewhere
     assert sum(k[0] == 0 for k in _hip._check_sets) == _hip._MAX_CHECK_SETS
-    assert set(_hip._last_use) == set(_hip._check_sets)
