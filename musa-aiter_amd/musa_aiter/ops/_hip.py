@@ -253,9 +253,9 @@ class _Claims(ctypes.Structure):
 
 _EPOCH_LAST = 0xFFFFFFFF
 _MIN_CLAIM_TAGS = 1 << 16
-# (device index, stream handle) -> (tag tensor, its _Claims).  The tags come from torch's caching
+# (device index, stream handle) -> (tag tensor, its _Claims, the address of those).  The tags come from torch's caching
 # allocator on the stream that uses them, so the library allocates nothing for these scatters.
-_claim_sets: dict[tuple[int, int], tuple[torch.Tensor, _Claims]] = {}
+_claim_sets: dict[tuple[int, int], tuple[torch.Tensor, _Claims, int]] = {}
 
 
 # Scatters and checked calls on one (device, stream) issue one at a time, from the advance of the epoch to
@@ -299,14 +299,14 @@ def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int, key: tu
         have = entry[1].capacity if entry is not None else 0
         cap = max(rows, 2 * have, _MIN_CLAIM_TAGS)
         tags = torch.zeros(cap, dtype=torch.int64, device=device)
-        entry = (tags, _Claims(tags.data_ptr(), cap, 0, 0))
-        _claim_sets[key] = entry
-    tags, c = entry
+        c = _Claims(tags.data_ptr(), cap, 0, 0)
+        entry = _claim_sets[key] = (tags, c, ctypes.addressof(c))
+    tags, c, address = entry
     if c.epoch == _EPOCH_LAST:
         tags.zero_()
         c.epoch = 0
     c.epoch += 1
-    return ctypes.addressof(c), entry
+    return address, entry
 
 
 @contextlib.contextmanager
@@ -449,7 +449,7 @@ def paged_native(op, key_cache, value_cache, linear, slots, scales, *, layered: 
     lock = _stream_locks.get(key)
     if lock is None:
         return None  # the stream's first call makes its lock, check set and claims
-    h = host()
+    h = _host or host()
     if not _paged_entry:
         _paged_entry.append(ctypes.cast(fn("musa_aiter_hip_paged_tiles_checked"), ctypes.c_void_p).value)
     scatter = linear is not None
@@ -462,10 +462,13 @@ def paged_native(op, key_cache, value_cache, linear, slots, scales, *, layered: 
         claims, entry = 0, None
         if scatter:
             entry = _claim_sets.get(key)
-            if entry is None or entry[1].epoch == _EPOCH_LAST:
+            if entry is None:
                 return None
-            entry[1].epoch += 1
-            claims = ctypes.addressof(entry[1])
+            _, own, claims = entry
+            epoch = own.epoch
+            if epoch == _EPOCH_LAST:
+                return None
+            own.epoch = epoch + 1
         checks.stamp = next(_stamps)
         rc, k, v = h.paged_call(key_cache, value_cache, lin_k, lin_v, slots, k_scale, v_scale, scatter, layered, codec,
                                 out_dtype, _paged_entry[0], claims, checks.report_ptr, checks.guard_ptr,

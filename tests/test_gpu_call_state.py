@@ -160,7 +160,7 @@ def test_failed_launches_name_the_operation(monkeypatch, layers):
     for name, args in calls.items():
         getattr(musa_aiter, name + suffix)(*args)  # the stream's state exists from here on
     failed = SimpleNamespace(paged_call=lambda *_: (1, None, None), NOT_TAKEN=_hip.host().NOT_TAKEN)
-    monkeypatch.setattr(_hip, "host", lambda: failed)
+    monkeypatch.setattr(_hip, "_host", failed)
     for name, args in calls.items():
         with pytest.raises(_hip.HipBackendError, match=f"^{name + suffix}: HIP launch failed with error 1 "):
             getattr(musa_aiter, name + suffix)(*args)
