@@ -164,3 +164,49 @@ def test_failed_launches_name_the_operation(monkeypatch, layers):
     for name, args in calls.items():
         with pytest.raises(_hip.HipBackendError, match=f"^{name + suffix}: HIP launch failed with error 1 "):
             getattr(musa_aiter, name + suffix)(*args)
+
+
+@pytest.mark.parametrize("tokens", [40, 700])  # the kernel's own duplicate table; claim tags
+def test_threads_sharing_a_stream_lose_no_rows(tokens):
+    # Scatters, refused scatters and block-table write-backs of several threads on one stream claim in one tag
+    # array: every accepted row arrives.
+    stream = torch.cuda.Stream()
+    n, pages = 4, (tokens + BS - 1) // BS
+    caches = [torch.zeros((n * pages + 1, NH, HD, BS), device=DEV) for _ in range(2)]
+    rows = [torch.randn((n, tokens, NH, HD), device=DEV) for _ in range(2)]
+    slots = [k * pages * BS + torch.randperm(pages * BS, device=DEV)[:tokens] for k in range(n)]
+    dense = [torch.randn((1, BS, NH, HD), device=DEV) for _ in range(2)]
+    table, length = torch.tensor([[n * pages]], device=DEV), torch.tensor([BS], device=DEV)
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(k):
+        try:
+            bad = slots[k].clone()
+            bad[0] = (n * pages + 1) * BS
+            for _ in range(50):
+                with torch.cuda.stream(stream):
+                    with pytest.raises(ValueError):
+                        musa_aiter.kv_linear_to_paged(rows[0][k], rows[1][k], *caches, bad)
+                    musa_aiter.kv_linear_to_paged(rows[0][k], rows[1][k], *caches, slots[k])
+                    if k == 0:
+                        musa_aiter.kv_reshape_and_cache_back_flash(*dense, *caches, table, length)
+        except BaseException as e:  # reported by the main thread
+            errors.append(repr(e))
+
+    for _ in range(3):
+        for c in caches:
+            c.zero_()
+        torch.cuda.synchronize()
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(n)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+        assert errors == []
+        for k in range(n):
+            for want, got in zip(rows, musa_aiter.kv_paged_to_linear(*caches, slots[k])):
+                assert torch.equal(want[k], got)
+        for want, got in zip(dense, musa_aiter.kv_load_and_reshape_flash(*caches, table, length)):
+            assert torch.equal(want, got)
