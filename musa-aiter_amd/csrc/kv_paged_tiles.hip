@@ -232,7 +232,7 @@ constexpr int kShortRunTokens = 6;
 
 // Gathers take token_rows only in launches of at most kTokenGatherTokens
 // tokens (a kernel instantiation of their own, TOKG): compiled into every
-// gather, the form cost configs[0]'s gather 4 % (5,030 -> 4,860 GB/s) though
+// gather, the form cost the one-layer fp16 gather 4 % (5,030 -> 4,860 GB/s) though
 // none of its tiles took it.  There a tile takes it when its runs average
 // fewer than kShortGatherRunTokens tokens and none goes on past the tile.
 constexpr int64_t kTokenGatherTokens = 256;
@@ -481,7 +481,7 @@ void paged_tile_kernel(const TileArgs a) {
 // plane, row group) in block order reads its BS tags, finds the runs of
 // consecutive tokens in consecutive slots, and copies each run like the
 // token-major kernel.  Cache blocks are then written in address order and the
-// linear rows read in slot order: on configs[1]'s buffers the block-pattern
+// linear rows read in slot order: on the buffers of 32 bf16 layers the block-pattern
 // copy moves the scatter's bytes at 6.19 TB/s this way against 5.80 TB/s
 // with the cache blocks written in token order (random writes cost more than
 // random reads on this GPU).  Blocks no token writes cost one tag read.
@@ -611,7 +611,7 @@ constexpr int64_t kXcdOrderPlanes = 32;
 // 16-bit gathers whose 256-thread grid has at most kFewGroups workgroups use
 // 128-thread workgroups (2 KiB chunks) for block sizes up to 16.  Measured on
 // 1-4 planes of short sequences: 3-4 % faster with skipped slots or several
-// layers (4 bf16 layers: 13.5 -> 12.9 us), unchanged on configs[0] without
+// layers (4 bf16 layers: 13.5 -> 12.9 us), unchanged on one fp16 layer without
 // skips (12.9 us), 1 % slower for fp32 (chunks of only 32 rows).
 constexpr int kShortGatherThreads = 128;
 
@@ -663,12 +663,12 @@ hipError_t launch_tile(const TileArgs& a0, int64_t planes, hipStream_t stream) {
         a0.num_slots / BS <= 0x7FFFFFFF && a0.num_slots % BS == 0) {
       // Two 4 KiB chunks per workgroup, and the four workgroups of a block
       // next to each other in the grid (x = block * groups + group): on the
-      // configs[1] scatter 5.60 TB/s, against 5.46-5.52 with four chunks (grid
+      // 32-layer scatter 5.60 TB/s, against 5.46-5.52 with four chunks (grid
       // z or folded), 5.33 with eight and 4.80 with one.
       // 16-bit launches over fewer planes than the XCD order wants take the
       // per-wave kernel (a workgroup per block, no workgroup barrier): the
       // dense write-back (2 planes) 5.50-5.58 -> 5.60-5.74 TB/s; over
-      // configs[1]'s 64 planes the two kernels measured level, and the
+      // 64 planes (32 bf16 layers) the two kernels measured level, and the
       // cooperative one below keeps them.
       if constexpr (ELT == 2) {
         if (planes < kXcdOrderPlanes) return launch_wave_copy_scatter<BS>(a0, planes, stream);
@@ -681,8 +681,8 @@ hipError_t launch_tile(const TileArgs& a0, int64_t planes, hipStream_t stream) {
         TileArgs a = a0;
         a.row_groups = static_cast<int32_t>(groups);
         // Whole blocks are written through the L2 (kBufWT): +1.1 % on the
-        // configs[1] scatter.  Launches over at least 32 planes give each XCD
-        // a contiguous range of planes: configs[1]'s scatter 5.65 -> 5.85
+        // 32-layer scatter.  Launches over at least 32 planes give each XCD
+        // a contiguous range of planes: their scatter 5.65 -> 5.85
         // TB/s (same buffers, three allocations), where a plane-fastest order
         // ran at 5.46 and non-temporal stores at 5.60; with 2 planes (the
         // dense write-back) the two orders are within noise.

@@ -1115,7 +1115,7 @@ hipError_t launch_wave_scatter(const TileArgs& a, int64_t planes, hipStream_t st
   const dim3 grid(static_cast<uint32_t>(blocks), static_cast<uint32_t>(planes), static_cast<uint32_t>(zs));
   // In block order one workgroup takes one block (grid z covers chunks past
   // the fourth) and the lane's scale load is issued before the tag load: on
-  // configs[2]'s quant-store 5.04-5.16 -> 5.21-5.38 TB/s, where either change
+  // the one-layer E4M3 quant-store 5.04-5.16 -> 5.21-5.38 TB/s, where either change
   // alone measured no faster.  Partial runs (a sequence's last block) once
   // loaded and encoded their columns one load at a time: those few waves ran
   // several load latencies long and set the kernel's tail; sharing the

@@ -17,11 +17,15 @@
 // unit, so every run that starts in the tile ends inside the window.
 //
 // Bound by HBM.  9,001 tokens of 16 layers with 64-token pages (1.18 GB, 8 x
-// 128 bf16): gather 217 us (5.45 TB/s), scatter 229 us, against
+// 128 bf16): gather 207-211 us (5.6-5.7 TB/s), scatter 224 us, against
 // 1,217 us for the element kernel that served these block sizes before (its
 // 2-byte loads, a cache row apart, touch a line per lane).  A workgroup-
 // cooperative form with an LDS tile (512 threads, two 8 KiB chunks, as in
-// kv_paged_tiles.hip) measured 258 us and 283 us.
+// kv_paged_tiles.hip) measured 258 us and 283 us.  Single tokens cost as many
+// lines here as there; those of many layers whose blocks several tokens share
+// run up to 1.6 times longer than with the element kernel, which finishes plane
+// by plane and finds the shared lines in the memory-side cache (256 tokens of 16
+// layers of 4,096 rows, 192 blocks: 534 against 326 us).
 #include "kv_hip_common.h"
 #include "kv_launch.h"
 #include "kv_paged_args.h"
