@@ -270,19 +270,15 @@ def _stream_key(device: torch.device, stream: ctypes.c_void_p) -> tuple[int, int
     return (torch.cuda.current_device() if index is None else index, stream.value or 0)
 
 
-def _key_lock(key: tuple[int, int]) -> threading.Lock:
+def stream_lock(key: tuple[int, int]) -> threading.Lock:
+    """The lock of a (device index, stream handle), held from claims_for to the return of the call using the claims."""
     return _stream_locks.get(key) or _stream_locks.setdefault(key, threading.Lock())
 
 
-def stream_lock(device: torch.device, stream: ctypes.c_void_p) -> threading.Lock:
-    """The lock to hold from claims_for to the return of the call that uses the claims."""
-    return _key_lock(_stream_key(device, stream))
-
-
-def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int, key: tuple[int, int] | None = None):
-    """The claims of one scatter with ``rows`` destination rows on ``stream``: returns the address of a
-    musa_aiter_hip_claims to pass and the objects to keep alive until the call has returned.  The caller
-    holds the stream's lock.
+def claims_for(device: torch.device, key: tuple[int, int], rows: int):
+    """The claims of one scatter with ``rows`` destination rows on the (device index, stream handle) ``key``:
+    returns the address of a musa_aiter_hip_claims to pass and the objects to keep alive until the call has
+    returned.  The caller holds the stream's lock.
 
     Eager calls share one tag array per (device, stream), zeroed when allocated, with an epoch that
     advances per call (no clearing pass; the array is re-zeroed when the 32-bit epoch runs out).
@@ -293,7 +289,6 @@ def claims_for(device: torch.device, stream: ctypes.c_void_p, rows: int, key: tu
         tags = torch.empty(rows, dtype=torch.int64, device=device)
         c = _Claims(tags.data_ptr(), rows, 0, 0)
         return ctypes.addressof(c), (tags, c)
-    key = key or _stream_key(device, stream)
     entry = _claim_sets.get(key)
     if entry is None or entry[1].capacity < rows:
         have = entry[1].capacity if entry is not None else 0
@@ -413,9 +408,9 @@ def paged_tiles_checked(*, op: str, scatter: bool, codec: int, cache_elt: int, l
     with on_device(device):
         stream = stream_ptr(device)
         key = _stream_key(device, stream)
-        with _key_lock(key):
+        with stream_lock(key):
             checks = _check_set(device, key[1], key)
-            claims, keep = (claims_for(device, stream, num_blocks * block_size, key) if scatter else (0, None))
+            claims, keep = (claims_for(device, key, num_blocks * block_size) if scatter else (0, None))
             checks.stamp = next(_stamps)
             call = _PAGED_TILES_CALL.pack(
                 scatter, codec, cache_elt, lin_elt, lin_dtype, scale_mode, fill_zeros, scatter, 0, 0,
@@ -495,9 +490,9 @@ def copy_rows_paged_checked(*, op: str, device: torch.device, src_planes: list[i
     with on_device(device):
         stream = stream_ptr(device)
         key = _stream_key(device, stream)
-        with _key_lock(key):
+        with stream_lock(key):
             checks = _check_set(device, key[1], key)
-            claims, keep = claims_for(device, stream, dst_rows, key)
+            claims, keep = claims_for(device, key, dst_rows)
             checks.stamp = next(_stamps)
             call = _COPY_ROWS_PAGED_CALL.pack(
                 src.buffer_info()[0], dst.buffer_info()[0], len(src), src_idx.data_ptr(), dst_idx.data_ptr(),
@@ -520,7 +515,7 @@ def block_tables_check(*, op: str, block_tables: torch.Tensor, seq_lens: torch.T
         stream = stream_ptr(device)
         out = (_i64 * 3)()
         key = _stream_key(device, stream)
-        with _key_lock(key):
+        with stream_lock(key):
             checks = _check_set(device, key[1], key)
             checks.stamp = next(_stamps)
             rc = fn("musa_aiter_hip_block_tables_check")(
@@ -587,9 +582,9 @@ def paged_tiles(
     device = key_cache.device
     with on_device(device):
         stream = stream_ptr(device)
-        with stream_lock(device, stream) if scatter and dedupe else _NOTHING:
-            claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter and dedupe
-                            else (None, None))
+        key = _stream_key(device, stream) if scatter and dedupe else None
+        with stream_lock(key) if key else _NOTHING:
+            claims, keep = claims_for(device, key, num_blocks * block_size) if key else (None, None)
             rc = fn("musa_aiter_hip_paged_tiles")(
                 int(scatter), int(codec), int(cache_elt), int(lin_elt), int(lin_dtype),
                 ptr(key_cache), ptr(value_cache), ptr(key_linear), ptr(value_linear), ptr(slots),
@@ -631,9 +626,9 @@ def copy_rows(
     dst_arr = _as_u64(dst_planes)
     with on_device(device):
         stream = stream_ptr(device)
-        with stream_lock(device, stream) if dedupe and dst_idx is not None else _NOTHING:
-            claims, keep = (claims_for(device, stream, dst_rows) if dedupe and dst_idx is not None
-                            else (0, None))
+        key = _stream_key(device, stream) if dedupe and dst_idx is not None else None
+        with stream_lock(key) if key else _NOTHING:
+            claims, keep = claims_for(device, key, dst_rows) if key else (0, None)
             # One struct (musa_aiter_hip_copy_rows_call) instead of 19 converted ctypes arguments; the plane
             # arrays stay referenced by src_arr / dst_arr until the call returns.
             call = _COPY_ROWS_CALL.pack(
@@ -679,9 +674,9 @@ def paged_dense_tiles(
     device = key_cache.device
     with on_device(device):
         stream = stream_ptr(device)
-        with stream_lock(device, stream) if scatter and dedupe else _NOTHING:
-            claims, keep = (claims_for(device, stream, num_blocks * block_size) if scatter and dedupe
-                            else (None, None))
+        key = _stream_key(device, stream) if scatter and dedupe else None
+        with stream_lock(key) if key else _NOTHING:
+            claims, keep = claims_for(device, key, num_blocks * block_size) if key else (None, None)
             rc = fn("musa_aiter_hip_paged_dense_tiles")(
                 int(scatter), int(codec), int(cache_elt), int(lin_elt), int(lin_dtype),
                 ptr(key_cache), ptr(value_cache), ptr(dense_k), ptr(dense_v), ptr(block_tables), ptr(seq_lens),
@@ -749,8 +744,9 @@ def copy_rows_paged(
         raise ValueError(f"{op}: source and destination plane lists differ in length")
     with on_device(device):
         stream = stream_ptr(device)
-        with stream_lock(device, stream) if dedupe else _NOTHING:
-            claims, keep = claims_for(device, stream, dst_rows) if dedupe else (None, None)
+        key = _stream_key(device, stream) if dedupe else None
+        with stream_lock(key) if key else _NOTHING:
+            claims, keep = claims_for(device, key, dst_rows) if key else (None, None)
             rc = fn("musa_aiter_hip_copy_rows_paged")(
                 u64_array(src_planes), u64_array(dst_planes), planes, ptr(src_idx), ptr(dst_idx), tokens,
                 int(src_rows), int(dst_rows), int(row_bytes), int(src_stride), int(dst_stride),
@@ -786,8 +782,9 @@ def copy_blocks(
     device = dst_k.device
     with on_device(device):
         stream = stream_ptr(device)
-        with stream_lock(device, stream):
-            claims, keep = claims_for(device, stream, dst_blocks)
+        key = _stream_key(device, stream)
+        with stream_lock(key):
+            claims, keep = claims_for(device, key, dst_blocks)
             rc = fn("musa_aiter_hip_copy_blocks")(
                 ptr(src_k), ptr(src_v), ptr(dst_k), ptr(dst_v), ptr(block_mapping), pairs, int(num_layers),
                 int(src_blocks), int(dst_blocks), int(block_bytes), claims, stream,

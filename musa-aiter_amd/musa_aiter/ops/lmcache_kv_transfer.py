@@ -378,9 +378,9 @@ def _two_x_nl_fast(op: str, kvcaches, memory_tensor, slot_mapping, skip: int, bl
         device = memory_tensor.device
         if device.index != index:
             return False
-        with _hip.stream_lock(device, ctypes.c_void_p(stream)):
-            claims, keep = _hip.claims_for(device, ctypes.c_void_p(stream),
-                                           int(kvcaches[0][0].shape[0]) * int(block_size))
+        key = (index, stream)
+        with _hip.stream_lock(key):
+            claims, keep = _hip.claims_for(device, key, int(kvcaches[0][0].shape[0]) * int(block_size))
             rc = h.two_x_nl_rows(*call, claims, stream, index)
             del keep
     else:
