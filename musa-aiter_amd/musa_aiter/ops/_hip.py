@@ -583,7 +583,10 @@ def paged_tiles(
     with on_device(device):
         stream = stream_ptr(device)
         key = _stream_key(device, stream) if scatter and dedupe else None
-        with stream_lock(key) if key else _NOTHING:
+        lock = stream_lock(key) if key else None
+        if lock:
+            lock.acquire()
+        try:
             claims, keep = claims_for(device, key, num_blocks * block_size) if key else (None, None)
             rc = fn("musa_aiter_hip_paged_tiles")(
                 int(scatter), int(codec), int(cache_elt), int(lin_elt), int(lin_dtype),
@@ -594,6 +597,9 @@ def paged_tiles(
                 int(bool(fill_zeros)), int(bool(dedupe)), claims, stream,
             )
             del keep
+        finally:
+            if lock:
+                lock.release()
     check(rc, op)
 
 
@@ -627,7 +633,10 @@ def copy_rows(
     with on_device(device):
         stream = stream_ptr(device)
         key = _stream_key(device, stream) if dedupe and dst_idx is not None else None
-        with stream_lock(key) if key else _NOTHING:
+        lock = stream_lock(key) if key else None
+        if lock:
+            lock.acquire()
+        try:
             claims, keep = claims_for(device, key, dst_rows) if key else (0, None)
             # One struct (musa_aiter_hip_copy_rows_call) instead of 19 converted ctypes arguments; the plane
             # arrays stay referenced by src_arr / dst_arr until the call returns.
@@ -637,6 +646,9 @@ def copy_rows(
                 row_bytes, src_stride, dst_stride, bool(zero_invalid), bool(dedupe), claims)
             rc = fn("musa_aiter_hip_copy_rows_packed")(call, stream)
             del keep
+        finally:
+            if lock:
+                lock.release()
     check(rc, op)
 
 
@@ -675,7 +687,10 @@ def paged_dense_tiles(
     with on_device(device):
         stream = stream_ptr(device)
         key = _stream_key(device, stream) if scatter and dedupe else None
-        with stream_lock(key) if key else _NOTHING:
+        lock = stream_lock(key) if key else None
+        if lock:
+            lock.acquire()
+        try:
             claims, keep = claims_for(device, key, num_blocks * block_size) if key else (None, None)
             rc = fn("musa_aiter_hip_paged_dense_tiles")(
                 int(scatter), int(codec), int(cache_elt), int(lin_elt), int(lin_dtype),
@@ -685,6 +700,9 @@ def paged_dense_tiles(
                 int(bool(fill_zeros)), int(bool(dedupe)), claims, stream,
             )
             del keep
+        finally:
+            if lock:
+                lock.release()
     check(rc, op)
 
 
@@ -745,7 +763,10 @@ def copy_rows_paged(
     with on_device(device):
         stream = stream_ptr(device)
         key = _stream_key(device, stream) if dedupe else None
-        with stream_lock(key) if key else _NOTHING:
+        lock = stream_lock(key) if key else None
+        if lock:
+            lock.acquire()
+        try:
             claims, keep = claims_for(device, key, dst_rows) if key else (None, None)
             rc = fn("musa_aiter_hip_copy_rows_paged")(
                 u64_array(src_planes), u64_array(dst_planes), planes, ptr(src_idx), ptr(dst_idx), tokens,
@@ -754,6 +775,9 @@ def copy_rows_paged(
                 int(bool(dedupe)), claims, stream,
             )
             del keep
+        finally:
+            if lock:
+                lock.release()
     check(rc, op)
 
 
