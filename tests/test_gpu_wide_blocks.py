@@ -195,3 +195,56 @@ def test_wide_fp8_blocks_with_more_row_chunks_than_a_grid_holds():
         assert np.array_equal(cache_d[0, :, :, slots].permute(2, 0, 1).cpu().numpy(), want[..., 0])
         assert int((cache_d != 0).sum()) == int((want != 0).sum())
         assert np.array_equal(bits(out), ko.paged_fp8_to_linear(want, np.array([0, 1]), scale.numpy(), "e4m3", "float32"))
+
+
+# The forms by elements over every layout that reaches them: rows of K and V apart, merged, and at a token stride
+# of the caller's; dense tensors through block tables.  A token of 23 x 88 = 2,024 elements is no whole chunk; slots are
+# skipped and repeated.  Every form only moves elements: results are equal bit for bit.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("bs", [64, 192])
+@pytest.mark.parametrize("tokens", [300, 700, 1500])  # 1.2, 2.8 and 6 Mi elements of K and V
+@pytest.mark.parametrize("layout", ["merged", "strided", "dense"])
+def test_wide_forms_in_every_layout(dtype, bs, tokens, layout):
+    nh, hd, nb = 23, 88, tokens // bs + 5
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    caches = [torch.randn((nb, nh, hd, bs), generator=gen, device=DEV).to(dtype) for _ in range(2)]
+
+    def paged_rows(cache):
+        return cache.permute(0, 3, 1, 2).reshape(nb * bs, nh, hd)
+
+    if layout == "dense":
+        batch, cols = 3, nb // 3
+        tables = torch.randperm(nb, generator=gen, device=DEV)[:batch * cols].view(batch, cols)
+        lens = torch.tensor([cols * bs - 7, bs // 2 + 1, cols * bs], device=DEV)
+        pos = torch.arange(cols * bs, device=DEV)
+        slots = torch.where(pos < lens[:, None], tables[:, pos // bs] * bs + pos % bs, -1).reshape(-1)
+    else:
+        runs = torch.arange(nb * bs, device=DEV).view(-1, 8)
+        slots = runs[torch.randperm(len(runs), generator=gen, device=DEV)].reshape(-1)[:tokens].clone()
+        slots[:64] = torch.arange(64, 128, device=DEV)           # a unit, in order
+        slots[64::37] = -1
+        slots[70] = slots[tokens - 3]                            # the later one wins
+    moves = slots >= 0
+    rows = [torch.randn((len(slots), nh, hd), generator=gen, device=DEV).to(dtype) for _ in range(2)]
+    want = [torch.where(moves[:, None, None], paged_rows(c)[slots.clamp(min=0)], 0) for c in caches]
+    stored = [paged_rows(c).clone() for c in caches]
+    last = {int(s): t for t, s in enumerate(slots.tolist()) if s >= 0}
+    at, by = (torch.tensor(x, device=DEV) for x in (list(last), list(last.values())))
+    for s, r in zip(stored, rows):
+        s[at] = r[by]
+    if layout == "merged":
+        got = musa_aiter.kv_paged_to_merged_linear(*caches, slots).unbind(1)
+        musa_aiter.kv_merged_linear_to_paged(torch.stack(rows, 1), *caches, slots)
+    elif layout == "strided":
+        pads = [torch.full((tokens, nh + 2, hd), 5.0, dtype=dtype, device=DEV) for _ in range(2)]
+        got = [p[:, :nh] for p in pads]
+        musa_aiter.kv_paged_to_linear(*caches, slots, out_k=got[0], out_v=got[1])
+        assert all(bool((p[:, nh:] == 5.0).all()) for p in pads)
+        musa_aiter.kv_linear_to_paged(*(torch.cat([r, r[:, :2]], 1)[:, :nh] for r in rows), *caches, slots)
+    else:
+        got = [g.reshape(-1, nh, hd) for g in musa_aiter.kv_load_and_reshape_flash(*caches, tables, lens)]
+        musa_aiter.kv_reshape_and_cache_back_flash(*(r.view(batch, -1, nh, hd) for r in rows), *caches, tables, lens)
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
+    for c, s in zip(caches, stored):
+        assert torch.equal(paged_rows(c), s)
